@@ -15,9 +15,7 @@
 namespace {
 
 constexpr int kRowsPerBlock = 32;  // 256 threads, 8 lanes per row
-static_assert(kRowsPerBlock == sgk::kRowKernelRows, "row kernels' workgroup rows");
 constexpr int kThreads = 256;
-constexpr int kQuantNbRows = 8192;  // the quantizers' branch-free form below this many rows
 
 __device__ __forceinline__ uint16_t rd_u16(const uint8_t* p) { return (uint16_t)(p[0] | (p[1] << 8)); }
 
@@ -213,9 +211,8 @@ __global__ __launch_bounds__(kThreads) void k_quantize(const float* __restrict__
 // when they folded max|xn| into amax (so every value, and the scale, is the
 // one the unfused path quantizes), then quantized as k_quantize does
 // (model_int8.go:194-199 / :216-221: RMSNorm, then QuantizeSymmetricINT8 of
-// the normed sequence).  Saves writing xn and reading it back.  NB: the
-// branch-free codes, for small launches.
-template <int NC, bool NB>
+// the normed sequence).  Saves writing xn and reading it back.
+template <int NC>
 __global__ __launch_bounds__(kThreads) void k_norm_quantize(const float* __restrict__ h, const float* __restrict__ w,
                                                             float eps, int T, const int32_t* __restrict__ row_seq,
                                                             const float* __restrict__ amax,
@@ -249,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void k_norm_quantize(const float* __restr
   for (int c = 0; c < NC; c++) {
     float cv[4];
 #pragma unroll
-    for (int t = 0; t < 4; t++) cv[t] = NB ? sg_quant_code_nb(x[c][t], inv) : sg_quant_code(x[c][t], inv);
+    for (int t = 0; t < 4; t++) cv[t] = sg_quant_code(x[c][t], inv);
     store_codes4(qr + (int64_t)c * a_rows * 32, cv);
   }
 }
@@ -257,9 +254,8 @@ __global__ __launch_bounds__(kThreads) void k_norm_quantize(const float* __restr
 // The GEMM-operand form of k_quantize on the float4 row layout: an 8-lane
 // group per row, lane j handling elements 32c + 4j .. + 3 of every chunk c
 // (chunk c is K-block c), so a wave's stores cover 8 consecutive rows' 64-byte
-// block pieces: 512 contiguous bytes per instruction.  NB: the branch-free
-// codes, for small launches (latency-bound rather than bandwidth-bound).
-template <int NC, bool NB>
+// block pieces: 512 contiguous bytes per instruction.
+template <int NC>
 __global__ __launch_bounds__(kThreads) void k_quantize_blocked(const float* __restrict__ x, int ldx, int rows,
                                                                const int32_t* __restrict__ row_seq,
                                                                const float* __restrict__ amax,
@@ -284,7 +280,7 @@ __global__ __launch_bounds__(kThreads) void k_quantize_blocked(const float* __re
   for (int c = 0; c < NC; c++) {
     float cv[4];
 #pragma unroll
-    for (int t = 0; t < 4; t++) cv[t] = NB ? sg_quant_code_nb(v[c][t], inv) : sg_quant_code(v[c][t], inv);
+    for (int t = 0; t < 4; t++) cv[t] = sg_quant_code(v[c][t], inv);
     store_codes4(qr + (int64_t)c * a_rows * 32, cv);
   }
 }
@@ -353,70 +349,182 @@ __global__ __launch_bounds__(kThreads) void k_post_res_norm(const float* __restr
   }
 }
 
-// k_post_res_norm followed by the next GEMM's operand, in one launch, for
-// batches in which every sequence's rows lie inside one workgroup's
-// kRowsPerBlock rows (the caller checks; short sequences, the serving case).
-// Each sequence's max|xn| is then complete inside the workgroup, so xn --
-// still in the lanes that formed it -- is quantized with it right away, as
-// k_norm_quantize would quantize the xn it recomputes from h: the same values,
-// scale, reciprocal and codes (quantize.go:29-103 per sequence), into the
-// block-major operand q8 [D/32][a_rows][32] and row_scale.  The sequences'
-// maxima also go to amax, as k_post_res_norm leaves them.
-template <int NC>
-__global__ __launch_bounds__(kThreads) void k_post_res_norm_q(const float* __restrict__ o, float* __restrict__ h,
-                                                              const float* __restrict__ w_post,
-                                                              const float* __restrict__ w_next, float eps, int T,
-                                                              const int32_t* __restrict__ row_seq,
-                                                              float* __restrict__ amax, int8_t* __restrict__ q8,
-                                                              int a_rows, float* __restrict__ row_scale) {
-  constexpr int D = NC * 32;
-  __shared__ __attribute__((aligned(16))) float tiles[kThreads / SG_WAVE][8 * 40];
-  __shared__ float rmax[kRowsPerBlock];
-  __shared__ int rseq[kRowsPerBlock];
-  const int rl = threadIdx.x >> 3, row = blockIdx.x * kRowsPerBlock + rl;
-  const int j = threadIdx.x & 7, r = rl & 7;
-  const bool valid = row < T;
-  // The row's sequence now: its load overlaps the row loads instead of
-  // following the norms.
-  const int sq = valid ? row_seq[row] : -1;
-  f32x4_t x[NC];
-  float m = 0.0f;
-  if (valid) {
-    f32x4_t hv[NC];
-    const f32x4_t* op = reinterpret_cast<const f32x4_t*>(o + (int64_t)row * D) + j;
-    const f32x4_t* hp = reinterpret_cast<const f32x4_t*>(h + (int64_t)row * D) + j;
+// A wave's row (lane l: elements 256k + 4l .. + 3) as block-major codes.
+template <int NV, int D = NV * 256>
+__device__ __forceinline__ void store_codes_wave(const f32x4_t (&x)[NV], float inv, int8_t* __restrict__ q, int a_rows,
+                                                 int row, int lane) {
+  int8_t* qr = q + ((int64_t)(lane >> 3) * a_rows + row) * 32 + 4 * (lane & 7);
 #pragma unroll
-    for (int c = 0; c < NC; c++) x[c] = __builtin_nontemporal_load(&op[8 * c]);
-#pragma unroll
-    for (int c = 0; c < NC; c++) hv[c] = __builtin_nontemporal_load(&hp[8 * c]);
-    m = sg_post_res_norm_f4<NC>(x, hv, h + (int64_t)row * D, w_post, w_next, eps, nullptr,
-                                tiles[threadIdx.x / SG_WAVE], r, j);
-  }
-  m = sg_max8(m);
-  if (j == 0) {
-    rmax[rl] = m;  // 0 for rows past T
-    rseq[rl] = sq;
-  }
-  __syncthreads();
-  if (!valid) return;
-  // The row's sequence maximum over this workgroup's rows (all of them).
-  float sm = 0.0f;
-  for (int i = 0; i < kRowsPerBlock; i++) sm = rseq[i] == sq ? fmaxf(sm, rmax[i]) : sm;
-  const bool first = rl == 0 || rseq[rl - 1] != sq;
-  if (amax && first && j == 0) sg_atomic_max_nonneg(amax + sq, sm);
-  float scale = 1.0f, inv = 0.0f;
-  if (sm != 0.0f) {
-    scale = sm / 127.0f;
-    inv = 1.0f / scale;
-  }
-  if (j == 0) row_scale[row] = scale;
-  int8_t* qr = q8 + (int64_t)row * 32 + 4 * j;
-#pragma unroll
-  for (int c = 0; c < NC; c++) {
+  for (int k = 0; k < NV; k++) {
     float cv[4];
 #pragma unroll
-    for (int t = 0; t < 4; t++) cv[t] = sg_quant_code_nb(x[c][t], inv);
-    store_codes4(qr + (int64_t)c * a_rows * 32, cv);
+    for (int t = 0; t < 4; t++) cv[t] = sg_quant_code_nb(x[k][t], inv);
+    if (256 * k + 256 <= D || 256 * k + 4 * lane < D) store_codes4(qr + (int64_t)(8 * k) * a_rows * 32, cv);
+  }
+}
+
+// ------------------------------------------------------ wave-per-row forms --
+//
+// The row kernels for launches of fewer than kWaveRows rows.  There a kernel's
+// time is the latency of one workgroup, not bandwidth: with 8 lanes per row a
+// lane carries 96 values of a 768-wide row through the elementwise work and
+// each norm makes 24 dependent LDS round trips, and 32 rows share a workgroup
+// while most CUs idle.  One wave per row leaves 12 values per lane, one LDS
+// round trip per norm (sg_wave_inv_rms) and eight times the workgroups.  Same
+// arithmetic and order, bit-identical.  Microseconds on MI355X at D = 768,
+// 8-lane groups -> wave per row (kernel trace):
+//   rows            509          1024         2048         4096          6144
+//   post-norm     8.3 -> 4.4   8.9 -> 5.0   9.6 -> 6.3  11.6 -> 8.9   14.1 -> 11.5
+//   norm-quantize 7.2 -> 4.2   7.2 -> 4.5   7.9 -> 5.2   8.4 -> 6.2    7.8 -> 7.4
+//   quantize 1152 6.9 -> 4.0   6.8 -> 4.9   7.1 -> 5.0   7.5 -> 5.9    8.6 -> 7.2
+// and the embedding 17 -> 4 us at 509 rows.  The chains' eightfold VALU and
+// LDS work costs about 1.7 us per 1000 rows of post-norm, so the two forms
+// meet near 8192 rows, where the 8-lane groups fill every CU (256 workgroups).
+constexpr int kWaveRows = 8192;
+constexpr int kWaveWaves = kThreads / SG_WAVE;  // rows per workgroup
+
+// k_embed_norm (h stored, xn not; the row's max|xn| into rmax).
+template <int NV>
+__global__ __launch_bounds__(kThreads) void k_embed_norm_wave(const int32_t* __restrict__ tokens, int T,
+                                                              const int8_t* __restrict__ eq,
+                                                              const float* __restrict__ es, int vocab, float sqrt_d,
+                                                              const float* __restrict__ w, float eps,
+                                                              float* __restrict__ h, float* __restrict__ rmax,
+                                                              int32_t* __restrict__ err) {
+  constexpr int D = NV * 256;
+  __shared__ __attribute__((aligned(16))) float tiles[kWaveWaves][kWaveTile<NV>];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = blockIdx.x * kWaveWaves + wave;
+  if (row >= T) return;
+  f32x4_t wv[NV];
+  sg_wave_load<NV>(wv, w, lane);
+  int id = tokens[row];
+  if (id < 0 || id >= vocab) {
+    if (lane == 0) atomicMin(err, row);  // the first offending row (rows run in request order)
+    id = 0;                              // keep the access in bounds; the call reports SG_ERR_TOKEN
+  }
+  const int8_t* qr = eq + (int64_t)id * D + 4 * lane;
+  const float* sr = es + (int64_t)id * (D / 32) + (lane >> 3);
+  f32x4_t x[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    const uint32_t q4 = *reinterpret_cast<const uint32_t*>(qr + 256 * k);
+    const float sc = sr[8 * k];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const float v = (float)(int8_t)(q4 >> (8 * t)) * sc;
+      x[k][t] = v * sqrt_d;
+    }
+  }
+  sg_wave_tile_put<NV>(x, tiles[wave], lane);
+  float* hr = h + (int64_t)row * D + 4 * lane;
+#pragma unroll
+  for (int k = 0; k < NV; k++) *reinterpret_cast<f32x4_t*>(hr + 256 * k) = x[k];
+  sg_wave_scale<NV>(x, sg_wave_inv_rms<NV>(tiles[wave], lane, eps), wv);
+  const float m = sg_wave_max(sg_wave_absmax<NV>(x));
+  if (lane == 0) rmax[row] = m;
+}
+
+// k_norm_quantize with the sequence's maximum taken over its rows' maxima.
+template <int NV>
+__global__ __launch_bounds__(kThreads) void k_norm_quantize_wave(const float* __restrict__ h,
+                                                                 const float* __restrict__ w, float eps, int T,
+                                                                 const int32_t* __restrict__ row_seq,
+                                                                 const int32_t* __restrict__ seq_off,
+                                                                 const float* __restrict__ rmax,
+                                                                 int8_t* __restrict__ qf, int a_rows,
+                                                                 float* __restrict__ row_scale) {
+  constexpr int D = NV * 256;
+  __shared__ __attribute__((aligned(16))) float tiles[kWaveWaves][kWaveTile<NV>];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = blockIdx.x * kWaveWaves + wave;
+  if (row >= T) return;
+  const int sq = row_seq[row];
+  f32x4_t x[NV], wv[NV];
+  sg_wave_load<NV>(x, h + (int64_t)row * D, lane);
+  sg_wave_load<NV>(wv, w, lane);
+  const float m = sg_wave_rows_max(rmax, seq_off[sq], seq_off[sq + 1], lane);
+  sg_wave_tile_put<NV>(x, tiles[wave], lane);
+  sg_wave_scale<NV>(x, sg_wave_inv_rms<NV>(tiles[wave], lane, eps), wv);
+  float scale = 1.0f, inv = 0.0f;
+  if (m != 0.0f) {
+    scale = m / 127.0f;
+    inv = 1.0f / scale;
+  }
+  if (lane == 0) row_scale[row] = scale;
+  store_codes_wave<NV>(x, inv, qf, a_rows, row, lane);
+}
+
+// k_quantize_blocked for D = cols columns (a multiple of 32).
+template <int D>
+__global__ __launch_bounds__(kThreads) void k_quantize_wave(const float* __restrict__ x, int ldx, int rows,
+                                                            const int32_t* __restrict__ row_seq,
+                                                            const float* __restrict__ amax, int8_t* __restrict__ qf,
+                                                            int a_rows, float* __restrict__ row_scale) {
+  constexpr int NV = (D + 255) / 256;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = blockIdx.x * kWaveWaves + wave;
+  if (row >= rows) return;
+  const int sq = row_seq[row];
+  const float* xr = x + (int64_t)row * ldx + 4 * lane;
+  f32x4_t v[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    v[k] = f32x4_t{0, 0, 0, 0};
+    if (256 * k + 256 <= D || 256 * k + 4 * lane < D) v[k] = *reinterpret_cast<const f32x4_t*>(xr + 256 * k);
+  }
+  const float m = amax[sq];
+  float scale = 1.0f, inv = 0.0f;
+  if (m != 0.0f) {
+    scale = m / 127.0f;
+    inv = 1.0f / scale;
+  }
+  if (lane == 0) row_scale[row] = scale;
+  store_codes_wave<NV, D>(v, inv, qf, a_rows, row, lane);
+}
+
+// k_post_res_norm (sg_post_res_norm_f4's arithmetic; w_post, w_next optional):
+// h = RMSNorm(o; w_post) + h, then xn = RMSNorm(h; w_next), stored when xn !=
+// null; the row's max|xn| into rmax when rmax != null.
+template <int NV>
+__global__ __launch_bounds__(kThreads) void k_post_res_norm_wave(const float* __restrict__ o, float* __restrict__ h,
+                                                                 const float* __restrict__ w_post,
+                                                                 const float* __restrict__ w_next, float eps, int T,
+                                                                 float* __restrict__ xn, float* __restrict__ rmax) {
+  constexpr int D = NV * 256;
+  __shared__ __attribute__((aligned(16))) float tiles[kWaveWaves][kWaveTile<NV>];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int row = blockIdx.x * kWaveWaves + wave;
+  if (row >= T) return;
+  float* tile = tiles[wave];
+  float* hr = h + (int64_t)row * D;
+  f32x4_t x[NV], hv[NV], wp[NV], wn[NV];
+  sg_wave_load<NV>(x, o + (int64_t)row * D, lane);
+  sg_wave_load<NV>(hv, hr, lane);
+  if (w_post) sg_wave_load<NV>(wp, w_post, lane);
+  if (w_next) sg_wave_load<NV>(wn, w_next, lane);
+  if (w_post) {
+    sg_wave_tile_put<NV>(x, tile, lane);
+    sg_wave_scale<NV>(x, sg_wave_inv_rms<NV>(tile, lane, eps), wp);
+  }
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) x[k][t] = x[k][t] + hv[k][t];
+    *reinterpret_cast<f32x4_t*>(hr + 256 * k + 4 * lane) = x[k];
+  }
+  if (w_next) {
+    sg_wave_tile_put<NV>(x, tile, lane);
+    sg_wave_scale<NV>(x, sg_wave_inv_rms<NV>(tile, lane, eps), wn);
+  }
+  if (xn) {
+    float* yr = xn + (int64_t)row * D + 4 * lane;
+#pragma unroll
+    for (int k = 0; k < NV; k++) *reinterpret_cast<f32x4_t*>(yr + 256 * k) = x[k];
+  }
+  if (rmax) {
+    const float m = sg_wave_max(sg_wave_absmax<NV>(x));
+    if (lane == 0) rmax[row] = m;
   }
 }
 
@@ -702,10 +810,28 @@ hipError_t first_bad_token(const int32_t* tokens, int T, int vocab, int32_t* fir
     default: return hipErrorInvalidValue;     \
   }
 
+// The wave-per-row forms: rows of whole float4 waves.
+#define SG_DISPATCH_NV(n, NVV, ...)           \
+  switch (n) {                                \
+    case 256: { constexpr int NVV = 1; __VA_ARGS__; break; }  \
+    case 512: { constexpr int NVV = 2; __VA_ARGS__; break; }  \
+    case 768: { constexpr int NVV = 3; __VA_ARGS__; break; }  \
+    case 1024: { constexpr int NVV = 4; __VA_ARGS__; break; } \
+    default: return hipErrorInvalidValue;     \
+  }
+bool row_max_form(int T, int d) { return T < kWaveRows && d <= 1024; }
+
 hipError_t embed_norm(const int32_t* tokens, int T, const int8_t* eq, const float* es, int vocab, int d,
                       float sqrt_d, const float* w, float eps, const int32_t* row_seq, float* h, float* xn,
-                      float* amax, int32_t* err, hipStream_t s) {
+                      float* amax, int32_t* err, hipStream_t s, float* rmax) {
   if (T <= 0) return hipSuccess;
+  if (rmax) {
+    if (xn || !row_max_form(T, d)) return hipErrorInvalidValue;
+    SG_DISPATCH_NV(d, NV,
+                   hipLaunchKernelGGL(k_embed_norm_wave<NV>, dim3(blocks_for(T, kWaveWaves)), dim3(kThreads), 0, s,
+                                      tokens, T, eq, es, vocab, sqrt_d, w, eps, h, rmax, err));
+    return hipGetLastError();
+  }
   SG_DISPATCH_NPL(d, NPL,
                   hipLaunchKernelGGL(k_embed_norm<NPL>, dim3(blocks_for(T, kRowsPerBlock)), dim3(kThreads), 0, s,
                                      tokens, T, eq, es, vocab, sqrt_d, w, eps, row_seq, h, xn, amax, err));
@@ -727,18 +853,17 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
   if (cols % 4 || ldx % 4 || (!q8 && !i8)) return hipErrorInvalidValue;
   if (q8 && (cols % 32 || a_rows < rows)) return hipErrorInvalidValue;
   if (q8 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
-    const unsigned nb = blocks_for(rows, kRowsPerBlock);
-    // At most one round of workgroups: latency-bound, the branch-free codes.
-    const bool small = rows < kQuantNbRows;
+    // Fewer rows than kWaveRows: latency-bound, a wave per row.
+    const bool small = rows < kWaveRows;
     switch (cols) {  // the widths the forward quantizes: attention output, hidden, FFN
-#define SG_QB(C)                                                                                                   \
-  case C:                                                                                                          \
-    if (small)                                                                                                     \
-      hipLaunchKernelGGL((k_quantize_blocked<C / 32, true>), dim3(nb), dim3(kThreads), 0, s, x, ldx, rows, row_seq, \
-                         amax, q8, a_rows, row_scale);                                                             \
-    else                                                                                                           \
-      hipLaunchKernelGGL((k_quantize_blocked<C / 32, false>), dim3(nb), dim3(kThreads), 0, s, x, ldx, rows,        \
-                         row_seq, amax, q8, a_rows, row_scale);                                                    \
+#define SG_QB(C)                                                                                                     \
+  case C:                                                                                                            \
+    if (small)                                                                                                       \
+      hipLaunchKernelGGL(k_quantize_wave<C>, dim3(blocks_for(rows, kWaveWaves)), dim3(kThreads), 0, s, x, ldx, rows, \
+                         row_seq, amax, q8, a_rows, row_scale);                                                      \
+    else                                                                                                             \
+      hipLaunchKernelGGL(k_quantize_blocked<C / 32>, dim3(blocks_for(rows, kRowsPerBlock)), dim3(kThreads), 0, s, x, \
+                         ldx, rows, row_seq, amax, q8, a_rows, row_scale);                                           \
     return hipGetLastError();
       SG_QB(256) SG_QB(512) SG_QB(768) SG_QB(1024) SG_QB(1152)
 #undef SG_QB
@@ -752,18 +877,20 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
 }
 
 hipError_t norm_quantize(const float* h, const float* w, float eps, int T, int d, const int32_t* row_seq,
-                         const float* amax, int8_t* q8, int a_rows, float* row_scale, hipStream_t s) {
+                         const float* amax, int8_t* q8, int a_rows, float* row_scale, hipStream_t s, const float* rmax,
+                         const int32_t* seq_off) {
   if (T <= 0) return hipSuccess;
   if (a_rows < T) return hipErrorInvalidValue;
-  if (T < kQuantNbRows) {
-    SG_DISPATCH_NPL(d, NPL,
-                    hipLaunchKernelGGL((k_norm_quantize<NPL / 4, true>), dim3(blocks_for(T, kRowsPerBlock)),
-                                       dim3(kThreads), 0, s, h, w, eps, T, row_seq, amax, q8, a_rows, row_scale));
-  } else {
-    SG_DISPATCH_NPL(d, NPL,
-                    hipLaunchKernelGGL((k_norm_quantize<NPL / 4, false>), dim3(blocks_for(T, kRowsPerBlock)),
-                                       dim3(kThreads), 0, s, h, w, eps, T, row_seq, amax, q8, a_rows, row_scale));
+  if (rmax) {
+    if (!seq_off || !row_max_form(T, d)) return hipErrorInvalidValue;
+    SG_DISPATCH_NV(d, NV,
+                   hipLaunchKernelGGL(k_norm_quantize_wave<NV>, dim3(blocks_for(T, kWaveWaves)), dim3(kThreads), 0, s,
+                                      h, w, eps, T, row_seq, seq_off, rmax, q8, a_rows, row_scale));
+    return hipGetLastError();
   }
+  SG_DISPATCH_NPL(d, NPL,
+                  hipLaunchKernelGGL(k_norm_quantize<NPL / 4>, dim3(blocks_for(T, kRowsPerBlock)), dim3(kThreads), 0,
+                                     s, h, w, eps, T, row_seq, amax, q8, a_rows, row_scale));
   return hipGetLastError();
 }
 
@@ -803,22 +930,18 @@ hipError_t qknorm_rope(float* q, int ldq, float* k, int ldk, const float* qw, co
 }
 
 hipError_t post_res_norm(const float* o, float* h, const float* w_post, const float* w_next, float eps, int T, int d,
-                         float* xn, const int32_t* row_seq, float* amax, hipStream_t s) {
+                         float* xn, const int32_t* row_seq, float* amax, hipStream_t s, float* rmax) {
   if (T <= 0) return hipSuccess;
+  if (rmax) {
+    if (amax || !row_max_form(T, d)) return hipErrorInvalidValue;
+    SG_DISPATCH_NV(d, NV,
+                   hipLaunchKernelGGL(k_post_res_norm_wave<NV>, dim3(blocks_for(T, kWaveWaves)), dim3(kThreads), 0, s,
+                                      o, h, w_post, w_next, eps, T, xn, rmax));
+    return hipGetLastError();
+  }
   SG_DISPATCH_NPL(d, NPL,
                   hipLaunchKernelGGL(k_post_res_norm<NPL / 4>, dim3(blocks_for(T, kRowsPerBlock)), dim3(kThreads),
                                      0, s, o, h, w_post, w_next, eps, T, xn, row_seq, amax));
-  return hipGetLastError();
-}
-
-hipError_t post_res_norm_quantize(const float* o, float* h, const float* w_post, const float* w_next, float eps,
-                                  int T, int d, const int32_t* row_seq, float* amax, int8_t* q8, int a_rows,
-                                  float* row_scale, hipStream_t s) {
-  if (T <= 0) return hipSuccess;
-  if (!q8 || !row_scale || !w_next || a_rows < T) return hipErrorInvalidValue;
-  SG_DISPATCH_NPL(d, NPL,
-                  hipLaunchKernelGGL(k_post_res_norm_q<NPL / 4>, dim3(blocks_for(T, kRowsPerBlock)), dim3(kThreads),
-                                     0, s, o, h, w_post, w_next, eps, T, row_seq, amax, q8, a_rows, row_scale));
   return hipGetLastError();
 }
 

@@ -58,10 +58,9 @@ struct Meta {
   int Tp = 0;         // V^T columns: every sequence padded to whole 32-key tiles
   int max_len = 0;    // longest sequence
   double sum_sq = 0;  // sum over sequences of S^2 (attention work)
-  // Every sequence inside one row-kernel workgroup's rows / one attention
-  // work item: the post-norms and the attention then quantize the next GEMM
-  // operand themselves (the short-sequence serving case).
-  bool seq_in_row_block = false, seq_one_item = false;
+  // Every sequence inside one attention work item: the attention then quantizes
+  // the next GEMM operand itself (the short-sequence serving case).
+  bool seq_one_item = false;
   // Every sequence starts on a 32-row boundary (so the QKV GEMM's 32-row
   // subtiles are whole 32-key V^T tiles, except a last sequence's tail).
   bool seq_start32 = false;
@@ -183,10 +182,6 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
   m.n_items = n_items;
   m.n_vtiles = n_vt;
   m.seq_one_item = n_items == n_seq;
-  m.seq_in_row_block = true;
-  for (int i = 0; i < n_seq; i++)
-    if (off[i + 1] > off[i] && off[i] / sgk::kRowKernelRows != (off[i + 1] - 1) / sgk::kRowKernelRows)
-      m.seq_in_row_block = false;
   m.seq_start32 = true;
   for (int i = 0; i < n_seq; i++)
     if (off[i] % 32) m.seq_start32 = false;
@@ -358,7 +353,7 @@ struct Profiler {
 // stream of its own (created on first use, non-blocking, default priority) with
 // the event that joins it back to the caller's stream.
 struct Lane {
-  DevBuf h, xn, qkv, att, o, g, a8, sx, amax, meta_d, err;
+  DevBuf h, xn, qkv, att, o, g, a8, sx, amax, rmax, meta_d, err;
   DevBuf ks, vt;  // attention operands, hi/lo fp16 (K row-major; V^T); Q is split inside the attention kernel
   DevBuf qs;      // Q hi/lo for launches too small to fill the GPU (attn_q_presplit)
   DevBuf xp;      // exact-order attention: scores / weights [H][T][ldp] (SG_ATTN_EXACT only)
@@ -378,7 +373,7 @@ struct Lane {
     return SG_OK;
   }
   ~Lane() {
-    for (DevBuf* b : {&h, &xn, &qkv, &att, &o, &g, &a8, &sx, &amax, &meta_d, &err, &ks, &vt, &qs, &xp, &spill})
+    for (DevBuf* b : {&h, &xn, &qkv, &att, &o, &g, &a8, &sx, &amax, &rmax, &meta_d, &err, &ks, &vt, &qs, &xp, &spill})
       b->release();
     meta_h.release();
     io_h.release();
@@ -543,8 +538,10 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   const double attn_flops = 4.0 * c.num_heads * m->hd * meta.sum_sq;
   const double attn_bytes = t * (2.0 * qd + 2.0 * kvd) * 4.0;
   (void)attn_bytes;
+  // Small batches hand the pre-norms' maxima on row by row (sgk::row_max_form).
+  float* rmax = sgk::row_max_form(T, d) ? w.rmax.as<float>() : nullptr;
   auto norm_q = [&](const float* w, float* am) {
-    return sgk::norm_quantize(h, w, eps, T, d, meta.row_seq, am, a8, ar, sx, s);
+    return sgk::norm_quantize(h, w, eps, T, d, meta.row_seq, am, a8, ar, sx, s, rmax, meta.seq_off);
   };
   auto quant = [&](const float* x, int cols, float* am) {
     return sgk::quantize(x, cols, T, cols, meta.row_seq, am, a8, ar, nullptr, sx, s);
@@ -582,24 +579,16 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
     SG_LAUNCH(SG_K_OTHER, 4.0, sgk::fill_i32(w.err.as<int32_t>(), INT32_MAX, 1, s));
     SG_LAUNCH(SG_K_NORM, t * (34.0 * d / 32 + 4.0 * d),
               sgk::embed_norm(d_tokens, T, m->emb_q, m->emb_s, c.vocab_size, d, m->sqrt_d, m->layers[0].attn_norm,
-                              eps, meta.row_seq, h, nullptr, site(0, 0), w.err.as<int32_t>(), s));
+                              eps, meta.row_seq, h, nullptr, site(0, 0), w.err.as<int32_t>(), s, rmax));
   }
-  // Short sequences (each inside one row-kernel workgroup / attention item):
-  // the unfused post-norms quantize the next GEMM operand in the same launch,
-  // and the attention its own output, so the separate quantizer launches go.
-  // a8_ready: the operand of the next QKV GEMM is already in a8.
-  const bool q_rows = meta.seq_in_row_block;
+  // Short sequences (each one attention item): the attention quantizes its own
+  // output, so that quantizer launch goes.
   const bool q_attn = meta.seq_one_item && c.num_kv_heads == 1 && meta.max_len <= sgk::kAttnRegKeys;
-  bool a8_ready = false;
-  auto post_norm_q = [&](const float* w_post, const float* w_next, float* am) {
-    return sgk::post_res_norm_quantize(o, h, w_post, w_next, eps, T, d, meta.row_seq, am, a8, ar, sx, s);
-  };
   for (int l = l0; l < l1; l++) {
     if (l == stop) break;
     const LayerDev& ly = m->layers[l];
     // The pre-norm's output xn is never stored: recomputed from h while quantizing.
-    if (!a8_ready) SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(d), norm_q(ly.attn_norm, site(l, 0)));
-    a8_ready = false;
+    SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(d), norm_q(ly.attn_norm, site(l, 0)));
     SG_LAUNCH(SG_K_GEMM, gemm_ops(nqkv, d),
               sgk::gemm_q8(a8, ar, ly.wqkv, ly.sqkv, sx, qkv, nullptr, T, nqkv, d, s, true, vt_fused ? &vto : nullptr));
     if (tr && tr->qkv) SG_HIP(tap(tr->qkv, qkv, l, nqkv));
@@ -640,16 +629,13 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
       SG_LAUNCH(SG_K_GEMM_NORM, gemm_ops(d, qd),
                 sgk::gemm_q8_res_norm(a8, ar, ly.wo, ly.so, sx, o, T, d, qd, h, ly.post_attn, ly.ffn_norm, eps,
                                       nullptr, meta.row_seq, site(l, 2), s));
-    } else if (q_rows) {
-      SG_LAUNCH(SG_K_GEMM, gemm_ops(d, qd), gemm(ly.wo, ly.so, o, d, qd));
-      SG_LAUNCH(SG_K_NORM, t * d * 13.0, post_norm_q(ly.post_attn, ly.ffn_norm, site(l, 2)));
     } else {
       SG_LAUNCH(SG_K_GEMM, gemm_ops(d, qd), gemm(ly.wo, ly.so, o, d, qd));
       SG_LAUNCH(SG_K_NORM, t * d * 12.0,
-                sgk::post_res_norm(o, h, ly.post_attn, ly.ffn_norm, eps, T, d, nullptr, meta.row_seq, site(l, 2), s));
+                sgk::post_res_norm(o, h, ly.post_attn, ly.ffn_norm, eps, T, d, nullptr, meta.row_seq,
+                                   rmax ? nullptr : site(l, 2), s, rmax));
     }
-    if (!(q_rows && !sgk::gemm_res_norm_fused(T, d, ly.post_attn, ly.ffn_norm)))
-      SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(d), norm_q(ly.ffn_norm, site(l, 2)));
+    SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(d), norm_q(ly.ffn_norm, site(l, 2)));
     SG_LAUNCH(SG_K_GEMM, gemm_ops(2 * ff, d),
               sgk::gemm_q8_gelu(a8, ar, ly.wgu, ly.sgu, sx, g, T, ff, d, meta.row_seq, site(l, 3), s, true));
     SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(ff), quant(g, ff, site(l, 3)));
@@ -659,15 +645,11 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
       SG_LAUNCH(SG_K_GEMM_NORM, gemm_ops(d, ff),
                 sgk::gemm_q8_res_norm(a8, ar, ly.wd, ly.sd, sx, o, T, d, ff, h, ly.post_ffw, w_next, eps,
                                       last ? xn : nullptr, meta.row_seq, last ? nullptr : site(l + 1, 0), s));
-    } else if (q_rows && !last) {
-      SG_LAUNCH(SG_K_GEMM, gemm_ops(d, ff), gemm(ly.wd, ly.sd, o, d, ff));
-      SG_LAUNCH(SG_K_NORM, t * d * 13.0, post_norm_q(ly.post_ffw, w_next, site(l + 1, 0)));
-      a8_ready = true;
     } else {
       SG_LAUNCH(SG_K_GEMM, gemm_ops(d, ff), gemm(ly.wd, ly.sd, o, d, ff));
       SG_LAUNCH(SG_K_NORM, t * d * (last ? 16.0 : 12.0),
                 sgk::post_res_norm(o, h, ly.post_ffw, w_next, eps, T, d, last ? xn : nullptr, meta.row_seq,
-                                   last ? nullptr : site(l + 1, 0), s));
+                                   last || rmax ? nullptr : site(l + 1, 0), s, rmax));
     }
     if (tr && tr->h) SG_HIP(tap(tr->h, h, l, d));
   }
@@ -743,6 +725,7 @@ int ensure_workspace(const sg_model* m, Lane& w, const Meta& meta) {
   SG_TRY(w.a8.ensure((size_t)sgk::gemm_pad_rows(T) * a_cols));
   if (attn_q_presplit(m, meta)) SG_TRY(w.qs.ensure(2 * sizeof(_Float16) * t * m->qd));
   SG_TRY(w.sx.ensure(sizeof(float) * t));
+  if (sgk::row_max_form(T, c.embed_dim)) SG_TRY(w.rmax.ensure(sizeof(float) * t));
   SG_TRY(w.amax.ensure(sizeof(float) * 4 * (size_t)c.num_layers * n_seq));
   SG_TRY(w.ks.ensure(2 * sizeof(_Float16) * t * m->kvd));
   SG_TRY(w.vt.ensure(2 * sizeof(_Float16) * (size_t)m->kvd * Tp));

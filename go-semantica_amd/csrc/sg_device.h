@@ -367,6 +367,91 @@ __device__ __forceinline__ void sg_rmsnorm8_f4(f32x4_t (&x)[NC], const float* __
 }
 
 
+// Wave-per-row forms, for launches too small to fill the GPU with the 8-lane
+// groups above: lane l of the wave holds elements 256k + 4l .. + 3 (NV = n/256
+// float4 slots, 1 KB per load instruction), so a lane's elementwise work is an
+// eighth of a group lane's.  The sum of squares keeps the AVX2 lane order:
+// the row goes through an LDS tile laid out [8 lanes v][n/8 + 8] (element
+// 8i + v at v * stride + i; the writes of a wave and the reads of its eight
+// distinct rows fall in distinct banks), every lane reads its lane v = l & 7 in
+// order with float4 reads and runs that lane's chain, so one LDS round trip
+// serves the whole row instead of one per 32 elements.
+template <int NV>
+constexpr int kWaveTile = 8 * (32 * NV + 8);  // floats of one row's tile
+
+template <int NV>
+__device__ __forceinline__ void sg_wave_tile_put(const f32x4_t (&x)[NV], float* tile, int lane) {
+  constexpr int STR = 32 * NV + 8;
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) tile[(4 * (lane & 1) + t) * STR + 32 * k + (lane >> 1)] = x[k][t];
+  asm volatile("" ::: "memory");
+}
+
+// 1 / rms of the row in `tile` (written by this wave; the LDS operations of a
+// wave complete in issue order), as sg_rmsnorm8 forms it.
+// 1 / rms of the row in `tile` (written by this wave; the LDS operations of a
+// wave complete in issue order), as sg_rmsnorm8 forms it, in every lane.
+template <int NV>
+__device__ __forceinline__ float sg_wave_inv_rms(const float* tile, int lane, float eps) {
+  constexpr int STR = 32 * NV + 8;
+  const f32x4_t* rd = reinterpret_cast<const f32x4_t*>(tile + (lane & 7) * STR);
+  float acc = 0.0f;
+#pragma unroll
+  for (int m = 0; m < 8 * NV; m++) {
+    const f32x4_t a = rd[m];
+#pragma unroll
+    for (int t = 0; t < 4; t++) acc = __builtin_fmaf(a[t], a[t], acc);
+  }
+  asm volatile("" ::: "memory");
+  const float ms = sg_hsum8(acc) / (float)(NV * 256);
+  return 1.0f / sg_sqrt(ms + eps);
+}
+
+// x = (x * inv) * w on the wave layout.
+template <int NV>
+__device__ __forceinline__ void sg_wave_scale(f32x4_t (&x)[NV], float inv, const f32x4_t (&w)[NV]) {
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      const float u = x[k][t] * inv;
+      x[k][t] = u * w[k][t];
+    }
+}
+
+template <int NV>
+__device__ __forceinline__ void sg_wave_load(f32x4_t (&x)[NV], const float* __restrict__ p, int lane) {
+#pragma unroll
+  for (int k = 0; k < NV; k++) x[k] = *reinterpret_cast<const f32x4_t*>(p + 256 * k + 4 * lane);
+}
+
+template <int NV>
+__device__ __forceinline__ float sg_wave_absmax(const f32x4_t (&x)[NV]) {
+  float m = 0.0f;
+#pragma unroll
+  for (int k = 0; k < NV; k++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) m = fmaxf(m, fabsf(x[k][t]));
+  return m;
+}
+
+// The maximum of rmax[a .. b) (row maxima, non-negative), in every lane of the
+// wave.  Sixteen loads of a batch go out together.
+__device__ __forceinline__ float sg_wave_rows_max(const float* __restrict__ rmax, int a, int b, int lane) {
+  float m = 0.0f;
+  for (int r = a; r < b; r += 16 * SG_WAVE) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = rmax[min(r + SG_WAVE * u + lane, b - 1)];
+#pragma unroll
+    for (int u = 0; u < 16; u++) m = fmaxf(m, v[u]);
+  }
+  return sg_wave_max(m);
+}
+
 // The residual post-norm of one row whose o (x) and h (hv) are already in
 // the lanes of its 8-lane group (model_int8.go:203-210 / :225-232):
 // h = RMSNorm(o; w_post) + h, stored to hrow, then xn = RMSNorm(h; w_next),

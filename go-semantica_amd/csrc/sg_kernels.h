@@ -68,12 +68,19 @@ hipError_t fill_i32(int32_t* p, int32_t v, int64_t n, hipStream_t s);
 hipError_t first_bad_token(const int32_t* tokens, int T, int vocab, int32_t* first, hipStream_t s);
 
 // ---- per-row kernels (k_rows.hip) ----
+// Small launches (row_max_form(T, d)) can pass the rows' maxima on instead of
+// the sequences': embed_norm and post_res_norm with rmax != null write each
+// row's max|xn| to rmax[T] (amax null or unused), and norm_quantize with rmax
+// (and the CSR seq_off) takes each sequence's maximum over its rows.  The
+// atomics on amax cost ~13 ns each, one after another (the sequences' maxima
+// share a cache line): with a wave per row they were most of the kernel.
+bool row_max_form(int T, int d);
 // Embedding gather * sqrt(d) -> h; then RMSNorm(w) -> xn (stored when xn != null) and
 // per-sequence max|xn| -> amax.  A token outside [0, vocab) is read as token 0
 // and its row folded into *err by atomicMin (*err starts at INT32_MAX).
 hipError_t embed_norm(const int32_t* tokens, int T, const int8_t* eq, const float* es, int vocab, int d,
                       float sqrt_d, const float* w, float eps, const int32_t* row_seq, float* h, float* xn,
-                      float* amax, int32_t* err, hipStream_t s);
+                      float* amax, int32_t* err, hipStream_t s, float* rmax = nullptr);
 // Per-sequence symmetric quantization of x[rows][cols] (stride ldx) using amax[row_seq[r]].
 // Writes the int8 codes block-major q8[cols/32][a_rows][32] (q8 != null, the GEMM
 // operand) or row-major i8[rows][cols] (q8 == null), and row_scale[rows].
@@ -83,7 +90,8 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
 // formed it, quantized with amax[row_seq[r]] into the block-major int8 GEMM
 // operand q8[d/32][a_rows][32] and row_scale[T] (quantize's arithmetic).
 hipError_t norm_quantize(const float* h, const float* w, float eps, int T, int d, const int32_t* row_seq,
-                         const float* amax, int8_t* q8, int a_rows, float* row_scale, hipStream_t s);
+                         const float* amax, int8_t* q8, int a_rows, float* row_scale, hipStream_t s,
+                         const float* rmax = nullptr, const int32_t* seq_off = nullptr);
 hipError_t absmax_rows(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, float* amax,
                        hipStream_t s);
 hipError_t seq_scales(const float* amax, int n_seq, float* out, hipStream_t s);
@@ -101,18 +109,8 @@ hipError_t qknorm_rope(float* q, int ldq, float* k, int ldk, const float* qw, co
 // h = RMSNorm(o; w_post) + h ; xn = RMSNorm(h; w_next) (stored when xn != null) ;
 // amax (optional) per sequence of max|xn|.
 hipError_t post_res_norm(const float* o, float* h, const float* w_post, const float* w_next, float eps, int T,
-                         int d, float* xn, const int32_t* row_seq, float* amax, hipStream_t s);
-// Rows per workgroup of the row kernels (post_res_norm, norm_quantize, ...).
-constexpr int kRowKernelRows = 32;
-// post_res_norm, then xn quantized per sequence into the block-major GEMM
-// operand q8[d/32][a_rows][32] and row_scale[T] -- the values, scale and codes
-// norm_quantize would produce from the new h -- in one launch.  Valid only when
-// every sequence's rows lie inside one block of kRowKernelRows rows
-// (off[s] / kRowKernelRows == (off[s+1] - 1) / kRowKernelRows); amax (optional)
-// receives the sequences' max|xn| as post_res_norm leaves them.
-hipError_t post_res_norm_quantize(const float* o, float* h, const float* w_post, const float* w_next, float eps,
-                                  int T, int d, const int32_t* row_seq, float* amax, int8_t* q8, int a_rows,
-                                  float* row_scale, hipStream_t s);
+                         int d, float* xn, const int32_t* row_seq, float* amax, hipStream_t s,
+                         float* rmax = nullptr);
 // g = geluquick(gate)*up over rows x cols; amax (optional) per sequence of max|g|.
 hipError_t gelu_mul(float* g, int ldd, const float* gate, int ldg, const float* up, int ldu, int rows, int cols,
                     const int32_t* row_seq, float* amax, hipStream_t s);

@@ -613,6 +613,27 @@ def test_exact_attention_forward_ragged_k_blocks(gpu_ctx, oracle, interm):
         m.close()
 
 
+@pytest.mark.parametrize("embed_dim", [256, 512, 1024])
+def test_exact_attention_forward_other_widths(gpu_ctx, oracle, embed_dim):
+    """The wave-per-row kernels of small batches (embedding, post-norms,
+    norm-quantize, quantize) at the other widths they are built for: one, two
+    and four float4 slots per lane, with sequences of 1 row, of under and over
+    one wave's workgroup, and of more than the 1024 row maxima one batch of
+    loads covers.  Two layers, exact attention, bit-identical to the oracle's
+    block-serial forward."""
+    from semantica_gpu import Model, synth
+    cfg = dict(synth.EMBEDDINGGEMMA_300M, num_layers=2, vocab_size=4096, embed_dim=embed_dim,
+               num_heads=embed_dim // 256)
+    mdl = synth.make_model(cfg)
+    off = synth.offsets_from_lengths([1, 3, 33, 1100, 70])
+    toks = synth.token_ids(int(off[-1]), cfg["vocab_size"], 9)
+    gpu = Model(gpu_ctx, mdl)
+    try:
+        _exact_forward(gpu, oracle.OracleModel(mdl), toks, off, embed_dim, f"width {embed_dim}")
+    finally:
+        gpu.close()
+
+
 def test_exact_attention_forward_config4(full_gpu, full_oracle):
     """Config 4 at full size: 256 log-uniform lengths in [8, 512] (seed 1),
     Matryoshka dim 256, 24 layers, two sequence groups on two streams, exact
