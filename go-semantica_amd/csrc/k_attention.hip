@@ -25,8 +25,8 @@
 // fastExp argument and, through fastExp's polynomial error, the weights by
 // ~1e-5).
 //
-// Operands arrive already split (the QK-norm/RoPE kernel writes Q and K hi/lo,
-// k_v_split_t writes V^T hi/lo), so every workgroup only copies fp16 tiles.
+// Operands arrive already split, K and V in MFMA fragment order (sg_kv_prep.h),
+// so every workgroup only copies fp16 tiles.
 //
 // Work split.  The G query heads that share a kv head are stacked into
 // G*ceil(S/16) chunks of 16 (head, query) rows.  A workgroup is 8 waves, one
@@ -70,9 +70,9 @@ __device__ __forceinline__ void split_pair(float x0, float x1, float scale, uint
       : "v"(x0), "v"(x1), "s"(scale));
 }
 
-template <bool B>
-struct bool_c {
-  static constexpr bool value = B;
+template <int I>
+struct int_c {
+  static constexpr int value = I;
 };
 static_assert(sgk::kAttnChunkRows == kQW, "host chunking must match the kernel");
 
@@ -86,18 +86,23 @@ __device__ __forceinline__ f32x4_t mfma16(half8_t a, half8_t b, f32x4_t c) {
 
 constexpr int kRegTiles = sgk::kAttnRegKeys / kBK;
 
+// Offset of the Q fragments of rows q0 .. q0 + 15 of the sequence at padded key vo.
+__device__ __forceinline__ int64_t q_subtile(int head, int n_tiles, int vo, int q0) {
+  return ((int64_t)head * n_tiles + ((vo + q0) >> 5)) * sgd::kFragTile + sgd::kfrag_piece((q0 >> 4) & 1, 0, 0);
+}
+
 // Q^T as the B operand of one wave's 16 (head, query) rows: lane (query ln,
 // group g4), k-step ks holds dims 32ks + 8g4 .. + 7 of row qr, scaled by 8
 // and split hi/lo.  QPRE: Q arrives as the QKV GEMM's fp32 output and the wave
 // applies attn_q_norm and RoPE to its 16 rows itself (the arithmetic of
-// k_qknorm_rope_split, so the operands are bit-identical), which saves writing
+// sgd::qk_split_group, so the operands are bit-identical), which saves writing
 // Q's hi/lo operands and reading them back; tile: the wave's 16 x 40 floats
 // of LDS for the norm, wtile its 256 floats for the norm weights.  Otherwise
-// Q arrives split (qh, ql).
+// Q arrives split, qf the chunk's subtile of fragments.
 template <bool QPRE>
 __device__ __forceinline__ void q_operand(half8_t (&bqh)[kHD / 32], half8_t (&bql)[kHD / 32],
-                                          const _Float16* __restrict__ qh, const _Float16* __restrict__ ql, int ldq,
-                                          const sg_attn_qpre& qp, int qr, int pos, int head, int ln, int g4,
+                                          const _Float16* __restrict__ qf, const sg_attn_qpre& qp, int qr, int pos,
+                                          int head, int ln, int g4,
                                           int lane, float* tile, float* wtile) {
   if constexpr (QPRE) {
     // Every global load (the norm weights, Q, the RoPE table rows of the
@@ -194,16 +199,16 @@ __device__ __forceinline__ void q_operand(half8_t (&bqh)[kHD / 32], half8_t (&bq
       bql[ks] = __builtin_bit_cast(half8_t, ul);
     }
   } else {
-    const int64_t qo = (int64_t)qr * ldq + head * kHD + 8 * g4;
 #pragma unroll
     for (int ks = 0; ks < kHD / 32; ks++) {
-      bqh[ks] = *reinterpret_cast<const half8_t*>(qh + qo + 32 * ks);
-      bql[ks] = *reinterpret_cast<const half8_t*>(ql + qo + 32 * ks);
+      bqh[ks] = *reinterpret_cast<const half8_t*>(qf + sgd::kfrag_piece(0, ks, 0) + 8 * lane);
+      bql[ks] = *reinterpret_cast<const half8_t*>(qf + sgd::kfrag_piece(0, ks, 1) + 8 * lane);
     }
   }
 }
 
-constexpr int kTileBytes = 32 * 1024;  // one K or V^T tile, hi and lo halves
+constexpr int kTileBytes = 32 * 1024;  // one K or V tile, hi and lo halves
+static_assert(kTileBytes == 2 * sgd::kFragTile && sgk::kAttnTileHalves == sgd::kFragTile, "tile layout");
 constexpr int kRing = 3;               // tile stages in LDS
 constexpr int kScoreBytes = sgk::kAttnSpillTileBytes;  // one tile's scores, 8 floats per lane and wave
 static_assert(kScoreBytes == kWaves * 2048, "spill tile layout");
@@ -223,19 +228,13 @@ static_assert(kScoreBytes == kWaves * 2048, "spill tile layout");
 // and the barrier after it publishes every wave's copies and retires the
 // stage the next copies overwrite.
 //
-// LDS layouts, XOR-swizzled in 16-byte chunks so that the 16x16x32 fragment
-// reads (16 rows x 4 lane groups) hit distinct banks with unpadded rows:
-//   K stage:   row R = 32 hl + key (hl 0 hi, 1 lo), 512 B per row; chunk c
-//              (dims 8c .. 8c + 7) at position c ^ (R & 15).
-//   V^T stage: row d = dim, 128 B per row (hi keys then lo keys, the global
-//              layout); chunk c at position c ^ ((d >> 1) & 7).
-// A copy lane picks the global chunk its LDS position holds, so the swizzle
-// costs nothing at copy time; fragment addresses are one XOR per k-step.
+// A tile's LDS stage is its 32 KB of fragments as they lie in memory, so a copy
+// is 1 KB to 1 KB and a fragment read is the wave's lanes in order (no bank
+// conflicts, an immediate offset per fragment).
 template <bool QPRE, bool SPILL>
 __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
-    const _Float16* __restrict__ qh, const _Float16* __restrict__ ql, int ldq, const _Float16* __restrict__ kh,
-    const _Float16* __restrict__ kl, int ldk, const _Float16* __restrict__ vt, int ldvt, float* __restrict__ out,
-    int ldo, const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff, const sg_item* __restrict__ items,
+    const _Float16* __restrict__ qf, const _Float16* __restrict__ kf, const _Float16* __restrict__ vf, int n_tiles, float* __restrict__ out, int ldo,
+    const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff, const sg_item* __restrict__ items,
     int G, float sscale, float* __restrict__ amax, sg_attn_qpre qp, sg_attn_qout qo, sg_attn_spill sp) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[kRing * kTileBytes];
   __shared__ __attribute__((aligned(16))) unsigned char slds[SPILL ? kRing * kScoreBytes : 16];
@@ -262,47 +261,16 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
   const int qr = r0 + min(qrow, S - 1);
 
   // ---- copies ----
-  // Wave w's four copies of an item land at w * 4 KB + i * 1 KB of the stage.
-  // K item: copy i moves rows R = 8w + 2i and 8w + 2i + 1 (hi for waves 0-3,
-  // lo for waves 4-7); lane L takes row R = 8w + 2i + L / 32 and LDS position
-  // L % 32, i.e. global chunk (L % 32) ^ (R & 15).  Keys past the sequence's
-  // end are clamped to its last key and masked out of the scores below.
-  // V^T item: copy i moves dims 32w + 8i .. + 7; lane L takes dim
-  // d = 32w + 8i + L / 8, position L % 8, global chunk (L % 8) ^ ((d >> 1) & 7);
-  // every tile of a sequence lies inside its padded V^T columns.
-  const i32x4_t rk = sg_raw_rsrc((w < 4 ? kh : kl) + (int64_t)r0 * ldk + kvh * kHD);
-  const i32x4_t rv = sg_raw_rsrc(vt + (int64_t)kvh * kHD * ldvt + 2 * vo);
-  // Per-lane byte offsets, loop-invariant: K copy i at key row kkey(i) of a
-  // tile (kvo; the tile's first row goes in the scalar offset), V^T copy i
-  // (voffs; the tile's columns go in the scalar offset).
-  auto kkey = [&](int i) { return ((8 * w + 2 * i) & 31) + (lane >> 5); };
-  uint32_t kvo[4], voffs[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int R = 8 * w + 2 * i + (lane >> 5);
-    kvo[i] = (uint32_t)kkey(i) * (uint32_t)ldk * 2u + 16u * (uint32_t)((lane & 31) ^ (R & 15));
-    const int d = 32 * (w & 7) + 8 * i + (lane >> 3), cv = (lane & 7) ^ ((d >> 1) & 7);
-    voffs[i] = (uint32_t)d * (uint32_t)ldvt * 2u + 16u * (uint32_t)cv;
-  }
-  // This wave's four copies of K tile `tile` (isk) or V^T tile `tile` into the
-  // ring stage at dst.
+  // Wave w's four copies of an item: pieces 4w .. 4w + 3 of the tile.  Keys past
+  // the sequence's end hold whatever the buffer held; their scores are masked
+  // below (V's pad keys are zeros).
+  const int64_t tile0 = (int64_t)kvh * n_tiles + (vo >> 5);
+  const i32x4_t rk = sg_raw_rsrc(kf + tile0 * sgd::kFragTile);
+  const i32x4_t rv = sg_raw_rsrc(vf + tile0 * sgd::kFragTile);
   auto copy_tile = [&](uint32_t dst, bool isk, int tile) {
-    if (!isk) {  // V^T: the tile's columns, 64 halves per 32 keys
-      const uint32_t soff = (uint32_t)tile * kBK * 4u;
+    const uint32_t soff = (uint32_t)tile * kTileBytes + (uint32_t)w * 4096u;
 #pragma unroll
-      for (int i = 0; i < 4; i++) sg_lds_copy16(dst + 1024u * i, voffs[i], rv, soff);
-    } else if (tile * kBK + kBK <= S) {  // a whole K tile
-      const uint32_t soff = (uint32_t)(tile * kBK) * (uint32_t)ldk * 2u;
-#pragma unroll
-      for (int i = 0; i < 4; i++) sg_lds_copy16(dst + 1024u * i, kvo[i], rk, soff);
-    } else {  // a sequence's last K tile: rows past S re-read its last key
-      const int kt = tile * kBK;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int key = min(kt + kkey(i), S - 1);
-        sg_lds_copy16(dst + 1024u * i, kvo[i] + (uint32_t)(key - kkey(i)) * (uint32_t)ldk * 2u, rk, 0u);
-      }
-    }
+    for (int i = 0; i < 4; i++) sg_lds_copy16(dst + 1024u * i, 16u * lane, isk ? rk : rv, soff + 1024u * i);
   };
   // SPILL: this workgroup's spilled scores, nt - kRegTiles tiles of
   // kScoreBytes (wave w's 2 KB at w * 2048: lane l's keys 4g4 + r at 16 l,
@@ -342,20 +310,17 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
   // The Q prologue's LDS tiles sit in stage 2, which no copy touches before
   // the first barrier.
   static_assert(kWaves * (16 * 40 + kHD) * 4 <= kTileBytes, "prologue tiles fit stage 2");
-  q_operand<QPRE>(bqh, bql, qh, ql, ldq, qp, qr, qr - r0, head, ln, g4, lane,
+  q_operand<QPRE>(bqh, bql, QPRE ? nullptr : qf + q_subtile(head, n_tiles, vo, q0), qp, qr, qr - r0, head, ln, g4, lane,
                   reinterpret_cast<float*>(lds + 2 * kTileBytes) + w * (16 * 40),
                   reinterpret_cast<float*>(lds + 2 * kTileBytes) + kWaves * (16 * 40) + w * kHD);
 
   auto key_of = [&](int kt, int st, int r) { return kt + 16 * st + 4 * g4 + r; };
   // ---- pass 1: S^T = K Q^T per tile, kept in registers; row max ----
-  // K fragment (row R = 32 hl + 16 st + ln, chunk 4 ks + g4) at
-  // R * 512 + 16 * ((4 ks + g4) ^ ln) = (xk ^ 64 ks) + 8192 st + 16384 hl.
-  const uint32_t xk = (uint32_t)ln * 512u + 16u * (uint32_t)(g4 ^ (ln & 3)) + 64u * (uint32_t)(ln >> 2);
   auto scores2 = [&](const unsigned char* kb, f32x4_t& a0, f32x4_t& a1) {
+    const _Float16* kp = reinterpret_cast<const _Float16*>(kb) + 8 * lane;
     auto rd = [&](int st, int ks, half8_t& h, half8_t& l) {
-      const unsigned char* p = kb + (xk ^ (64u * ks)) + 8192 * st;
-      h = *reinterpret_cast<const half8_t*>(p);
-      l = *reinterpret_cast<const half8_t*>(p + 16384);
+      h = *reinterpret_cast<const half8_t*>(kp + sgd::kfrag_piece(st, ks, 0));
+      l = *reinterpret_cast<const half8_t*>(kp + sgd::kfrag_piece(st, ks, 1));
     };
     a0 = f32x4_t{0, 0, 0, 0};
     a1 = f32x4_t{0, 0, 0, 0};
@@ -447,20 +412,16 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
   m = fmaxf(m, __shfl_xor(m, 32));
 
   // ---- pass 2: e = fastExp(s - m), row sums, O^T += V^T P^T ----
-  // V^T fragment (dim 16 mt + ln, chunk g4 hi / 4 + g4 lo) at
-  // (16 mt + ln) * 128 + 16 * (chunk ^ ((ln >> 1) & 7)): xv (+ 64 for lo)
-  // + 2048 mt.
-  const uint32_t xv = (uint32_t)ln * 128u + 16u * (uint32_t)(g4 ^ ((ln >> 1) & 7));
   f32x4_t o[kHD / 16];
 #pragma unroll
   for (int mt = 0; mt < kHD / 16; mt++) o[mt] = f32x4_t{0, 0, 0, 0};
   float lsum = 0.0f;
   auto pv = [&](const unsigned char* vb, const half8_t& ph, const half8_t& pl) {
-    const unsigned char* p0 = vb + xv;
+    const _Float16* vp = reinterpret_cast<const _Float16*>(vb) + 8 * lane;
     half8_t fr[3][2];  // [buffer][hi, lo]
     auto rd = [&](int mt, half8_t(&f)[2]) {
-      f[0] = *reinterpret_cast<const half8_t*>(p0 + 2048 * mt);
-      f[1] = *reinterpret_cast<const half8_t*>(vb + ((xv ^ 64u) + 2048u * mt));
+      f[0] = *reinterpret_cast<const half8_t*>(vp + sgd::vfrag_piece(mt, 0));
+      f[1] = *reinterpret_cast<const half8_t*>(vp + sgd::vfrag_piece(mt, 1));
     };
     rd(0, fr[0]);
     rd(1, fr[1]);
@@ -575,25 +536,332 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
   }
 }
 
-// V^T split, one 32-key tile per workgroup (sgd::v_split_tile); kv head blockIdx.y.
-__global__ __launch_bounds__(sgd::kKvThreads) void k_v_split_t(const float* __restrict__ v, int ldv,
-                                                             const int32_t* __restrict__ seq_off,
-                                                             const int32_t* __restrict__ voff,
-                                                             const sg_item* __restrict__ vtiles,
-                                                             _Float16* __restrict__ vt, int ldvt) {
-  __shared__ __attribute__((aligned(16))) float tv[kBK][sgd::kVtRowStride];
-  sgd::v_split_tile(vtiles[blockIdx.x], blockIdx.y, tv, v, ldv, seq_off, voff, vt, ldvt);
+// ---- small launches ----
+//
+// A launch of few workgroups leaves most CUs idle in k_attn_rs: its wave walks
+// every key tile of its chunk alone, whatever else the GPU has to do (one
+// 512-token sequence: 12 workgroups, 47 us; here 18 us, of which ~8 us are
+// the megabyte of K and V fragments through each CU's 64 B/clk).  Here a workgroup's eight waves
+// share C chunks of 16 (head, query) rows instead: pass 1 deals the 16-key
+// subtiles to the waves, pass 2 the output dims, so a chunk's serial chain is
+// an eighth as long and there are 8 / C times the workgroups.  Every sum keeps
+// k_attn_rs's order -- a score's chain over the dims, a row sum's over the
+// tiles, an output's over the tiles -- so the results are the same bits.
+//   Pass 1: wave w scores subtiles w, w + 8, ...; K fragments come straight
+//           from global memory (this wave alone uses them), one subtile ahead;
+//           scores go to LDS (2 KB per tile), the row maximum is combined over
+//           the waves.
+//   exp:    each wave turns its own subtiles' scores into weights, in place.
+//   Pass 2: wave w owns dims 32 w .. + 31; V fragments straight from global
+//           memory, four to eight tiles ahead; every wave reads all weights,
+//           splits them and keeps the row sums (identical in all waves).
+// LDS holds every score (NT tiles), so nothing spills.  One workgroup per CU
+// (two waves per SIMD, up to 256 VGPRs for the fragments in flight).
+// The chunk maxima of |out| go to cmax (attn_cmax_base), not by atomics.
+//
+// Barrier over LDS only: loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
-// K's QK-norm/RoPE split and V's V^T split in one launch: workgroups
-// [0, nkb) take 32 (token, kv head) rows of K each, the rest one (V tile,
-// kv head) each, so the two halves' loads and stores overlap.
+template <int C, int NT>
+__global__ __launch_bounds__(kNT, 2) void k_attn_small(
+    const _Float16* __restrict__ qf, const _Float16* __restrict__ kf, const _Float16* __restrict__ vf,
+    int n_tiles, float* __restrict__ out, int ldo,
+    const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff, const sg_item* __restrict__ items,
+    int n_items, int npad, int G, float sscale, float* __restrict__ cmax) {
+  constexpr int NS = kHD / 32;  // k-steps
+  constexpr int KN = NS / C;    // k-steps per fragment load group (the Q operands of C chunks leave room for that)
+  __shared__ __attribute__((aligned(16))) f32x4_t sc[C][2 * NT][SG_WAVE];
+  __shared__ float red[C][kWaves][kQW];
+  static_assert(kHD == 32 * kWaves && (C == 1 || C == 2), "32 output dims per wave");
+  // Item k's workgroups are blocks k, k + npad, ...: the same XCD each (npad
+  // is a multiple of 8), so an item's K and V stay in one L2.
+  const int k_it = blockIdx.x % npad, kvh = blockIdx.y;
+  if (k_it >= n_items) return;
+  const sg_item it = items[k_it];
+  const int r0 = seq_off[it.seq];
+  const int S = seq_off[it.seq + 1] - r0;
+  const int vo = voff[it.seq];
+  const int64_t tile0 = (int64_t)kvh * n_tiles + (vo >> 5);
+  const int nqb = (S + kQW - 1) / kQW, nt = (S + kBK - 1) / kBK, nch = G * nqb;
+  const int c0 = it.c0 + C * (int)(blockIdx.x / npad);
+  if (c0 >= nch) return;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ln = lane & 15, g4 = lane >> 4;
+
+  half8_t bqh[C][NS], bql[C][NS];
+#pragma unroll
+  for (int j = 0; j < C; j++) {  // past the last chunk: that one again, never stored
+    const int c = min(c0 + j, nch - 1);
+    const _Float16* qp = qf + q_subtile(kvh * G + c / nqb, n_tiles, vo, (c % nqb) * kQW) + 8 * lane;
+#pragma unroll
+    for (int ks = 0; ks < NS; ks++) {
+      bqh[j][ks] = *reinterpret_cast<const half8_t*>(qp + sgd::kfrag_piece(0, ks, 0));
+      bql[j][ks] = *reinterpret_cast<const half8_t*>(qp + sgd::kfrag_piece(0, ks, 1));
+    }
+  }
+
+  // ---- pass 1 ----
+  struct KFrag {
+    half8_t h[KN], l[KN];
+  };
+  auto load_k = [&](KFrag& f, int u, int k0) {
+    const _Float16* kp = kf + (tile0 + (u >> 1)) * sgd::kFragTile + sgd::kfrag_piece(u & 1, k0, 0) + 8 * lane;
+#pragma unroll
+    for (int ks = 0; ks < KN; ks++) {
+      f.h[ks] = *reinterpret_cast<const half8_t*>(kp + sgd::kfrag_piece(0, ks, 0));
+      f.l[ks] = *reinterpret_cast<const half8_t*>(kp + sgd::kfrag_piece(0, ks, 1));
+    }
+  };
+  float m[C];
+  f32x4_t a[C];
+#pragma unroll
+  for (int j = 0; j < C; j++) m[j] = -INFINITY;
+  auto clear = [&]() {
+#pragma unroll
+    for (int j = 0; j < C; j++) a[j] = f32x4_t{0, 0, 0, 0};
+  };
+  auto dot = [&](const KFrag& f, auto k0c) {
+    constexpr int K0 = decltype(k0c)::value;
+#pragma unroll
+    for (int ks = 0; ks < KN; ks++) {
+#pragma unroll
+      for (int j = 0; j < C; j++) a[j] = mfma16(f.h[ks], bqh[j][K0 + ks], a[j]);
+#pragma unroll
+      for (int j = 0; j < C; j++) a[j] = mfma16(f.h[ks], bql[j][K0 + ks], a[j]);
+#pragma unroll
+      for (int j = 0; j < C; j++) a[j] = mfma16(f.l[ks], bqh[j][K0 + ks], a[j]);
+    }
+  };
+  auto keep = [&](int u) {
+    const int k0 = 16 * u + 4 * g4;  // keys past S are masked
+#pragma unroll
+    for (int j = 0; j < C; j++) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        a[j][r] = k0 + r < S ? a[j][r] * sscale : -INFINITY;
+        m[j] = fmaxf(m[j], a[j][r]);
+      }
+      sc[j][u][lane] = a[j];
+    }
+  };
+  // The prefetches are unconditional (past the last subtile they re-load it).
+  KFrag f0, f1;
+  const int last = 2 * nt - 1;
+  load_k(f0, min(w, last), 0);
+  if constexpr (C == 1) {
+#pragma unroll 1
+    for (int u = w; u <= last; u += 2 * kWaves) {
+      load_k(f1, min(u + kWaves, last), 0);
+      __builtin_amdgcn_sched_barrier(0);
+      clear();
+      dot(f0, int_c<0>{});
+      keep(u);
+      load_k(f0, min(u + 2 * kWaves, last), 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (u + kWaves <= last) {
+        clear();
+        dot(f1, int_c<0>{});
+        keep(u + kWaves);
+      }
+    }
+  } else {
+#pragma unroll 1
+    for (int u = w; u <= last; u += kWaves) {
+      load_k(f1, u, KN);
+      __builtin_amdgcn_sched_barrier(0);
+      clear();
+      dot(f0, int_c<0>{});
+      load_k(f0, min(u + kWaves, last), 0);
+      __builtin_amdgcn_sched_barrier(0);
+      dot(f1, int_c<KN>{});
+      keep(u);
+    }
+  }
+
+  // V fragments of tiles t0 .. + 3: dim groups 2 w + i, hi (0) and lo (1).
+  struct VFrag {
+    half8_t v[4][2][2];
+  };
+  const _Float16* vp = vf + tile0 * sgd::kFragTile + sgd::vfrag_piece(2 * w, 0) + 8 * lane;
+  auto load_v = [&](VFrag& f, int t0) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const _Float16* p = vp + (int64_t)min(t0 + u, nt - 1) * sgd::kFragTile;
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        f.v[u][i][0] = *reinterpret_cast<const half8_t*>(p + sgd::vfrag_piece(i, 0));
+        f.v[u][i][1] = *reinterpret_cast<const half8_t*>(p + sgd::vfrag_piece(i, 1));
+      }
+    }
+  };
+  VFrag v0, v1;
+  load_v(v0, 0);
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    m[j] = fmaxf(m[j], __shfl_xor(m[j], 16));
+    m[j] = fmaxf(m[j], __shfl_xor(m[j], 32));
+    if (g4 == 0) red[j][w][ln] = m[j];
+  }
+  lds_barrier();
+#pragma unroll
+  for (int j = 0; j < C; j++)
+#pragma unroll
+    for (int i = 0; i < kWaves; i++) m[j] = fmaxf(m[j], red[j][i][ln]);
+
+  // ---- weights: this wave's subtiles ----
+#pragma unroll 1
+  for (int u = w; u <= last; u += kWaves)
+#pragma unroll
+    for (int j = 0; j < C; j++) {
+      f32x4_t e = sc[j][u][lane];
+#pragma unroll
+      for (int r = 0; r < 4; r++) e[r] = sg_fast_exp_nonpos(e[r] - m[j]);
+      sc[j][u][lane] = e;
+    }
+  lds_barrier();
+
+  // ---- pass 2 ----
+  f32x4_t o[C][2];
+  float lsum[C];
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    o[j][0] = o[j][1] = f32x4_t{0, 0, 0, 0};
+    lsum[j] = 0.0f;
+  }
+  auto group = [&](const VFrag& f, int t0) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      if (t0 + u >= nt) break;
+#pragma unroll
+      for (int j = 0; j < C; j++) {
+        const f32x4_t e0 = sc[j][2 * (t0 + u)][lane], e1 = sc[j][2 * (t0 + u) + 1][lane];
+        const float e[8] = {e0[0], e0[1], e0[2], e0[3], e1[0], e1[1], e1[2], e1[3]};
+#pragma unroll
+        for (int k = 0; k < 8; k++) lsum[j] = lsum[j] + e[k];
+        u32x4_t uh, ul;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+          uint32_t h, l;
+          split_pair(e[2 * k], e[2 * k + 1], kPScale, h, l);
+          uh[k] = h;
+          ul[k] = l;
+        }
+        const half8_t ph = __builtin_bit_cast(half8_t, uh), pl = __builtin_bit_cast(half8_t, ul);
+#pragma unroll
+        for (int i = 0; i < 2; i++) o[j][i] = mfma16(f.v[u][i][0], ph, o[j][i]);
+#pragma unroll
+        for (int i = 0; i < 2; i++) o[j][i] = mfma16(f.v[u][i][0], pl, o[j][i]);
+#pragma unroll
+        for (int i = 0; i < 2; i++) o[j][i] = mfma16(f.v[u][i][1], ph, o[j][i]);
+      }
+    }
+  };
+#pragma unroll 1
+  for (int t0 = 0; t0 < nt; t0 += 8) {
+    load_v(v1, t0 + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    group(v0, t0);
+    load_v(v0, t0 + 8);
+    __builtin_amdgcn_sched_barrier(0);
+    group(v1, t0 + 4);
+  }
+
+  // O^T: lane holds query ln, dims 32 w + 16 i + 4 g4 + r.
+#pragma unroll
+  for (int j = 0; j < C; j++) {
+    lsum[j] = lsum[j] + __shfl_xor(lsum[j], 16);
+    lsum[j] = lsum[j] + __shfl_xor(lsum[j], 32);
+    const float f = (1.0f / lsum[j]) * kPUnscale;
+    const int c = min(c0 + j, nch - 1), qrow = (c % nqb) * kQW + ln;
+    float mx = 0.0f;
+    if (c0 + j < nch && qrow < S) {
+      float* op = out + (int64_t)(r0 + qrow) * ldo + (kvh * G + c / nqb) * kHD + 32 * w + 4 * g4;
+#pragma unroll
+      for (int i = 0; i < 2; i++) {
+        f32x4_t y;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          y[r] = o[j][i][r] * f;
+          mx = fmaxf(mx, fabsf(y[r]));
+        }
+        *reinterpret_cast<f32x4_t*>(op + 16 * i) = y;
+      }
+    }
+    if (cmax) {
+      mx = sg_wave_max(mx);
+      if (lane == 0) red[j][w][0] = mx;  // the row maxima were read before the weights' barrier
+    }
+  }
+  if (!cmax) return;
+  lds_barrier();
+  if (threadIdx.x < C && c0 + (int)threadIdx.x < nch) {
+    float mm = red[threadIdx.x][0][0];
+#pragma unroll
+    for (int i = 1; i < kWaves; i++) mm = fmaxf(mm, red[threadIdx.x][i][0]);
+    cmax[sgk::attn_cmax_base(r0, it.seq, G * gridDim.y) + kvh * nch + c0 + threadIdx.x] = mm;
+  }
+}
+
+// The fragments of already normed and rotated Q, K and of V in one launch: a
+// workgroup per 32-key tile and operand head (query heads, kv heads of K, of
+// V).  Q and K: a wave per 16-key subtile and half of the dims, lane l fragment
+// lane l, so every store is 1 KB contiguous; pad keys repeat the last one.
+__global__ __launch_bounds__(sgd::kKvThreads) void k_qkv_split(
+    const float* __restrict__ q, int ldq, const float* __restrict__ k, const float* __restrict__ v, int ldkv, int H,
+    int HKV, const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff,
+    const sg_item* __restrict__ vtiles, _Float16* __restrict__ qf, _Float16* __restrict__ kf,
+    _Float16* __restrict__ vf, int n_tiles) {
+  __shared__ __attribute__((aligned(16))) float tv[kBK][sgd::kVtRowStride];
+  const sg_item t = vtiles[blockIdx.x];
+  const int y = blockIdx.y;
+  if (y >= H + HKV) {  // workgroup-uniform
+    sgd::v_split_tile(t, y - H - HKV, tv, v, ldkv, seq_off, voff, vf, n_tiles);
+    return;
+  }
+  const int h = y < H ? y : y - H;
+  const float* x0 = y < H ? q : k;
+  const int ld = y < H ? ldq : ldkv;
+  const int lane = threadIdx.x & 63, st = (threadIdx.x >> 6) & 1, k0 = 4 * (threadIdx.x >> 7);
+  const int r0 = seq_off[t.seq], S = seq_off[t.seq + 1] - r0;
+  const int key = min(t.c0 + 16 * st + (lane & 15), S - 1);
+  const float* src = x0 + (int64_t)(r0 + key) * ld + h * kHD + 32 * k0 + 8 * (lane >> 4);
+  _Float16* dst = (y < H ? qf : kf) + ((int64_t)h * n_tiles + (voff[t.seq] + t.c0) / kBK) * sgd::kFragTile +
+                  sgd::kfrag_piece(st, 0, 0) + k0 * 1024 + 8 * lane;
+  f32x4_t x[4][2];
+#pragma unroll
+  for (int ks = 0; ks < 4; ks++) {
+    x[ks][0] = *reinterpret_cast<const f32x4_t*>(src + 32 * ks);
+    x[ks][1] = *reinterpret_cast<const f32x4_t*>(src + 32 * ks + 4);
+  }
+#pragma unroll
+  for (int ks = 0; ks < 4; ks++) {
+    u32x4_t uh, ul;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      uint32_t hi, lo;
+      split_pair(x[ks][i >> 1][2 * (i & 1)], x[ks][i >> 1][2 * (i & 1) + 1], kQKScale, hi, lo);
+      uh[i] = hi;
+      ul[i] = lo;
+    }
+    *reinterpret_cast<u32x4_t*>(dst + sgd::kfrag_piece(0, ks, 0)) = uh;
+    *reinterpret_cast<u32x4_t*>(dst + sgd::kfrag_piece(0, ks, 1)) = ul;
+  }
+}
+
+// K's QK-norm/RoPE split and V's split in one launch: workgroups [0, nkb) take
+// 32 (token, head) rows of K (and Q) each, the rest one (V tile, kv head)
+// each, so the two halves' loads and stores overlap.
 __global__ __launch_bounds__(sgd::kKvThreads) void k_kv_prep(
     const float* __restrict__ k, const float* __restrict__ v, int ldkv, const float* __restrict__ kw, int HKV, int T,
     const int32_t* __restrict__ row_pos, const float* __restrict__ cos_t, const float* __restrict__ sin_t, float eps,
-    _Float16* __restrict__ ks_h, _Float16* __restrict__ ks_l, int ldks, int nkb, const int32_t* __restrict__ seq_off,
-    const int32_t* __restrict__ voff, const sg_item* __restrict__ vtiles, int n_vtiles, _Float16* __restrict__ vt, int ldvt,
-    sgk::sg_kv_q qp) {
+    const int32_t* __restrict__ row_key, _Float16* __restrict__ kf, int nkb, const int32_t* __restrict__ seq_off,
+    const int32_t* __restrict__ voff, const sg_item* __restrict__ vtiles, int n_vtiles, _Float16* __restrict__ vf,
+    int n_tiles, sgk::sg_kv_q qp) {
   __shared__ __attribute__((aligned(16))) float tv[kBK][sgd::kVtRowStride];
   const int b = blockIdx.x;
   if (b < nkb) {  // workgroup-uniform
@@ -603,29 +871,10 @@ __global__ __launch_bounds__(sgd::kKvThreads) void k_kv_prep(
     // 0) the Q arguments are never read; they then point at K (passing null
     // for them crashed this compiler's device pass).
     sgd::qk_split_group(g, threadIdx.x & 7, (threadIdx.x >> 3) & 7, tile, qp.q, qp.ldq, k, ldkv, qp.qw, kw, qp.H,
-                        HKV, T, row_pos, cos_t, sin_t, eps, qp.qs_h, qp.qs_l, qp.ldqs, ks_h, ks_l, ldks);
+                        HKV, T, row_pos, cos_t, sin_t, eps, qp.qf, row_key, kf, n_tiles);
   } else {
     const int vb = b - nkb;
-    sgd::v_split_tile(vtiles[vb % n_vtiles], vb / n_vtiles, tv, v, ldkv, seq_off, voff, vt, ldvt);
-  }
-}
-
-// Rows of x (fp32) -> hi/lo fp16 of x*scale.
-__global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x, int ldx, int cols, float scale,
-                                                    _Float16* __restrict__ hi, _Float16* __restrict__ lo,
-                                                    int ldo) {
-  const int row = blockIdx.x;
-  for (int c4 = threadIdx.x; c4 < cols / 4; c4 += 256) {
-    const f32x4_t a = *reinterpret_cast<const f32x4_t*>(x + (int64_t)row * ldx + 4 * c4);
-    half4_t vh, vl;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const hl16 s = split_f16(a[j] * scale);
-      vh[j] = s.hi;
-      vl[j] = s.lo;
-    }
-    *reinterpret_cast<half4_t*>(hi + (int64_t)row * ldo + 4 * c4) = vh;
-    *reinterpret_cast<half4_t*>(lo + (int64_t)row * ldo + 4 * c4) = vl;
+    sgd::v_split_tile(vtiles[vb % n_vtiles], vb / n_vtiles, tv, v, ldkv, seq_off, voff, vf, n_tiles);
   }
 }
 
@@ -633,27 +882,27 @@ __global__ __launch_bounds__(256) void k_split_rows(const float* __restrict__ x,
 
 namespace sgk {
 
-hipError_t v_split_t(const float* v, int ldv, const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles,
-                     int n_vtiles, int HKV, _Float16* vt, int ldvt, hipStream_t s) {
+hipError_t qkv_split(const float* q, int ldq, const float* k, const float* v, int ldkv, int H, int HKV,
+                     const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* qf,
+                     _Float16* kf, _Float16* vf, int n_tiles, hipStream_t s) {
   if (n_vtiles <= 0) return hipSuccess;
-  if ((ldv & 3) || (ldvt & 7)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_v_split_t, dim3(n_vtiles, HKV), dim3(256), 0, s, v, ldv, seq_off, voff, vtiles, vt,
-                     ldvt);
+  if ((ldq & 3) || (ldkv & 3) || H <= 0 || HKV <= 0 || H + 2 * HKV > 65535) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_qkv_split, dim3(n_vtiles, H + 2 * HKV), dim3(sgd::kKvThreads), 0, s, q, ldq, k, v, ldkv, H, HKV,
+                     seq_off, voff, vtiles, qf, kf, vf, n_tiles);
   return hipGetLastError();
 }
 
 hipError_t kv_prep(const float* k, const float* v, int ldkv, const float* kw, int HKV, int T, const int32_t* row_pos,
-                   const float* cos_t, const float* sin_t, float eps, _Float16* ks_h, _Float16* ks_l, int ldks,
-                   const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* vt, int ldvt, hipStream_t s,
-                   const sg_kv_q* qpart) {
+                   const float* cos_t, const float* sin_t, float eps, const int32_t* row_key, _Float16* kf,
+                   const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* vf,
+                   int n_tiles, hipStream_t s, const sg_kv_q* qpart) {
   if (T <= 0 || n_vtiles < 0 || HKV <= 0) return hipSuccess;
-  if ((ldkv & 3) || (ldks & 7) || (ldvt & 7) || (reinterpret_cast<uintptr_t>(k) & 15) ||
-      (reinterpret_cast<uintptr_t>(v) & 15) || (kw && (reinterpret_cast<uintptr_t>(kw) & 15)))
+  if ((ldkv & 3) || (reinterpret_cast<uintptr_t>(k) & 15) || (reinterpret_cast<uintptr_t>(v) & 15) ||
+      (kw && (reinterpret_cast<uintptr_t>(kw) & 15)))
     return hipErrorInvalidValue;  // float4 loads of K and V rows and of the weights
-  sgk::sg_kv_q qp{k, ldkv, kw, 0, ks_h, ks_l, ldks};
+  sgk::sg_kv_q qp{k, ldkv, kw, 0, kf};
   if (qpart && qpart->H > 0) {
-    if (!qpart->q || !qpart->qs_h || !qpart->qs_l || (qpart->ldq & 3) || (qpart->ldqs & 7) ||
-        (reinterpret_cast<uintptr_t>(qpart->q) & 15) || (qpart->qw && (reinterpret_cast<uintptr_t>(qpart->qw) & 15)))
+    if (!qpart->q || !qpart->qf || (qpart->ldq & 3) || (reinterpret_cast<uintptr_t>(qpart->q) & 15) || (qpart->qw && (reinterpret_cast<uintptr_t>(qpart->qw) & 15)))
       return hipErrorInvalidValue;  // float4 loads of the Q rows and weights, 16-byte split stores
     qp = *qpart;
   }
@@ -661,32 +910,53 @@ hipError_t kv_prep(const float* k, const float* v, int ldkv, const float* kw, in
   const int64_t nb = nkb + (int64_t)n_vtiles * HKV;
   if (nb > INT32_MAX) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_kv_prep, dim3((unsigned)nb), dim3(sgd::kKvThreads), 0, s, k, v, ldkv, kw, HKV, T, row_pos, cos_t,
-                     sin_t, eps, ks_h, ks_l, ldks, (int)nkb, seq_off, voff, vtiles, n_vtiles, vt, ldvt, qp);
-  return hipGetLastError();
-}
-
-hipError_t split_rows(const float* x, int ldx, int rows, int cols, float scale, _Float16* hi, _Float16* lo, int ldo,
-                      hipStream_t s) {
-  if (rows <= 0) return hipSuccess;
-  if ((ldx & 3) || (cols & 3) || (ldo & 3)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_split_rows, dim3(rows), dim3(256), 0, s, x, ldx, cols, scale, hi, lo, ldo);
+                     sin_t, eps, row_key, kf, (int)nkb, seq_off, voff, vtiles, n_vtiles, vf, n_tiles, qp);
   return hipGetLastError();
 }
 
 namespace {
+template <int C, int NT>
+void launch_small(int n_items, int HKV, hipStream_t s, const _Float16* qf, const _Float16* kf,
+                  const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off,
+                  const int32_t* voff, const sg_item* items, int G, float sscale, float* cmax) {
+  const int npad = (n_items + 7) & ~7;
+  hipLaunchKernelGGL((k_attn_small<C, NT>), dim3(npad * (kWaves / C), HKV), dim3(kNT), 0, s, qf, kf, vf, n_tiles, out, ldo,
+                     seq_off, voff, items, n_items, npad, G, sscale, cmax);
+}
+
 template <bool QPRE, bool SPILL>
-void launch_attn(dim3 grid, hipStream_t s, const _Float16* qh, const _Float16* ql, int ldq, const _Float16* kh,
-                 const _Float16* kl, int ldk, const _Float16* vt, int ldvt, float* out, int ldo,
-                 const int32_t* seq_off, const int32_t* voff, const sg_item* items, int G, float sscale, float* amax,
+void launch_attn(dim3 grid, hipStream_t s, const _Float16* qf, const _Float16* kf,
+                 const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off, const int32_t* voff, const sg_item* items, int G, float sscale, float* amax,
                  const sg_attn_qpre& qp, const sg_attn_qout& qo, const sg_attn_spill& sp) {
-  hipLaunchKernelGGL((k_attn_rs<QPRE, SPILL>), grid, dim3(kNT), 0, s, qh, ql, ldq, kh, kl, ldk, vt, ldvt, out, ldo,
-                     seq_off, voff, items, G, sscale, amax, qp, qo, sp);
+  hipLaunchKernelGGL((k_attn_rs<QPRE, SPILL>), grid, dim3(kNT), 0, s, qf, kf, vf, n_tiles, out, ldo, seq_off,
+                     voff, items, G, sscale, amax, qp, qo, sp);
 }
 }  // namespace
 
-hipError_t attention(const _Float16* qh, const _Float16* ql, int ldq, const _Float16* kh, const _Float16* kl, int ldk,
-                     const _Float16* vt, int ldvt, float* out, int ldo, const int32_t* seq_off,
-                     const int32_t* voff, const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
+bool attn_small_form(int n_items, int HKV, int max_len) {
+  return (int64_t)n_items * HKV <= kAttnSmallItems && max_len <= kAttnSmallKeys;
+}
+
+hipError_t attention_small(const _Float16* qf, const _Float16* kf, const _Float16* vf, int n_tiles,
+                           float* out, int ldo, const int32_t* seq_off, const int32_t* voff,
+                           const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
+                           float* cmax, int max_len, hipStream_t s) {
+  if (n_items <= 0) return hipSuccess;
+  if (hd != kHD || HKV <= 0 || H % HKV || max_len <= 0 || !attn_small_form(n_items, HKV, max_len))
+    return hipErrorInvalidValue;
+  if (!qf || (ldo & 3)) return hipErrorInvalidValue;  // float4 stores
+  const float sscale = scale / (kQKScale * kQKScale);
+  using fn = void (*)(int, int, hipStream_t, const _Float16*, const _Float16*, const _Float16*, int, float*, int, const int32_t*, const int32_t*, const sg_item*, int, float, float*);
+  const bool two = max_len <= 1024 && (int64_t)n_items * HKV > kAttnSmallOneItems;
+  const fn f = max_len <= 512    ? (two ? launch_small<2, 16> : launch_small<1, 16>)
+               : max_len <= 1024 ? (two ? launch_small<2, 32> : launch_small<1, 32>)
+                                 : launch_small<1, 64>;
+  f(n_items, HKV, s, qf, kf, vf, n_tiles, out, ldo, seq_off, voff, items, H / HKV, sscale, cmax);
+  return hipGetLastError();
+}
+
+hipError_t attention(const _Float16* qf, const _Float16* kf, const _Float16* vf, int n_tiles,
+                     float* out, int ldo, const int32_t* seq_off, const int32_t* voff, const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
                      float* amax, int max_len, hipStream_t s, const sg_attn_qpre* qpre,
                      const sg_attn_qout* qout, const sg_attn_spill* spill) {
   if (n_items <= 0) return hipSuccess;
@@ -697,7 +967,7 @@ hipError_t attention(const _Float16* qh, const _Float16* ql, int ldq, const _Flo
                (H / HKV) * ((max_len + kQW - 1) / kQW) > kWaves))
     return hipErrorInvalidValue;
   const sg_attn_qout qo = qout ? *qout : sg_attn_qout{nullptr, 0, nullptr};
-  if ((ldk | ldvt) & 7 || (ldo & 3)) return hipErrorInvalidValue;
+  if (ldo & 3) return hipErrorInvalidValue;
   static_assert(kBK == 32 && kRegTiles == sgk::kAttnRegKeys / 32, "attention_spill_tiles");
   const bool spills = attention_spill_tiles(max_len) > 0;
   if (spills && (!spill || !spill->buf || !spill->off || spill->total <= 0 ||
@@ -713,15 +983,14 @@ hipError_t attention(const _Float16* qh, const _Float16* ql, int ldq, const _Flo
         (reinterpret_cast<uintptr_t>(qpre->cos_t) & 15) || (reinterpret_cast<uintptr_t>(qpre->sin_t) & 15))
       return hipErrorInvalidValue;  // float4 loads of Q rows, weights and table rows
     qp = *qpre;
-  } else if (ldq & 7) {
+  } else if (!qf) {
     return hipErrorInvalidValue;
   }
-  using fn = void (*)(dim3, hipStream_t, const _Float16*, const _Float16*, int, const _Float16*, const _Float16*, int,
-                      const _Float16*, int, float*, int, const int32_t*, const int32_t*, const sg_item*, int, float,
+  using fn = void (*)(dim3, hipStream_t, const _Float16*, const _Float16*, const _Float16*, int, float*, int, const int32_t*, const int32_t*, const sg_item*, int, float,
                       float*, const sg_attn_qpre&, const sg_attn_qout&, const sg_attn_spill&);
   static const fn table[2][2] = {{launch_attn<false, false>, launch_attn<false, true>},
                                  {launch_attn<true, false>, launch_attn<true, true>}};
-  table[qpre != nullptr][spills](grid, s, qh, ql, ldq, kh, kl, ldk, vt, ldvt, out, ldo, seq_off, voff, items, H / HKV,
+  table[qpre != nullptr][spills](grid, s, qf, kf, vf, n_tiles, out, ldo, seq_off, voff, items, H / HKV,
                                  sscale, amax, qp, qo, sp);
   return hipGetLastError();
 }

@@ -133,13 +133,13 @@ __device__ __forceinline__ void store_subtile(float* stage, const float (&v)[16]
   }
 }
 
-// One 32 x 32 subtile of V (tokens row0 .., dims dim0 ..) into V^T, through
-// the wave's LDS slice.  A subtile whose 32 tokens are one whole 32-key tile
-// of a sequence (the usual case for sequences that start on a 32-row
-// boundary) goes out as 16-byte hi and lo chunks: lane l covers dim l % 32,
-// positions 8c .. 8c + 7 (c = 2 (l / 32), + 1), each position p holding key
-// vt_key(p), 128 contiguous bytes per dim.  Any other subtile is written value
-// by value at its key's tile and position.
+// One 32 x 32 subtile of V (tokens row0 .., dims dim0 ..) into V's attention
+// fragments (sg_kv_prep.h), through the wave's LDS slice.  A subtile whose 32
+// tokens are one whole 32-key tile of a sequence (the usual case for sequences
+// that start on a 32-row boundary) goes out as 16-byte hi and lo fragments:
+// lane l covers dim l % 32, key chunks c = 2 (l / 32), + 1, each position p
+// holding key vt_key(p), 256 contiguous bytes per 16 lanes.  Any other subtile
+// is written value by value at its key's tile and position.
 __device__ __forceinline__ void store_vt_subtile(float* stage, const float (&v)[16], const sg_vt_out& vo, int row0,
                                                  int dim0, int rows, int lr, int lh, int lane) {
 #pragma unroll
@@ -149,7 +149,9 @@ __device__ __forceinline__ void store_vt_subtile(float* stage, const float (&v)[
   const int key0 = row0 - vo.seq_off[s0];
   const bool whole = (key0 & 31) == 0 && row0 + 31 < rows && vo.row_seq[row0 + 31] == s0;  // wave-uniform
   if (whole) {
-    _Float16* base = vo.vt + ((dim0 + dim) * vo.ldvt + 2 * (vo.voff[s0] + key0));  // < 2^31 (checked at launch)
+    const int dg = dim0 + dim;  // offsets < 2^31 (checked at launch)
+    _Float16* base = vo.vf + (((dg >> 8) * vo.n_tiles + ((vo.voff[s0] + key0) >> 5)) * sgd::kFragTile +
+                              sgd::vfrag_piece((dg & 255) >> 4, 0) + (dg & 15) * 8);
 #pragma unroll 1
     for (int cc = 0; cc < 2; cc++) {
       const int c = 2 * (lane >> 5) + cc;
@@ -166,8 +168,8 @@ __device__ __forceinline__ void store_vt_subtile(float* stage, const float (&v)[
         hw[m] = hb[0] | (hb[1] << 16);
         lw[m] = lb[0] | (lb[1] << 16);
       }
-      *reinterpret_cast<uint4*>(base + 8 * c) = uint4{hw[0], hw[1], hw[2], hw[3]};
-      *reinterpret_cast<uint4*>(base + 32 + 8 * c) = uint4{lw[0], lw[1], lw[2], lw[3]};
+      *reinterpret_cast<uint4*>(base + 128 * c) = uint4{hw[0], hw[1], hw[2], hw[3]};
+      *reinterpret_cast<uint4*>(base + 128 * c + 512) = uint4{lw[0], lw[1], lw[2], lw[3]};
     }
   } else {
 #pragma unroll 1
@@ -176,10 +178,12 @@ __device__ __forceinline__ void store_vt_subtile(float* stage, const float (&v)[
       if (t < rows) {
         const int sq = vo.row_seq[t], key = t - vo.seq_off[sq];
         const int p = 8 * ((key & 15) >> 2) + 4 * ((key >> 4) & 1) + (key & 3);  // vt_key(p) == key & 31
-        _Float16* base = vo.vt + ((dim0 + dim) * vo.ldvt + 2 * (vo.voff[sq] + (key & ~31)));
+        const int dg = dim0 + dim;
+        _Float16* base = vo.vf + (((dg >> 8) * vo.n_tiles + ((vo.voff[sq] + key) >> 5)) * sgd::kFragTile +
+                                  sgd::vfrag_piece((dg & 255) >> 4, 0) + (16 * (p >> 3) + (dg & 15)) * 8 + (p & 7));
         const hl16 sp = split_f16(stage[rl * 32 + dim]);
-        base[p] = sp.hi;
-        base[32 + p] = sp.lo;
+        base[0] = sp.hi;
+        base[512] = sp.lo;
       }
     }
   }
@@ -284,7 +288,7 @@ __device__ __forceinline__ void gemm_epilogue(const f32x16_t (&acc)[TM][TN], int
         for (int tn = 0; tn < TN; tn++)
 #pragma unroll
           for (int r = 0; r < 16; r++) v[tn][r] = acc[tm][tn][r] * rs[r];
-        if (vto.vt && n0 >= vto.col0) {  // workgroup-uniform: the tile is V columns only
+        if (vto.vf && n0 >= vto.col0) {  // workgroup-uniform: the tile is V columns only
 #pragma unroll
           for (int tn = 0; tn < TN; tn++)
             store_vt_subtile(stage, v[tn], vto, mb, n0 + tn * 32 - vto.col0, M, lr, lh, lane);
@@ -789,10 +793,10 @@ hipError_t launch_lds(const int8_t* A, int a_rows, const int8_t* W, const float*
   constexpr int BM = NW * 32, BN = TN * 32;
   const int gm = (M + BM - 1) / BM;
   if ((int64_t)gm * BM > a_rows) return hipErrorInvalidValue;
-  if (vto && (GELU || !vto->vt || vto->col0 <= 0 || vto->col0 % BN || vto->col0 >= N || (vto->ldvt & 7) ||
-              !vto->row_seq || !vto->seq_off || !vto->voff || (reinterpret_cast<uintptr_t>(vto->vt) & 15) ||
-              (int64_t)(N - vto->col0) * vto->ldvt > INT32_MAX))
-    return hipErrorInvalidValue;  // whole V tiles; 16-byte chunk stores; 32-bit V^T offsets
+  if (vto && (GELU || !vto->vf || vto->col0 <= 0 || vto->col0 % BN || vto->col0 >= N || vto->n_tiles <= 0 ||
+              !vto->row_seq || !vto->seq_off || !vto->voff || (reinterpret_cast<uintptr_t>(vto->vf) & 15) ||
+              (N - vto->col0) % 256 || (int64_t)((N - vto->col0) / 256) * vto->n_tiles * sgd::kFragTile > INT32_MAX))
+    return hipErrorInvalidValue;  // whole V tiles; 16-byte fragment stores; 32-bit offsets
   const sg_vt_out vo = vto ? *vto : sg_vt_out{nullptr, 0, 0, nullptr, nullptr, nullptr};
   dim3 grid((N + BN - 1) / BN, gm);
   hipLaunchKernelGGL((k_gemm_q8_lds<NW, TN, GELU, STAGES>), grid, dim3(NW * SG_WAVE), 0, s, A, a_rows, W, St, rs, Y,

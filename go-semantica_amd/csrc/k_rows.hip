@@ -455,12 +455,15 @@ __global__ __launch_bounds__(kThreads) void k_norm_quantize_wave(const float* __
   store_codes_wave<NV>(x, inv, qf, a_rows, row, lane);
 }
 
-// k_quantize_blocked for D = cols columns (a multiple of 32).
+// k_quantize_blocked for D = cols columns (a multiple of 32); cmax: the
+// sequence's maximum over attention_small's chunk maxima.
 template <int D>
 __global__ __launch_bounds__(kThreads) void k_quantize_wave(const float* __restrict__ x, int ldx, int rows,
                                                             const int32_t* __restrict__ row_seq,
                                                             const float* __restrict__ amax, int8_t* __restrict__ qf,
-                                                            int a_rows, float* __restrict__ row_scale) {
+                                                            int a_rows, float* __restrict__ row_scale,
+                                                            const float* __restrict__ cmax,
+                                                            const int32_t* __restrict__ seq_off, int H) {
   constexpr int NV = (D + 255) / 256;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int row = blockIdx.x * kWaveWaves + wave;
@@ -473,7 +476,14 @@ __global__ __launch_bounds__(kThreads) void k_quantize_wave(const float* __restr
     v[k] = f32x4_t{0, 0, 0, 0};
     if (256 * k + 256 <= D || 256 * k + 4 * lane < D) v[k] = *reinterpret_cast<const f32x4_t*>(xr + 256 * k);
   }
-  const float m = amax[sq];
+  float m;
+  if (cmax) {
+    const int a = seq_off[sq], S = seq_off[sq + 1] - a;
+    const float* cm = cmax + sgk::attn_cmax_base(a, sq, H);
+    m = sg_wave_rows_max(cm, 0, H * ((S + sgk::kAttnChunkRows - 1) / sgk::kAttnChunkRows), lane);
+  } else {
+    m = amax[sq];
+  }
   float scale = 1.0f, inv = 0.0f;
   if (m != 0.0f) {
     scale = m / 127.0f;
@@ -540,10 +550,7 @@ __global__ __launch_bounds__(kThreads) void k_qknorm_rope(float* __restrict__ q,
                                                           const float* __restrict__ kw, int H, int HKV, int T,
                                                           const int32_t* __restrict__ row_pos,
                                                           const float* __restrict__ cos_t,
-                                                          const float* __restrict__ sin_t, float eps,
-                                                          _Float16* __restrict__ qs_h, _Float16* __restrict__ qs_l,
-                                                          int ldqs, _Float16* __restrict__ ks_h,
-                                                          _Float16* __restrict__ ks_l, int ldks) {
+                                                          const float* __restrict__ sin_t, float eps) {
   constexpr int NPL = 32, HALF = 128;
   const int g = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 3);
   const int j = threadIdx.x & 7;
@@ -575,44 +582,8 @@ __global__ __launch_bounds__(kThreads) void k_qknorm_rope(float* __restrict__ q,
     x[i] = a - b;
     x[i + NPL / 2] = cc + dd;
   }
-  if (!qs_h) {
 #pragma unroll
-    for (int i = 0; i < NPL; i++) p[8 * i + j] = x[i];
-    return;
-  }
-  // Attention operands: hi/lo fp16 of x * kAttnQKScale.
-  _Float16 *dh, *dl;
-  if (hh < H) {
-    dh = qs_h + (int64_t)t * ldqs + hh * 256;
-    dl = qs_l + (int64_t)t * ldqs + hh * 256;
-  } else {
-    dh = ks_h + (int64_t)t * ldks + (hh - H) * 256;
-    dl = ks_l + (int64_t)t * ldks + (hh - H) * 256;
-  }
-#pragma unroll
-  for (int i = 0; i < NPL; i++) {
-    const hl16 sp = split_f16(x[i] * sgk::kAttnQKScale);
-    dh[8 * i + j] = sp.hi;
-    dl[8 * i + j] = sp.lo;
-  }
-}
-
-// The same per-(token, head) arithmetic as k_qknorm_rope, writing the split
-// attention operands, in the float4 row layout (sg_rmsnorm8_f4): lane j of
-// the row's 8-lane group holds elements 32c + 4j .. 32c + 4j + 3, so loads
-// are 128 contiguous bytes per row and the RoPE partner e + 128 of element e
-// (chunk c + 4) sits in the same lane and slot.  Stores are 8-byte half4 hi
-// and lo pieces, 64 contiguous bytes per row and chunk.
-__global__ __launch_bounds__(kThreads) void k_qknorm_rope_split(
-    const float* __restrict__ q, int ldq, const float* __restrict__ k, int ldk, const float* __restrict__ qw,
-    const float* __restrict__ kw, int H, int HKV, int T, const int32_t* __restrict__ row_pos,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t, float eps, _Float16* __restrict__ qs_h,
-    _Float16* __restrict__ qs_l, int ldqs, _Float16* __restrict__ ks_h, _Float16* __restrict__ ks_l, int ldks) {
-  static_assert(kThreads == sgd::kKvThreads && kRowsPerBlock == sgd::kKvRows, "one 8-lane group per row");
-  __shared__ __attribute__((aligned(16))) float tiles[kThreads / SG_WAVE][8 * 40];
-  const int64_t g = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 3);
-  sgd::qk_split_group(g, threadIdx.x & 7, (threadIdx.x >> 3) & 7, tiles[threadIdx.x / SG_WAVE], q, ldq, k, ldk, qw,
-                      kw, H, HKV, T, row_pos, cos_t, sin_t, eps, qs_h, qs_l, ldqs, ks_h, ks_l, ldks);
+  for (int i = 0; i < NPL; i++) p[8 * i + j] = x[i];
 }
 
 // ------------------------------------------------------------ GELU * up --
@@ -848,8 +819,12 @@ hipError_t embed_only(const int32_t* tokens, int T, const int8_t* eq, const floa
 }
 
 hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, const float* amax,
-                    int8_t* q8, int a_rows, int8_t* i8, float* row_scale, hipStream_t s) {
+                    int8_t* q8, int a_rows, int8_t* i8, float* row_scale, hipStream_t s, const float* cmax,
+                    const int32_t* seq_off, int H) {
   if (rows <= 0) return hipSuccess;
+  if (cmax && (!seq_off || H <= 0 || !q8 || rows >= kWaveRows || (reinterpret_cast<uintptr_t>(x) & 15) ||
+               (cols != 256 && cols != 512 && cols != 768 && cols != 1024)))
+    return hipErrorInvalidValue;  // the wave form's launches
   if (cols % 4 || ldx % 4 || (!q8 && !i8)) return hipErrorInvalidValue;
   if (q8 && (cols % 32 || a_rows < rows)) return hipErrorInvalidValue;
   if (q8 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
@@ -860,7 +835,7 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
   case C:                                                                                                            \
     if (small)                                                                                                       \
       hipLaunchKernelGGL(k_quantize_wave<C>, dim3(blocks_for(rows, kWaveWaves)), dim3(kThreads), 0, s, x, ldx, rows, \
-                         row_seq, amax, q8, a_rows, row_scale);                                                      \
+                         row_seq, amax, q8, a_rows, row_scale, cmax, seq_off, H);                                    \
     else                                                                                                             \
       hipLaunchKernelGGL(k_quantize_blocked<C / 32>, dim3(blocks_for(rows, kRowsPerBlock)), dim3(kThreads), 0, s, x, \
                          ldx, rows, row_seq, amax, q8, a_rows, row_scale);                                           \
@@ -909,23 +884,12 @@ hipError_t rmsnorm(float* dst, const float* src, const float* w, int rows, int n
 }
 
 hipError_t qknorm_rope(float* q, int ldq, float* k, int ldk, const float* qw, const float* kw, int H, int HKV, int T,
-                       const int32_t* row_pos, const float* cos_t, const float* sin_t, float eps, _Float16* qs_h,
-                       _Float16* qs_l, int ldqs, _Float16* ks_h, _Float16* ks_l, int ldks, hipStream_t s) {
+                       const int32_t* row_pos, const float* cos_t, const float* sin_t, float eps, hipStream_t s) {
   if (T <= 0) return hipSuccess;
-  const bool split = ks_h != nullptr;
-  if (split && (!ks_l || (H > 0 && (!qs_h || !qs_l)))) return hipErrorInvalidValue;
   const int64_t groups = (int64_t)T * (H + HKV);
   if (groups <= 0) return hipSuccess;
-  if (split) {
-    if ((ldks & 7) || (ldk & 3) || (reinterpret_cast<uintptr_t>(k) & 15) ||
-        (H > 0 && ((ldqs & 7) || (ldq & 3) || (reinterpret_cast<uintptr_t>(q) & 15))))
-      return hipErrorInvalidValue;  // float4 loads of every head row
-    hipLaunchKernelGGL(k_qknorm_rope_split, dim3(blocks_for(groups, kRowsPerBlock)), dim3(kThreads), 0, s, q, ldq, k,
-                       ldk, qw, kw, H, HKV, T, row_pos, cos_t, sin_t, eps, qs_h, qs_l, ldqs, ks_h, ks_l, ldks);
-  } else {
-    hipLaunchKernelGGL(k_qknorm_rope, dim3(blocks_for(groups, kRowsPerBlock)), dim3(kThreads), 0, s, q, ldq, k, ldk,
-                       qw, kw, H, HKV, T, row_pos, cos_t, sin_t, eps, nullptr, nullptr, 0, nullptr, nullptr, 0);
-  }
+  hipLaunchKernelGGL(k_qknorm_rope, dim3(blocks_for(groups, kRowsPerBlock)), dim3(kThreads), 0, s, q, ldq, k, ldk, qw,
+                     kw, H, HKV, T, row_pos, cos_t, sin_t, eps);
   return hipGetLastError();
 }
 

@@ -55,7 +55,7 @@ using sgi::HostBuf;
 // Per-call sequence metadata built on the host from CSR offsets.
 struct Meta {
   int T = 0, n_seq = 0, n_items = 0, n_vtiles = 0;
-  int Tp = 0;         // V^T columns: every sequence padded to whole 32-key tiles
+  int Tp = 0;         // padded keys: every sequence padded to whole 32-key tiles
   int max_len = 0;    // longest sequence
   double sum_sq = 0;  // sum over sequences of S^2 (attention work)
   // Every sequence inside one attention work item: the attention then quantizes
@@ -67,8 +67,9 @@ struct Meta {
   // device views into one buffer
   int32_t* row_seq = nullptr;
   int32_t* row_pos = nullptr;
+  int32_t* row_key = nullptr;  // the row's key in the padded key numbering
   int32_t* seq_off = nullptr;
-  int32_t* voff = nullptr;   // [n_seq + 1] V^T column of each sequence
+  int32_t* voff = nullptr;   // [n_seq + 1] first padded key of each sequence
   sg_item* items = nullptr;  // attention workgroups (sequence, first chunk)
   sg_item* vtiles = nullptr; // V^T split tiles (sequence, first key)
   int32_t* spill_off = nullptr;  // [n_seq] first attention spill tile of each sequence
@@ -81,7 +82,7 @@ int seq_groups(int S, int G) {
   return (chunks + sgk::kAttnChunks - 1) / sgk::kAttnChunks;
 }
 
-// Fills `host` with [row_seq | row_pos | seq_off | voff | items | vtiles |
+// Fills `host` with [row_seq | row_pos | row_key | seq_off | voff | items | vtiles |
 // spill_off] and
 // copies it to `dev` on stream s, asynchronously: kernels launched on s after
 // this see the metadata, and the next stage_meta waits for the copy before it
@@ -107,14 +108,15 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
     n_spill += (int64_t)seq_groups(S, G) * sgk::attention_spill_tiles(S);
   }
   if (n_spill > INT32_MAX) return fail(SG_ERR_INVALID, "batch too large for the attention spill layout");
-  const size_t bytes = sizeof(int32_t) * ((size_t)2 * T + 2 * (n_seq + 1)) +
+  const size_t bytes = sizeof(int32_t) * ((size_t)3 * T + 2 * (n_seq + 1)) +
                        sizeof(sg_item) * ((size_t)n_items + n_vt) + sizeof(int32_t) * (size_t)n_seq + 64;
   SG_TRY(host.ensure(bytes));
   SG_TRY(dev.ensure(bytes));
   int32_t* h = host.as<int32_t>();
   int32_t* rs = h;
   int32_t* rp = rs + T;
-  int32_t* so = rp + T;
+  int32_t* rk = rp + T;
+  int32_t* so = rk + T;
   int32_t* vo = so + n_seq + 1;
   sg_item* it = reinterpret_cast<sg_item*>(vo + n_seq + 1);
   sg_item* vt = it + n_items;
@@ -128,6 +130,7 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
     for (int r = off[i]; r < off[i + 1]; r++) {
       rs[r] = i;
       rp[r] = r - off[i];
+      rk[r] = vo[i] + r - off[i];
     }
     for (int k0 = 0; k0 < S; k0 += 32) vt[nv++] = sg_item{i, k0};
     sp[i] = ns;
@@ -188,9 +191,10 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
   m.Tp = vo[n_seq];
   m.row_seq = d;
   m.row_pos = d + T;
-  m.seq_off = d + 2 * T;
-  m.voff = d + 2 * T + n_seq + 1;
-  m.items = reinterpret_cast<sg_item*>(d + 2 * T + 2 * (n_seq + 1));
+  m.row_key = d + 2 * (size_t)T;
+  m.seq_off = d + 3 * (size_t)T;
+  m.voff = m.seq_off + n_seq + 1;
+  m.items = reinterpret_cast<sg_item*>(m.voff + n_seq + 1);
   m.vtiles = m.items + n_items;
   m.spill_off = reinterpret_cast<int32_t*>(m.vtiles + n_vt);
   m.spill_total = ns;
@@ -353,9 +357,9 @@ struct Profiler {
 // stream of its own (created on first use, non-blocking, default priority) with
 // the event that joins it back to the caller's stream.
 struct Lane {
-  DevBuf h, xn, qkv, att, o, g, a8, sx, amax, rmax, meta_d, err;
-  DevBuf ks, vt;  // attention operands, hi/lo fp16 (K row-major; V^T); Q is split inside the attention kernel
-  DevBuf qs;      // Q hi/lo for launches too small to fill the GPU (attn_q_presplit)
+  DevBuf h, xn, qkv, att, o, g, a8, sx, amax, rmax, cmax, meta_d, err;
+  DevBuf ks, vt;  // K and V fragments (hi/lo fp16); Q is split inside the attention kernel
+  DevBuf qs;      // Q fragments for launches too small to fill the GPU (attn_small)
   DevBuf xp;      // exact-order attention: scores / weights [H][T][ldp] (SG_ATTN_EXACT only)
   DevBuf spill;   // attention scores past the kernel's register tiles (sequences > 512 keys)
   HostBuf meta_h, io_h;
@@ -373,7 +377,7 @@ struct Lane {
     return SG_OK;
   }
   ~Lane() {
-    for (DevBuf* b : {&h, &xn, &qkv, &att, &o, &g, &a8, &sx, &amax, &rmax, &meta_d, &err, &ks, &vt, &qs, &xp, &spill})
+    for (DevBuf* b : {&h, &xn, &qkv, &att, &o, &g, &a8, &sx, &amax, &rmax, &cmax, &meta_d, &err, &ks, &vt, &qs, &xp, &spill})
       b->release();
     meta_h.release();
     io_h.release();
@@ -494,16 +498,16 @@ struct Trace {
   float *qkv = nullptr, *att = nullptr, *h = nullptr;
 };
 
-// Attention launches of fewer workgroups than the GPU has CUs run latency-
-// bound, and there the in-kernel Q prologue (one memory round trip, the QK-norm
-// through the LDS tile, RoPE, the split: over half of a 32-token sequence's
-// workgroup) is on the critical path.  Such launches take Q pre-split from
-// k_kv_prep (the same arithmetic, bit-identical operands), which prepares it
-// over many more threads; larger launches keep the prologue, which saves
-// writing Q's operands and reading them back.
-constexpr int kAttnQPresplitItems = 256;
-bool attn_q_presplit(const sg_model* m, const Meta& meta) {
-  return m->attn_mode != SG_ATTN_EXACT && (int64_t)meta.n_items * m->cfg.num_kv_heads < kAttnQPresplitItems;
+// Attention launches that leave most CUs idle run the small form
+// (sgk::attn_small_form, when the chunk maxima it leaves have a quantizer:
+// sgk::quantize's cmax).  It takes Q pre-split by k_kv_prep (the same
+// arithmetic, bit-identical operands): there the in-kernel Q prologue would sit
+// on the critical path.  Larger launches keep the prologue, which saves writing
+// Q's operands and reading them back (15 x 512 tokens, one round of 180
+// workgroups: attention + k_kv_prep 55.5 + 5.8 us against 55.5 + 13.9).
+bool attn_small(const sg_model* m, const Meta& meta) {
+  return m->attn_mode != SG_ATTN_EXACT && sgk::attn_small_form(meta.n_items, m->cfg.num_kv_heads, meta.max_len) &&
+         sgk::row_max_form(meta.T, m->qd);
 }
 
 // Layers [l0, l1) of one sequence group's forward on lane w, stream s: the
@@ -524,10 +528,9 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   float* g = w.g.as<float>();
   int8_t* a8 = w.a8.as<int8_t>();
   const int ar = sgk::gemm_pad_rows(T);
-  _Float16* ks_h = w.ks.as<_Float16>();
-  _Float16* ks_l = ks_h + (size_t)T * kvd;
-  _Float16* vt_h = w.vt.as<_Float16>();
-  const int ldvt = 2 * meta.Tp;  // per dim: each 32-key tile's hi then lo halves
+  _Float16* kf = w.ks.as<_Float16>();
+  _Float16* vf = w.vt.as<_Float16>();
+  const int n_tiles = meta.Tp / 32;
   float* sx = w.sx.as<float>();
   float* amax = w.amax.as<float>();
   auto site = [&](int l, int k) { return amax + ((size_t)4 * l + k) * ns; };
@@ -543,8 +546,8 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   auto norm_q = [&](const float* w, float* am) {
     return sgk::norm_quantize(h, w, eps, T, d, meta.row_seq, am, a8, ar, sx, s, rmax, meta.seq_off);
   };
-  auto quant = [&](const float* x, int cols, float* am) {
-    return sgk::quantize(x, cols, T, cols, meta.row_seq, am, a8, ar, nullptr, sx, s);
+  auto quant = [&](const float* x, int cols, float* am, const float* cmax = nullptr) {
+    return sgk::quantize(x, cols, T, cols, meta.row_seq, am, a8, ar, nullptr, sx, s, cmax, meta.seq_off, c.num_heads);
   };
   auto tap = [&](float* dst, const float* src, int l, int cols) {
     return hipMemcpyAsync(dst + (size_t)l * T * cols, src, sizeof(float) * (size_t)T * cols, hipMemcpyDeviceToDevice,
@@ -563,11 +566,10 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   // (its attention reads V in fp32) nor when Q|K|V is traced.
   const bool vt_fused = m->attn_mode != SG_ATTN_EXACT && !(tr && tr->qkv) && sgk::gemm_writes_vt(T) &&
                         meta.seq_start32;
-  const sgk::sg_vt_out vto{vt_h, ldvt, qd + kvd, meta.row_seq, meta.seq_off, meta.voff};
-  // Small attention launches take Q pre-split by k_kv_prep (attn_q_presplit).
-  const bool q_pre = attn_q_presplit(m, meta);
-  _Float16* qs_h = q_pre ? w.qs.as<_Float16>() : nullptr;
-  _Float16* qs_l = q_pre ? qs_h + (size_t)T * qd : nullptr;
+  const sgk::sg_vt_out vto{vf, n_tiles, qd + kvd, meta.row_seq, meta.seq_off, meta.voff};
+  // Small attention launches take Q pre-split by k_kv_prep.
+  const bool a_small = attn_small(m, meta);
+  _Float16* qf = a_small ? w.qs.as<_Float16>() : nullptr;
 
   if (l0 == 0) {
     SG_LAUNCH(SG_K_OTHER, 4.0 * 4 * L * ns, sgk::fill_f32(amax, 0.0f, (int64_t)4 * L * ns, s));
@@ -575,7 +577,7 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
     // (the fused epilogue writes only the sequences' keys).
     if (vt_fused)
       SG_LAUNCH(SG_K_OTHER, 4.0 * kvd * meta.Tp,
-                sgk::fill_i32(reinterpret_cast<int32_t*>(vt_h), 0, (int64_t)kvd * meta.Tp, s));
+                sgk::fill_i32(reinterpret_cast<int32_t*>(vf), 0, (int64_t)kvd * meta.Tp, s));
     SG_LAUNCH(SG_K_OTHER, 4.0, sgk::fill_i32(w.err.as<int32_t>(), INT32_MAX, 1, s));
     SG_LAUNCH(SG_K_NORM, t * (34.0 * d / 32 + 4.0 * d),
               sgk::embed_norm(d_tokens, T, m->emb_q, m->emb_s, c.vocab_size, d, m->sqrt_d, m->layers[0].attn_norm,
@@ -583,7 +585,8 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   }
   // Short sequences (each one attention item): the attention quantizes its own
   // output, so that quantizer launch goes.
-  const bool q_attn = meta.seq_one_item && c.num_kv_heads == 1 && meta.max_len <= sgk::kAttnRegKeys;
+  const bool q_attn = meta.seq_one_item && c.num_kv_heads == 1 && meta.max_len <= sgk::kAttnRegKeys && !a_small;
+  float* cmax = a_small ? w.cmax.as<float>() : nullptr;
   for (int l = l0; l < l1; l++) {
     if (l == stop) break;
     const LayerDev& ly = m->layers[l];
@@ -598,7 +601,7 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
       // max|o| into amax for the quantizer).
       SG_LAUNCH(SG_K_NORM, t * (qd + kvd) * 8.0,
                 sgk::qknorm_rope(qkv, nqkv, qkv + qd, nqkv, ly.q_norm, ly.k_norm, c.num_heads, c.num_kv_heads, T,
-                                 meta.row_pos, m->cos_t, m->sin_t, eps, nullptr, nullptr, 0, nullptr, nullptr, 0, s));
+                                 meta.row_pos, m->cos_t, m->sin_t, eps, s));
       SG_LAUNCH(SG_K_ATTENTION, attn_flops,
                 sgk::attention_exact(qkv, nqkv, qkv + qd, qkv + qd + kvd, nqkv, att, qd, meta.seq_off, meta.row_seq,
                                      ns, T, c.num_heads, c.num_kv_heads, m->hd, m->attn_scale, meta.max_len,
@@ -606,23 +609,25 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
     } else {
       // K's QK-norm + RoPE + split and V's V^T split in one launch; Q's norm and
       // RoPE run inside the attention kernel.
-      const sgk::sg_kv_q qpart{qkv, nqkv, ly.q_norm, c.num_heads, qs_h, qs_l, qd};
-      SG_LAUNCH(SG_K_NORM, t * ((vt_fused ? 8.0 : 16.0) * kvd + (q_pre ? 8.0 * qd : 0.0)),
+      const sgk::sg_kv_q qpart{qkv, nqkv, ly.q_norm, c.num_heads, qf};
+      SG_LAUNCH(SG_K_NORM, t * ((vt_fused ? 8.0 : 16.0) * kvd + (a_small ? 8.0 * qd : 0.0)),
                 sgk::kv_prep(qkv + qd, qkv + qd + kvd, nqkv, ly.k_norm, c.num_kv_heads, T, meta.row_pos, m->cos_t,
-                             m->sin_t, eps, ks_h, ks_l, kvd, meta.seq_off, meta.voff, meta.vtiles,
-                             vt_fused ? 0 : meta.n_vtiles, vt_h, ldvt, s, q_pre ? &qpart : nullptr));
+                             m->sin_t, eps, meta.row_key, kf, meta.seq_off, meta.voff, meta.vtiles,
+                             vt_fused ? 0 : meta.n_vtiles, vf, n_tiles, s, a_small ? &qpart : nullptr));
       const sg_attn_qpre qpre{qkv, nqkv, ly.q_norm, m->cos_t, m->sin_t, eps};
       const sg_attn_qout qout{a8, ar, sx};
       const sg_attn_spill spill{w.spill.as<float>(), meta.spill_off, meta.spill_total};
       SG_LAUNCH(SG_K_ATTENTION, attn_flops,
-                sgk::attention(q_pre ? qs_h : nullptr, q_pre ? qs_l : nullptr, q_pre ? qd : 0, ks_h, ks_l, kvd, vt_h,
-                               ldvt, att, qd, meta.seq_off, meta.voff, meta.items, meta.n_items, c.num_heads,
-                               c.num_kv_heads, m->hd, m->attn_scale, site(l, 1), meta.max_len, s,
-                               q_pre ? nullptr : &qpre, q_attn ? &qout : nullptr, &spill));
+                a_small ? sgk::attention_small(qf, kf, vf, n_tiles, att, qd, meta.seq_off, meta.voff,
+                                               meta.items, meta.n_items, c.num_heads, c.num_kv_heads, m->hd,
+                                               m->attn_scale, cmax, meta.max_len, s)
+                        : sgk::attention(nullptr, kf, vf, n_tiles, att, qd, meta.seq_off, meta.voff, meta.items, meta.n_items,
+                                         c.num_heads, c.num_kv_heads, m->hd, m->attn_scale, site(l, 1), meta.max_len,
+                                         s, &qpre, q_attn ? &qout : nullptr, &spill));
     }
     if (tr && tr->att) SG_HIP(tap(tr->att, att, l, qd));
     if (!(q_attn && m->attn_mode != SG_ATTN_EXACT))
-      SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(qd), quant(att, qd, site(l, 1)));
+      SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(qd), quant(att, qd, site(l, 1), cmax));
     // The O projection and the residual post-norm: one launch for large
     // batches (o stays on chip), else the GEMM then k_post_res_norm.
     if (sgk::gemm_res_norm_fused(T, d, ly.post_attn, ly.ffn_norm)) {
@@ -723,15 +728,17 @@ int ensure_workspace(const sg_model* m, Lane& w, const Meta& meta) {
   SG_TRY(w.o.ensure(sizeof(float) * t * c.embed_dim));
   SG_TRY(w.g.ensure(sizeof(float) * t * c.interm_dim));
   SG_TRY(w.a8.ensure((size_t)sgk::gemm_pad_rows(T) * a_cols));
-  if (attn_q_presplit(m, meta)) SG_TRY(w.qs.ensure(2 * sizeof(_Float16) * t * m->qd));
+  if (attn_small(m, meta)) SG_TRY(w.qs.ensure(2 * sizeof(_Float16) * (size_t)m->qd * Tp));
   SG_TRY(w.sx.ensure(sizeof(float) * t));
   if (sgk::row_max_form(T, c.embed_dim)) SG_TRY(w.rmax.ensure(sizeof(float) * t));
   SG_TRY(w.amax.ensure(sizeof(float) * 4 * (size_t)c.num_layers * n_seq));
-  SG_TRY(w.ks.ensure(2 * sizeof(_Float16) * t * m->kvd));
+  SG_TRY(w.ks.ensure(2 * sizeof(_Float16) * (size_t)m->kvd * Tp));
   SG_TRY(w.vt.ensure(2 * sizeof(_Float16) * (size_t)m->kvd * Tp));
   SG_TRY(w.err.ensure(64));
   if (m->attn_mode == SG_ATTN_EXACT)
     SG_TRY(w.xp.ensure(sgk::attention_exact_scratch(T, c.num_heads, meta.max_len)));
+  else if (attn_small(m, meta))
+    SG_TRY(w.cmax.ensure(sizeof(float) * (size_t)sgk::attn_cmax_base(T, n_seq, c.num_heads)));
   else
     SG_TRY(w.spill.ensure((size_t)c.num_kv_heads * meta.spill_total * sgk::kAttnSpillTileBytes));
   return SG_OK;
@@ -1338,7 +1345,7 @@ int sg_qknorm_rope(sg_ctx* ctx, float* q, int32_t ldq, float* k, int32_t ldk, co
   SG_HIP(hipMemcpy(tc, ct.data(), sizeof(float) * ct.size(), hipMemcpyHostToDevice));
   SG_HIP(hipMemcpy(tc + ct.size(), st.data(), sizeof(float) * st.size(), hipMemcpyHostToDevice));
   SG_HIP(sgk::qknorm_rope(q, ldq, k, ldk, q_norm, k_norm, n_heads, n_kv_heads, meta.T, meta.row_pos, tc,
-                          tc + ct.size(), eps, nullptr, nullptr, 0, nullptr, nullptr, 0, s));
+                          tc + ct.size(), eps, s));
   SG_HIP(hipStreamSynchronize(s));
   return SG_OK;
 }
@@ -1357,23 +1364,28 @@ int sg_attention(sg_ctx* ctx, float* out, const float* q, int32_t ldq, const flo
   SG_TRY(stage_meta(off, n_seq, n_heads / n_kv_heads, ctx->meta_h, ctx->meta_d, s, meta));
   const float scale = 1.0f / (float)std::sqrt((double)head_dim);
   // Split operands as the forward's producers write them.
-  const size_t T = (size_t)meta.T, qd = (size_t)n_heads * head_dim, kvd = (size_t)n_kv_heads * head_dim;
-  const size_t split_bytes = (2 * sizeof(_Float16) * (T * qd + T * kvd + kvd * (size_t)meta.Tp) + 255) & ~(size_t)255;
-  SG_TRY(ctx->split.ensure(split_bytes + (size_t)n_kv_heads * meta.spill_total * sgk::kAttnSpillTileBytes));
+  const size_t qd = (size_t)n_heads * head_dim, kvd = (size_t)n_kv_heads * head_dim, Tp = (size_t)meta.Tp;
+  const size_t split_bytes = (2 * sizeof(_Float16) * (qd + 2 * kvd) * Tp + 255) & ~(size_t)255;
+  const bool small = sgk::attn_small_form(meta.n_items, n_kv_heads, meta.max_len);
+  SG_TRY(ctx->split.ensure(split_bytes + (small ? 0 : (size_t)n_kv_heads * meta.spill_total * sgk::kAttnSpillTileBytes)));
   SG_TRY(gemm_scratch_begin(ctx, s));  // after the asynchronous GEMM calls of this context
-  _Float16* qs_h = ctx->split.as<_Float16>();
-  _Float16* qs_l = qs_h + T * qd;
-  _Float16* ks_h = qs_l + T * qd;
-  _Float16* ks_l = ks_h + T * kvd;
-  _Float16* vt_h = ks_l + T * kvd;
-  const int ldvt = 2 * meta.Tp;  // per dim: each 32-key tile's hi then lo halves
-  SG_HIP(sgk::split_rows(q, ldq, meta.T, (int)qd, sgk::kAttnQKScale, qs_h, qs_l, (int)qd, s));
-  SG_HIP(sgk::split_rows(k, ldkv, meta.T, (int)kvd, sgk::kAttnQKScale, ks_h, ks_l, (int)kvd, s));
-  SG_HIP(sgk::v_split_t(v, ldkv, meta.seq_off, meta.voff, meta.vtiles, meta.n_vtiles, n_kv_heads, vt_h, ldvt, s));
+  _Float16* qf = ctx->split.as<_Float16>();
+  _Float16* kf = qf + 2 * qd * Tp;
+  _Float16* vf = kf + 2 * kvd * Tp;
+  const int n_tiles = meta.Tp / 32;
+  SG_HIP(sgk::qkv_split(q, ldq, k, v, ldkv, n_heads, n_kv_heads, meta.seq_off, meta.voff, meta.vtiles, meta.n_vtiles,
+                        qf, kf, vf, n_tiles, s));
+  if (small) {
+    SG_HIP(sgk::attention_small(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items,
+                                meta.n_items, n_heads, n_kv_heads, head_dim, scale, nullptr,
+                                meta.max_len, s));
+    SG_HIP(hipStreamSynchronize(s));
+    return SG_OK;
+  }
   const sg_attn_spill spill{reinterpret_cast<float*>(ctx->split.as<unsigned char>() + split_bytes), meta.spill_off,
                             meta.spill_total};
-  SG_HIP(sgk::attention(qs_h, qs_l, (int)qd, ks_h, ks_l, (int)kvd, vt_h, ldvt, out, (int)qd, meta.seq_off,
-                        meta.voff, meta.items, meta.n_items, n_heads, n_kv_heads, head_dim, scale, nullptr,
+  SG_HIP(sgk::attention(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items,
+                        meta.n_items, n_heads, n_kv_heads, head_dim, scale, nullptr,
                         meta.max_len, s, nullptr, nullptr, &spill));
   SG_HIP(hipStreamSynchronize(s));
   return SG_OK;

@@ -84,8 +84,12 @@ hipError_t embed_norm(const int32_t* tokens, int T, const int8_t* eq, const floa
 // Per-sequence symmetric quantization of x[rows][cols] (stride ldx) using amax[row_seq[r]].
 // Writes the int8 codes block-major q8[cols/32][a_rows][32] (q8 != null, the GEMM
 // operand) or row-major i8[rows][cols] (q8 == null), and row_scale[rows].
+// cmax (with the CSR seq_off, H heads; q8 and rows < the row_max_form limit):
+// the sequence's maximum is taken over attention_small's chunk maxima instead
+// of amax.
 hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, const float* amax,
-                    int8_t* q8, int a_rows, int8_t* i8, float* row_scale, hipStream_t s);
+                    int8_t* q8, int a_rows, int8_t* i8, float* row_scale, hipStream_t s, const float* cmax = nullptr,
+                    const int32_t* seq_off = nullptr, int H = 0);
 // xn = RMSNorm(h; w) recomputed row by row exactly as post_res_norm / embed_norm
 // formed it, quantized with amax[row_seq[r]] into the block-major int8 GEMM
 // operand q8[d/32][a_rows][32] and row_scale[T] (quantize's arithmetic).
@@ -98,13 +102,9 @@ hipError_t seq_scales(const float* amax, int n_seq, float* out, hipStream_t s);
 // RMSNorm rows in the reference's order; amax (optional) collects per-sequence max|y|.
 hipError_t rmsnorm(float* dst, const float* src, const float* w, int rows, int n, float eps,
                    const int32_t* row_seq, float* amax, hipStream_t s);
-// QK-norm + RoPE; head_dim 256.  In place (fp32) when ks_h is null, else
-// written as the attention operands: hi/lo fp16 of x * kAttnQKScale into
-// qs_h/qs_l [T][ldqs] and ks_h/ks_l [T][ldks] (q and k are only read; H = 0
-// processes K alone, for attention() with qpre).
+// QK-norm + RoPE in place (fp32); head_dim 256.
 hipError_t qknorm_rope(float* q, int ldq, float* k, int ldk, const float* qw, const float* kw, int H, int HKV,
                        int T, const int32_t* row_pos, const float* cos_t, const float* sin_t, float eps,
-                       _Float16* qs_h, _Float16* qs_l, int ldqs, _Float16* ks_h, _Float16* ks_l, int ldks,
                        hipStream_t s);
 // h = RMSNorm(o; w_post) + h ; xn = RMSNorm(h; w_next) (stored when xn != null) ;
 // amax (optional) per sequence of max|xn|.
@@ -132,13 +132,13 @@ hipError_t issue_probe(int kind, int blocks, float* sink, long long* clk, int it
 // the exact block sums int32 [M][N][K/32].  cold_weights: W is not expected
 // in L2 (the forward, one layer after another), which selects deeper load
 // pipelines for small grids; the results are the same either way.
-// The V columns [col0, N) of the QKV GEMM written straight as attention's
-// V^T operand (hi/lo fp16 in the layout and key order k_kv_prep's V half
-// writes: per sequence s at key columns voff[s] ..) instead of fp32 into Y;
+// The V columns [col0, N) of the QKV GEMM written straight as attention's V
+// fragments (vf, n_tiles 32-key tiles per kv head, as k_kv_prep's V half
+// writes them: sequence s from tile voff[s] / 32 on) instead of fp32 into Y;
 // the bits are the same.  Positions past a sequence's end are not written.
 struct sg_vt_out {
-  _Float16* vt;
-  int ldvt;
+  _Float16* vf;
+  int n_tiles;
   int col0;
   const int32_t* row_seq;
   const int32_t* seq_off;
@@ -175,49 +175,67 @@ constexpr float kAttnQKScale = 8.0f;  // Q and K are split after scaling by 8 (e
 constexpr int kAttnChunkRows = 16;    // (head, query) rows per attention chunk (one wave)
 constexpr int kAttnChunks = 8;        // chunks per attention workgroup
 constexpr int kAttnRegKeys = 512;     // longest sequence whose scores pass 1 keeps in registers
-// Columns of V^T a sequence of S keys occupies (whole 32-key tiles).
+// Keys a sequence of S keys occupies in the padded numbering (whole 32-key tiles).
 inline int attn_key_pad(int S) { return (S + 31) / 32 * 32; }
-// V fp32 [T][ldv] -> V^T fp16 [HKV*256][ldvt] (sequence s at key column voff[s],
-// keys permuted within 32-key tiles, zero past S; the tile at key column c of
-// a dim row holds its hi halves at 2c .. 2c+31 and its lo halves at 2c+32 ..
-// 2c+63, so ldvt >= 2 * key columns); vtiles: (seq, key0) per 32 keys.
-hipError_t v_split_t(const float* v, int ldv, const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles,
-                     int n_vtiles, int HKV, _Float16* vt, int ldvt, hipStream_t s);
-// qknorm_rope's K-only split (H = 0) and v_split_t in one launch: K and V
-// share the row stride ldkv (columns of the QKV output).  n_vtiles = 0: K
-// only (V^T written by the QKV GEMM, sg_vt_out).
+// Padded key numbering: sequence s holds keys voff[s] .. voff[s] + S - 1 of
+// Tp = sum of attn_key_pad(S), row_key[row] its row's key.  K and V are held in
+// MFMA fragment order (sg_kv_prep.h), kf and vf [HKV][n_tiles] tiles of
+// kAttnTileHalves, n_tiles = Tp / 32.
+constexpr int kAttnTileHalves = 16384;
+// The kernel seam's operands: Q and K (already normed and rotated) and V split
+// into qf [H][n_tiles], kf and vf; vtiles: (seq, key0) per 32 keys.
+hipError_t qkv_split(const float* q, int ldq, const float* k, const float* v, int ldkv, int H, int HKV,
+                     const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* qf,
+                     _Float16* kf, _Float16* vf, int n_tiles, hipStream_t s);
+// K's QK-norm, RoPE and split, and V's split, in one launch: K and V share the
+// row stride ldkv (columns of the QKV output).  n_vtiles = 0: K only (V written
+// by the QKV GEMM, sg_vt_out).
 // Optional Q part of kv_prep: the H query heads' norm (qw), RoPE and hi/lo
-// split as well (k_qknorm_rope_split's arithmetic), into qs_h / qs_l
-// [T][ldqs], for launches that run the attention on pre-split Q.
+// split as well, into Q's
+// fragments qf [H][n_tiles], for launches that run the attention on pre-split Q.
 struct sg_kv_q {
   const float* q;
   int ldq;
   const float* qw;
   int H;
-  _Float16* qs_h;
-  _Float16* qs_l;
-  int ldqs;
+  _Float16* qf;
 };
 hipError_t kv_prep(const float* k, const float* v, int ldkv, const float* kw, int HKV, int T, const int32_t* row_pos,
-                   const float* cos_t, const float* sin_t, float eps, _Float16* ks_h, _Float16* ks_l, int ldks,
-                   const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* vt,
-                   int ldvt, hipStream_t s, const sg_kv_q* qpart = nullptr);
-// rows x cols of x -> hi/lo fp16 of x*scale (row stride ldo).
-hipError_t split_rows(const float* x, int ldx, int rows, int cols, float scale, _Float16* hi, _Float16* lo, int ldo,
-                      hipStream_t s);
+                   const float* cos_t, const float* sin_t, float eps, const int32_t* row_key, _Float16* kf,
+                   const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* vf,
+                   int n_tiles, hipStream_t s, const sg_kv_q* qpart = nullptr);
 // out[T][ldo] = attention over the split operands; items: (seq, first chunk)
 // per workgroup, chunk c of a sequence = (head c / ceil(S/16), rows 16*(c % ceil(S/16))).
 // qpre != null: Q is taken from qpre (fp32, normed and rotated in the kernel
-// exactly as qknorm_rope does) and qh/ql/ldq are ignored.  max_len: the
+// with qknorm_rope's arithmetic) and qf is ignored.  max_len: the
 // longest sequence of the launch.  Pass 1's scores stay in registers up to
 // kAttnRegKeys keys; a longer sequence keeps the rest in spill (required
 // when max_len exceeds kAttnRegKeys).  A sequence gives the same bits
 // whatever the launch's max_len.
-hipError_t attention(const _Float16* qh, const _Float16* ql, int ldq, const _Float16* kh, const _Float16* kl, int ldk,
-                     const _Float16* vt, int ldvt, float* out, int ldo, const int32_t* seq_off,
-                     const int32_t* voff, const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
+hipError_t attention(const _Float16* qf, const _Float16* kf, const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off, const int32_t* voff, const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
                      float* amax, int max_len, hipStream_t s, const sg_attn_qpre* qpre = nullptr,
                      const sg_attn_qout* qout = nullptr, const sg_attn_spill* spill = nullptr);
+// The same for launches too small to fill the GPU (attn_small_form), with Q
+// pre-split: the same bits as attention(), no spill buffer.  cmax (optional)
+// receives each chunk's max|out|, sequence i's chunks (kv head by kv head) from
+// attn_cmax_base(seq_off[i], i, H) on; it holds attn_cmax_base(T, n_seq, H)
+// floats.
+// Where the lines lie (us per launch on MI355X, k_attn_rs / one chunk per
+// workgroup / two; 512 tokens unless said): 12 items 47 / 18 / -, 24 items
+// 47 / 19 / -, 48 items 47 / 33 / 23, 72 items 48 / - / 44; 128 tokens, 48 items
+// 21 / - / 13; 1024 tokens, 24 items 88 / 30 / -, 48 items 88 / - / 37; 2048
+// tokens, 48 items 166 / 96 / -, 144 items 170 / 245 / -.  The small form wins
+// while its workgroups (8 or 4 per item, one per CU) make about one round.
+constexpr int kAttnSmallItems = 64;     // up to this many (items x kv heads): the small form
+constexpr int kAttnSmallKeys = 2048;    // ... for sequences of up to this many keys (scores in LDS)
+constexpr int kAttnSmallOneItems = 32;  // up to this many: one chunk per workgroup, above: two (to 1024 keys)
+bool attn_small_form(int n_items, int HKV, int max_len);
+__host__ __device__ inline int64_t attn_cmax_base(int row0, int seq, int H) {
+  return ((int64_t)row0 / kAttnChunkRows + seq) * H;  // >= H * (chunks of 16 rows of the sequences before)
+}
+hipError_t attention_small(const _Float16* qf, const _Float16* kf, const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off, const int32_t* voff,
+                           const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
+                           float* cmax, int max_len, hipStream_t s);
 // Score tiles a sequence of S keys spills per attention workgroup (one 32-key
 // tile of one workgroup: kAttnSpillTileBytes).
 constexpr int kAttnSpillTileBytes = kAttnChunks * 2048;
