@@ -33,14 +33,14 @@ struct BfElem<int8_t> {
   static constexpr bool kQuant = true;
   static constexpr int kLo = -127;
   __device__ static float inv() { return (float)(1.0 / 127.0); }
-  __device__ static double scale() { return 127.0; }
+  __device__ static float scale() { return 127.0f; }
 };
 template <>
 struct BfElem<int16_t> {
   static constexpr bool kQuant = true;
   static constexpr int kLo = -32767;
   __device__ static float inv() { return (float)(1.0 / 32767.0); }
-  __device__ static double scale() { return 32767.0; }
+  __device__ static float scale() { return 32767.0f; }
 };
 template <>
 struct BfElem<float> {
@@ -101,48 +101,99 @@ __device__ __forceinline__ float bf_lut(T c) {
 
 // ------------------------------------------------------------------ build --
 
-// builder.go:131-141 on one row: float64 sum of the float32 squares in index
+// builder.go:131-141 on each row: float64 sum of the float32 squares in index
 // order, norm = float32(1/sqrt(sum)), v *= norm (a zero vector stays as is);
 // then quant.go:17-41: clamp to [-1, 1] and math.Round(float64(v) * 127 or
-// 32767) (the product is exact in float64, so C round() of it is the same).
-// One thread per vector (the float64 sum is sequential by definition).
+// 32767) (sg_round_prod_f_nb: the product rounded once, half away from zero).
+// A workgroup takes 64 vectors, staged through LDS 64 dimensions at a time with
+// coalesced loads (the next chunk's in flight meanwhile), twice: one lane per
+// vector runs the sums, then a thread per (vector, group) quantizes, a wave's
+// stores covering one group of 64 vectors.  (A lane per vector reading its own
+// row from memory moved 0.2 TB/s: 21.9 ms for 10^6 x 768 to int8; now 1.14.)
+constexpr int kBuildDims = 64, kBuildRows = 64;
 template <typename T>
 __global__ __launch_bounds__(kBfThreads) void k_bf_build(const float* __restrict__ src, int64_t ld, int n, int dim,
                                                         int row0, int N, T* __restrict__ grp, T* __restrict__ tail,
                                                         int normalize) {
-  const int r = blockIdx.x * kBfThreads + threadIdx.x;
-  if (r >= n) return;
-  const float* v = src + (int64_t)r * ld;
-  float norm = 1.0f;
-  bool scale = false;
+  __shared__ float tile[kBuildRows][kBuildDims + 1];
+  __shared__ float norms[kBuildRows];
+  __shared__ int scales[kBuildRows];
+  constexpr int L = kBuildRows * kBuildDims / kBfThreads;  // loads per thread and chunk
+  const int tid = threadIdx.x, v0 = blockIdx.x * kBuildRows;
+  const int lc = tid % kBuildDims, lrow = tid / kBuildDims;  // column, first row of this thread's loads
+  const int chunks = (dim + kBuildDims - 1) / kBuildDims;
+  float r[L];
+  auto fetch = [&](int c) {
+    const int col = min(c * kBuildDims + lc, dim - 1);
+#pragma unroll
+    for (int u = 0; u < L; u++)
+      r[u] = src[(int64_t)min(v0 + lrow + (kBfThreads / kBuildDims) * u, n - 1) * ld + col];
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int u = 0; u < L; u++) tile[lrow + (kBfThreads / kBuildDims) * u][lc] = r[u];
+  };
+  double sum = 0.0;
+  fetch(0);
   if (normalize) {
-    double sum = 0.0;
-    for (int i = 0; i < dim; i++) {
-      const float sq = v[i] * v[i];
-      sum += (double)sq;
+    for (int c = 0; c < chunks; c++) {
+      __syncthreads();
+      stage();
+      __syncthreads();
+      fetch(c + 1 < chunks ? c + 1 : 0);
+      if (tid < kBuildRows) {
+        const int cn = min(kBuildDims, dim - c * kBuildDims);
+        for (int i0 = 0; i0 < cn; i0 += 16) {
+          float v[16];
+#pragma unroll
+          for (int u = 0; u < 16; u++) v[u] = tile[tid][min(i0 + u, kBuildDims - 1)];
+#pragma unroll
+          for (int u = 0; u < 16; u++) {
+            const float sq = v[u] * v[u];
+            if (i0 + u < cn) sum += (double)sq;
+          }
+        }
+      }
     }
-    if (sum != 0.0) {
-      norm = (float)(1.0 / sqrt(sum));
-      scale = true;
+    if (tid < kBuildRows) {
+      scales[tid] = sum != 0.0;
+      norms[tid] = sum != 0.0 ? (float)(1.0 / sqrt(sum)) : 1.0f;
     }
   }
   const int G = dim >> 3, R = dim & 7;
-  const int64_t row = row0 + r;
-  for (int i = 0; i < dim; i++) {
-    float x = v[i];
-    if (scale) x = x * norm;
-    T q;
-    if constexpr (BfElem<T>::kQuant) {
-      x = x > 1.0f ? 1.0f : (x < -1.0f ? -1.0f : x);
-      q = (T)round((double)x * BfElem<T>::scale());
-    } else {
-      q = x;
+  const int vec = tid % kBuildRows;
+  const bool live = v0 + vec < n;
+  const int64_t row = row0 + v0 + vec;
+  for (int c = 0; c < chunks; c++) {
+    __syncthreads();
+    stage();
+    __syncthreads();
+    if (c + 1 < chunks) fetch(c + 1);
+    const float norm = normalize ? norms[vec] : 1.0f;
+    const bool scale = normalize && scales[vec];
+#pragma unroll
+    for (int u = 0; u < kBuildDims / 8 * kBuildRows / kBfThreads; u++) {
+      const int gl = tid / kBuildRows + (kBfThreads / kBuildRows) * u, g = c * (kBuildDims / 8) + gl;
+      T q[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        float x = tile[vec][8 * gl + e];
+        if (scale) x = x * norm;
+        if constexpr (BfElem<T>::kQuant) {
+          x = x > 1.0f ? 1.0f : (x < -1.0f ? -1.0f : x);
+          q[e] = (T)(int)sg_round_prod_f_nb(x, BfElem<T>::scale());
+        } else {
+          q[e] = x;
+        }
+      }
+      if (live && g < G) {
+        __builtin_memcpy(__builtin_assume_aligned(grp + ((int64_t)g * N + row) * 8, 8 * sizeof(T)), q, sizeof q);
+      } else if (live && g == G) {
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+          if (e < R) tail[row * R + e] = q[e];
+      }
     }
-    const int g = i >> 3;
-    if (g < G)
-      grp[((int64_t)g * N + row) * 8 + (i & 7)] = q;
-    else
-      tail[row * R + (i & 7)] = q;
   }
 }
 
@@ -208,6 +259,34 @@ __global__ void k_bf_unpack(const T* __restrict__ grp, const T* __restrict__ tai
 }
 
 // ---------------------------------------------------------------- scoring --
+
+// The eight lane sums' reduction and the scalar tail (x, tp: the query's and the
+// vector's last R elements).
+template <typename T>
+__device__ __forceinline__ float bf_finish(const float (&l)[8], int G, int R, const float* __restrict__ x,
+                                           const T* __restrict__ tp) {
+  float sum = 0.0f;
+  if (G > 0) sum += ((l[0] + l[4]) + (l[1] + l[5])) + ((l[2] + l[6]) + (l[3] + l[7]));
+  if constexpr (BfElem<T>::kQuant) {
+    float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+    int i = 0;
+    if (R >= 4) {
+      s0 += x[0] * bf_lut<T>(tp[0]);
+      s1 += x[1] * bf_lut<T>(tp[1]);
+      s2 += x[2] * bf_lut<T>(tp[2]);
+      s3 += x[3] * bf_lut<T>(tp[3]);
+      i = 4;
+    }
+    sum += s0 + s1 + s2 + s3;
+    for (; i < R; i++) sum += x[i] * bf_lut<T>(tp[i]);
+  } else {
+    for (int i = 0; i < R; i++) {
+      const float p = (float)tp[i] * x[i];
+      sum += p;
+    }
+  }
+  return sum;
+}
 
 // scores[q][n] for QB queries (rows q0.. of `queries`, already normalized)
 // against every stored vector; lane = vector.  The workgroup stages the
@@ -279,31 +358,8 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_score(const T* __restrict__ g
 #pragma unroll
   for (int j = 0; j < QB; j++) {
     if (q0 + j >= nq) break;
-    float sum = 0.0f;
-    if (G > 0) {
-      const float* l = acc[j];
-      sum += ((l[0] + l[4]) + (l[1] + l[5])) + ((l[2] + l[6]) + (l[3] + l[7]));
-    }
-    const float* x = queries + (int64_t)(q0 + j) * dim + 8 * G;
-    if constexpr (BfElem<T>::kQuant) {
-      float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
-      int i = 0;
-      if (R >= 4) {
-        s0 += x[0] * bf_lut<T>(tp[0]);
-        s1 += x[1] * bf_lut<T>(tp[1]);
-        s2 += x[2] * bf_lut<T>(tp[2]);
-        s3 += x[3] * bf_lut<T>(tp[3]);
-        i = 4;
-      }
-      sum += s0 + s1 + s2 + s3;
-      for (; i < R; i++) sum += x[i] * bf_lut<T>(tp[i]);
-    } else {
-      for (int i = 0; i < R; i++) {
-        const float p = (float)tp[i] * x[i];
-        sum += p;
-      }
-    }
-    scores[(int64_t)(q0 + j) * ld_scores + n] = sum;
+    scores[(int64_t)(q0 + j) * ld_scores + n] =
+        bf_finish<T>(acc[j], G, R, queries + (int64_t)(q0 + j) * dim + 8 * G, tp);
   }
 }
 
@@ -505,6 +561,546 @@ __global__ __launch_bounds__(64) void k_bf_stream(const float* __restrict__ scor
   }
 }
 
+// ------------------------------------------------------------- prefiltering --
+//
+// Scoring every (query, vector) pair in the reference's float32 order costs two
+// VALU operations per dimension that no matrix core can do, and the scores are
+// then written and re-read by the selection.  For the indexes and batches
+// bf_prefilter_ok accepts, the search instead
+//   1. k_bf_approx: scores blocks of 64 vectors against up to 64 queries on the
+//      fp16 matrix cores and keeps only each block's maximum per query;
+//   2. k_bf_blocks: per query, takes a value T that at least k block maxima reach
+//      and lists the blocks whose maximum reaches T - 2 eps;
+//   3. k_bf_rescore: scores the listed blocks' vectors in the reference's order;
+//   4. k_bf_top: selects the exact top k of those scores.
+// eps bounds |approximate - reference-order| score for every stored vector
+// (bf_prep: fp16 rounding of both operands, the accumulation on either side,
+// against the largest stored norm).  At least k vectors have an exact score of
+// T - eps or more, so the k-th best exact score v_k is at least that and every
+// vector that reaches v_k has an approximate score of at least T - 2 eps: it is
+// in a listed block, and the result is the exact top k.  A query for which this
+// does not decide -- a tie straddling the k-th place, more than `cap` listed
+// blocks, a query that is zero, tiny, huge or not finite -- is flagged, and the
+// caller runs it through bf_score / bf_select.
+// 64 queries x 10^6 x 768 int8, top 10, MI355X: 151 us for step 1 (5.1 TB/s, the
+// rate of a large copy) and 76 for the rest, against 2796 for the reference-order
+// scores of every pair and 870 for selecting among them.
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+
+constexpr int kPfBlock = sgk::kBfBlock;  // vectors per block: two 32-row MFMA tiles
+// Threads per workgroup: two column tiles' fragments fill much of the LDS (one
+// workgroup per CU); one leaves room for several smaller workgroups, which
+// share a short index out more evenly.
+template <int CT>
+constexpr int kPfThreads = CT == 2 ? 512 : 256;
+
+// 8 stored elements as fp16 (exact for int8; int16 and v * vscale rounded).
+template <typename T>
+__device__ __forceinline__ half8 pf_half8(const BfRaw<T>& r, float vscale);
+template <>
+__device__ __forceinline__ half8 pf_half8<int8_t>(const BfRaw<int8_t>& r, float) {
+  // c + 128 as the low mantissa bits of 1024: 0x6400 | u is 1024 + u exactly.
+  const half2_t off = {(_Float16)1152.0f, (_Float16)1152.0f};
+  half8 h;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const uint32_t u = (i ? r.w.y : r.w.x) ^ 0x80808080u;
+    const half2_t a = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05010500u)) - off;
+    const half2_t b = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x05030502u)) - off;
+    h[4 * i] = a[0];
+    h[4 * i + 1] = a[1];
+    h[4 * i + 2] = b[0];
+    h[4 * i + 3] = b[1];
+  }
+  return h;
+}
+template <>
+__device__ __forceinline__ half8 pf_half8<int16_t>(const BfRaw<int16_t>& r, float) {
+  const uint32_t u[4] = {r.w.x, r.w.y, r.w.z, r.w.w};
+  half8 h;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    h[2 * i] = (_Float16)(int16_t)(u[i] & 0xffffu);
+    h[2 * i + 1] = (_Float16)(int16_t)(u[i] >> 16);
+  }
+  return h;
+}
+template <>
+__device__ __forceinline__ half8 pf_half8<float>(const BfRaw<float>& r, float vscale) {
+  float v[8];
+  r.get(v);
+  half8 h;
+#pragma unroll
+  for (int i = 0; i < 8; i++) h[i] = (_Float16)(v[i] * vscale);
+  return h;
+}
+
+// Largest L2 norm of the stored vectors in stored units (codes, or floats),
+// as float bits folded by atomicMax; +inf when any is not finite.
+template <typename T>
+__global__ __launch_bounds__(kBfThreads) void k_bf_vnorm(const T* __restrict__ grp, const T* __restrict__ tail, int N,
+                                                        int dim, uint32_t* __restrict__ vmax) {
+  const int n = blockIdx.x * kBfThreads + threadIdx.x;
+  const int nn = min(n, N - 1);
+  const int G = dim >> 3, R = dim & 7;
+  float ss = 0.0f;
+  for (int g = 0; g < G; g += 8) {
+    BfRaw<T> raw[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) raw[u].load(grp + ((int64_t)min(g + u, G - 1) * N + nn) * 8);
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      float v[8], sq = 0.0f;
+      raw[u].get(v);
+#pragma unroll
+      for (int l = 0; l < 8; l++) sq += v[l] * v[l];
+      ss += g + u < G ? sq : 0.0f;
+    }
+  }
+  for (int i = 0; i < R; i++) {
+    float t = (float)tail[(int64_t)nn * R + i];
+    if constexpr (BfElem<T>::kQuant) t = t * BfElem<T>::inv();
+    ss += t * t;
+  }
+  float m = sqrtf(ss);
+  if (!(m <= 3.0e38f)) m = __builtin_inff();
+  m = sg_wave_max(m);
+  if ((threadIdx.x & 63) == 0) atomicMax(vmax, __float_as_uint(m));
+}
+
+// Queries of one pass: normalized in place when asked (builder.go:131-141, as
+// k_bf_normalize), then scaled by a power of two to a largest element in
+// [256, 512) and rounded to fp16 in the MFMA B operand's order, qfrag [k-step
+// of two 8-element groups][col_tiles][64 lanes][8] (lane 32 h + c: query c of
+// the tile, group 2 s + h; the last k-step's first half holds the tail when
+// dim % 8; zeros elsewhere and for queries past nq).  eps[q] = the bound above
+// in k_bf_approx's units; negative: flagged.  One wave per query.
+__global__ __launch_bounds__(64) void k_bf_prep(float* __restrict__ queries, int nq, int dim, int normalize,
+                                               float vnorm_s, int exact_v, int col_tiles, _Float16* __restrict__ qfrag,
+                                               float* __restrict__ eps, int32_t* __restrict__ flags) {
+  extern __shared__ __attribute__((aligned(16))) float buf[];  // dim rounded up to 16, floats then doubles
+  __shared__ float norm;
+  __shared__ int scale;
+  const int q = blockIdx.x, lane = threadIdx.x;
+  const bool live = q < nq;
+  const int dimp = (dim + 15) & ~15;
+  float* x = queries + (int64_t)q * dim;
+  double* sqs = reinterpret_cast<double*>(buf + dimp);
+  for (int i = lane; i < dimp; i += 64) {
+    const float v = live && i < dim ? x[i] : 0.0f;
+    const float sq = v * v;
+    buf[i] = v;
+    sqs[i] = (double)sq;
+  }
+  __syncthreads();
+  if (normalize && live) {
+    if (lane == 0) {
+      // The float64 sum in index order (the pad's zeros add nothing): a chain of
+      // additions, the next 16 squares read under the current 16.
+      double sum = 0.0;
+      double2 cur[8], nxt[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) cur[u] = reinterpret_cast<const double2*>(sqs)[u];
+      for (int i = 0; i < dimp; i += 16) {
+        const int j = min(i + 16, dimp - 16);
+#pragma unroll
+        for (int u = 0; u < 8; u++) nxt[u] = reinterpret_cast<const double2*>(sqs + j)[u];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          sum += cur[u].x;
+          sum += cur[u].y;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) cur[u] = nxt[u];
+      }
+      scale = sum != 0.0;  // a zero vector stays as it is
+      norm = sum != 0.0 ? (float)(1.0 / sqrt(sum)) : 1.0f;
+    }
+    __syncthreads();
+    const float n = norm;
+    if (scale)
+      for (int i = lane; i < dim; i += 64) {
+        buf[i] = buf[i] * n;
+        x[i] = buf[i];
+      }
+    __syncthreads();
+  }
+  float m = 0.0f, ss = 0.0f;
+  bool finite = true;
+  for (int i = lane; i < dim; i += 64) {
+    const float a = fabsf(buf[i]);
+    finite = finite && a <= 1.0e30f;
+    m = fmaxf(m, a);
+  }
+  finite = __ballot(!finite) == 0;
+  m = sg_wave_max(m);
+  const bool ok = live && finite && m >= 1.0e-30f;
+  int e = 0;
+  if (ok) (void)frexpf(m, &e);  // m = f * 2^e, f in [0.5, 1)
+  const float sc = ok ? ldexpf(1.0f, 9 - e) : 0.0f;
+  for (int i = lane; i < dim; i += 64) {
+    const float t = buf[i] * sc;
+    ss += t * t;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+  if (lane == 0 && live) {
+    // Per product: fp16 rounding of x (2^-11) and of v unless exact; the two
+    // accumulations: at most dim + 32 float32 roundings of up to an ulp (2^-23)
+    // each on the matrix cores, dim / 8 + 24 (2^-24) in the reference's order;
+    // sums of |x v| bounded by the norms' product (Cauchy-Schwarz).  fp16
+    // subnormals: 2^-25 per element on either side.
+    const float xn = sqrtf(ss) * 1.001f;
+    const float rel = 4.8829e-4f * (exact_v ? 1.0f : 2.0f) + (float)(dim + 32) * 1.2e-7f +
+                      (float)(dim / 8 + 24) * 6.0e-8f + 1.0e-6f;
+    const float rd = sqrtf((float)dim) * 3.0e-8f;
+    eps[q] = 1.05f * (rel * xn * vnorm_s + rd * (xn + vnorm_s));
+    flags[q] = ok ? 0 : 1;
+  }
+  const int G = dim >> 3, R = dim & 7, ct = q >> 5, c = q & 31;
+  const int ks_main = (G + 1) >> 1, ks = ks_main + (R ? 1 : 0);
+  for (int i = lane; i < ks * 2; i += 64) {  // one 8-element piece per lane
+    const int s = i >> 1, h = i & 1;
+    int src = -1, cnt = 8;
+    if (s < ks_main) {
+      if (2 * s + h < G) src = 8 * (2 * s + h);
+    } else if (h == 0) {
+      src = 8 * G;
+      cnt = R;
+    }
+    half8 v;
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = src >= 0 && u < cnt ? (_Float16)(buf[src + u] * sc) : (_Float16)0.0f;
+    *reinterpret_cast<half8*>(qfrag + (((int64_t)s * col_tiles + ct) * 64 + 32 * h + c) * 8) = v;
+  }
+}
+
+// blockmax[q][nb]: the largest approximate score of each block's 64 vectors,
+// in scaled units.  Bound by reading the index once per pass (HBM): the fp16
+// MFMAs of 64 queries take about a third of that time.  A wave walks blocks
+// b, b + waves, ... with PF k-steps of loads in flight (the ring runs on from
+// block to block); lane (row, h) of a 32-row tile loads group 2 s + h of its
+// vector: 8, 16 or 32 contiguous bytes, 32 vectors side by side.  The queries'
+// fragments sit in LDS.
+template <typename T, int CT, int PF>
+__global__ __launch_bounds__(kPfThreads<CT>, 2) void k_bf_approx(const T* __restrict__ grp, const T* __restrict__ tail,
+                                                            int N, int dim, float vscale,
+                                                            const _Float16* __restrict__ qfrag, int nq,
+                                                            float* __restrict__ blockmax, int nb) {
+  extern __shared__ __attribute__((aligned(16))) _Float16 qs[];  // [ks][CT][64][8]
+  const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int G = dim >> 3, R = dim & 7;
+  const int ks_main = (G + 1) >> 1, ks = ks_main + (R ? 1 : 0);
+  for (int i = threadIdx.x; i < ks * CT * 64; i += kPfThreads<CT>)
+    reinterpret_cast<uint4*>(qs)[i] = reinterpret_cast<const uint4*>(qfrag)[i];
+  __syncthreads();
+  const int nwaves = gridDim.x * (kPfThreads<CT> / 64);
+  const int b0 = blockIdx.x * (kPfThreads<CT> / 64) + wave;
+  if (b0 >= nb) return;
+  const int nblk = (nb - b0 + nwaves - 1) / nwaves;  // this wave's blocks
+  const int64_t steps = (int64_t)nblk * ks_main;
+
+  // Load stream: block lb, k-step ls (past the last step the last one again).
+  int lb = b0, ls = 0;
+  auto fetch = [&](BfRaw<T>(&r)[2]) {
+    const int64_t g = min(2 * ls + lh, G - 1);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      r[t].load(grp + (g * N + min(lb * kPfBlock + 32 * t + lr, N - 1)) * 8);
+    if (ls + 1 < ks_main) {
+      ls++;
+    } else if (lb + nwaves < nb) {
+      ls = 0;
+      lb += nwaves;
+    }
+  };
+  BfRaw<T> ring[PF][2];
+#pragma unroll
+  for (int i = 0; i < PF; i++) fetch(ring[i]);
+
+  f32x16_t acc[2][CT];
+  auto clear = [&]() {
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int c = 0; c < CT; c++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][c][r] = 0.0f;
+  };
+  auto mul = [&](int s, const half8 (&a)[2]) {
+#pragma unroll
+    for (int c = 0; c < CT; c++) {
+      const half8 b = *reinterpret_cast<const half8*>(qs + ((s * CT + c) * 64 + lane) * 8);
+#pragma unroll
+      for (int t = 0; t < 2; t++) acc[t][c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t], b, acc[t][c], 0, 0, 0);
+    }
+  };
+  clear();
+  int b = b0, s = 0;
+  for (int64_t st = 0; st < steps; st += PF) {
+#pragma unroll
+    for (int i = 0; i < PF; i++) {
+      if (st + i < steps) {
+        half8 a[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) a[t] = pf_half8<T>(ring[i][t], vscale);
+        fetch(ring[i]);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(s, a);
+        if (++s == ks_main) {  // wave-uniform: the block is complete
+          if (R) {
+            half8 tl[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+              const T* tp = tail + (int64_t)min(b * kPfBlock + 32 * t + lr, N - 1) * R;
+#pragma unroll
+              for (int u = 0; u < 8; u++) {
+                float v = u < R ? (float)tp[min(u, R - 1)] : 0.0f;
+                if constexpr (!BfElem<T>::kQuant) v = v * vscale;
+                tl[t][u] = lh == 0 ? (_Float16)v : (_Float16)0.0f;
+              }
+            }
+            mul(ks_main, tl);
+          }
+#pragma unroll
+          for (int c = 0; c < CT; c++) {
+            float m = acc[0][c][0];
+#pragma unroll
+            for (int r = 0; r < 16; r++) m = fmaxf(m, fmaxf(acc[0][c][r], acc[1][c][r]));
+            m = fmaxf(m, __shfl_xor(m, 32));
+            const int q = 32 * c + lr;
+            if (lh == 0 && q < nq) blockmax[(int64_t)q * nb + b] = m;
+          }
+          clear();
+          s = 0;
+          b += nwaves;
+        }
+      }
+    }
+  }
+}
+
+// The value T of a workgroup's radix select over n keys key(i), i < n: the keys'
+// top bits (kSelBits0 + kSelBits1 [+ kSelBits2]) of the k-th largest key with
+// the rest zero; above = keys above T's bin, at = keys in it.  hist: 2048 + 64
+// words of LDS.  Every thread of the workgroup calls this.
+constexpr int kTopThreads = 1024;
+template <int PASSES, typename F>
+__device__ __forceinline__ void wg_select(F key, int n, int k, uint32_t* hist, uint32_t& T, int& above, int& at) {
+  __shared__ uint32_t sh_prefix;
+  __shared__ int sh_above, sh_at;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  uint32_t prefix = 0;
+  int gone = 0, in_bin = 0;
+#pragma unroll
+  for (int p = 0; p < PASSES; p++) {
+    const int bits = p < 2 ? 11 : 10, shift = p == 0 ? 21 : p == 1 ? 10 : 0;
+    const uint32_t mask = p == 0 ? 0u : ~0u << (p == 1 ? 21 : 10);
+    for (int i = tid; i < 2048; i += kTopThreads) hist[i] = 0;
+    __syncthreads();
+    for (int i0 = 0; i0 < n; i0 += kTopThreads) {
+      const int i = i0 + tid;
+      int bin = -1;
+      if (i < n) {
+        const uint32_t u = key(i);
+        if ((u & mask) == prefix) bin = (int)((u >> shift) & ((1u << bits) - 1u));
+      }
+      // Scores crowd into a few bins of the top digit: one addition per
+      // distinct bin of the wave there.
+      if (p == 0) {
+        uint64_t todo = __ballot(bin >= 0);
+        while (todo) {
+          const int lb = __shfl(bin, __builtin_ctzll(todo));
+          const uint64_t same = __ballot(bin == lb);
+          if (lane == 0) atomicAdd(&hist[lb], (uint32_t)__popcll(same));
+          todo &= ~same;
+        }
+      } else if (bin >= 0) {
+        atomicAdd(&hist[bin], 1u);
+      }
+    }
+    __syncthreads();
+    // Suffix counts: thread t owns bins 2t, 2t + 1.
+    uint32_t* wsum = hist + 2048;
+    const uint32_t c0 = hist[2 * tid], c1 = hist[2 * tid + 1];
+    uint32_t run = c0 + c1;  // inclusive suffix over the wave's lanes >= this one
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t v = __shfl_down(run, o);
+      if (lane + o < 64) run += v;
+    }
+    if (lane == 0) wsum[wave] = run;
+    __syncthreads();
+    uint32_t after = run - c0 - c1;
+    for (int w2 = wave + 1; w2 < kTopThreads / 64; w2++) after += wsum[w2];
+    const uint32_t need = (uint32_t)(k - gone);
+    // bin b with (keys in higher bins) < need <= (those + its own)
+    if (after < need && need <= after + c1) {
+      sh_prefix = prefix | ((uint32_t)(2 * tid + 1) << shift);
+      sh_above = gone + (int)after;
+      sh_at = (int)c1;
+    } else if (after + c1 < need && need <= after + c1 + c0) {
+      sh_prefix = prefix | ((uint32_t)(2 * tid) << shift);
+      sh_above = gone + (int)(after + c1);
+      sh_at = (int)c0;
+    }
+    __syncthreads();
+    prefix = sh_prefix;
+    gone = sh_above;
+    in_bin = sh_at;
+    __syncthreads();
+  }
+  T = prefix;
+  above = gone;
+  at = in_bin;
+}
+
+// The float whose bf_key is u.
+__device__ __forceinline__ float bf_unkey(uint32_t u) {
+  return __uint_as_float((u & 0x80000000u) ? u & 0x7fffffffu : ~u);
+}
+
+// list[q][0 .. count[q]): the blocks that can hold one of query q's k best.
+__global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restrict__ blockmax, int nb, int k,
+                                                          const float* __restrict__ eps, int cap,
+                                                          int32_t* __restrict__ list, int32_t* __restrict__ count,
+                                                          int32_t* __restrict__ flags) {
+  __shared__ uint32_t hist[2048 + 64];
+  __shared__ int cnt;
+  const int q = blockIdx.x;
+  const float* bm = blockmax + (int64_t)q * nb;
+  if (flags[q]) {  // workgroup-uniform
+    if (threadIdx.x == 0) count[q] = 0;
+    return;
+  }
+  uint32_t T;
+  int above, at;
+  // The k-th largest maximum of four blocks each: at least k blocks reach it,
+  // for a quarter of the keys.  Its low bits are zero, and the cut's own
+  // rounding is covered by eps' slack.
+  wg_select<2>(
+      [&](int i) {
+        float m = bm[4 * i];
+#pragma unroll
+        for (int u = 1; u < 4; u++) m = fmaxf(m, bm[min(4 * i + u, nb - 1)]);
+        return bf_key(m);
+      },
+      (nb + 3) / 4, k, hist, T, above, at);
+  const float cut = bf_unkey(T) - 2.0f * eps[q];
+  if (threadIdx.x == 0) cnt = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < nb; i += kTopThreads)
+    if (bm[i] >= cut) {
+      const int slot = atomicAdd(&cnt, 1);
+      if (slot < cap) list[(int64_t)q * cap + slot] = i;
+    }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    count[q] = cnt <= cap ? cnt : 0;
+    if (cnt > cap) flags[q] = 1;
+  }
+}
+
+// cand[q][64 i + l]: the score of vector 64 list[q][i] + l in the reference's
+// order (k_bf_score's arithmetic; one query, lane = vector); a wave per listed
+// block.  Vectors past N: NaN bits 0xffffffff, whose key is 0.
+template <typename T>
+__global__ __launch_bounds__(kBfThreads) void k_bf_rescore(const T* __restrict__ grp, const T* __restrict__ tail, int N,
+                                                          int dim, const float* __restrict__ queries,
+                                                          const int32_t* __restrict__ list,
+                                                          const int32_t* __restrict__ count, int cap,
+                                                          float* __restrict__ cand) {
+  constexpr int B = sizeof(T) == 4 ? 8 : 16;  // groups in flight per lane
+  const int q = blockIdx.y, lane = threadIdx.x & 63;
+  const int i = blockIdx.x * (kBfThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (i >= count[q]) return;
+  const int n = list[(int64_t)q * cap + i] * kPfBlock + lane;
+  const int nn = min(n, N - 1);
+  const int G = dim >> 3, R = dim & 7;
+  const float* x = queries + (int64_t)q * dim;
+  float acc[8];
+#pragma unroll
+  for (int l = 0; l < 8; l++) acc[l] = 0.0f;
+  auto add = [&](const BfRaw<T>& raw, int g) {
+    float v[8];
+    raw.get(v);
+#pragma unroll
+    for (int l = 0; l < 8; l++) {
+      const float xv = x[8 * g + l];
+      if constexpr (BfElem<T>::kQuant) {
+        const float p = v[l] * xv;
+        acc[l] = acc[l] + p;
+      } else {
+        acc[l] = __builtin_fmaf(v[l], xv, acc[l]);
+      }
+    }
+  };
+  // Batches of B loads, the next batch in flight under the current one's sums
+  // (no branch between a load and its use: it would sink the loads).
+  const T* gp = grp + (int64_t)nn * 8;
+  const int64_t gs = (int64_t)N * 8;
+  BfRaw<T> cur[B], nxt[B];
+#pragma unroll
+  for (int u = 0; u < B; u++) cur[u].load(gp + min(u, G - 1) * gs);
+  int g = 0;
+  for (; g + B <= G; g += B) {
+#pragma unroll
+    for (int u = 0; u < B; u++) nxt[u].load(gp + min(g + B + u, G - 1) * gs);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < B; u++) add(cur[u], g + u);
+#pragma unroll
+    for (int u = 0; u < B; u++) cur[u] = nxt[u];
+  }
+#pragma unroll
+  for (int u = 0; u < B; u++)
+    if (g + u < G) add(cur[u], g + u);
+  const float sum = bf_finish<T>(acc, G, R, x + 8 * G, tail + (int64_t)nn * R);
+  cand[((int64_t)q * cap + i) * kPfBlock + lane] = n < N ? sum : __uint_as_float(0xffffffffu);
+}
+
+// The exact top k of the candidates: out_idx/out_dist [q][k] in arbitrary
+// order; a tie straddling the k-th place flags the query.
+__global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict__ cand,
+                                                       const int32_t* __restrict__ list,
+                                                       const int32_t* __restrict__ count, int cap, int k,
+                                                       int32_t* __restrict__ out_idx, float* __restrict__ out_dist,
+                                                       int32_t* __restrict__ flags) {
+  __shared__ uint32_t hist[2048 + 64];
+  __shared__ int cnt;
+  const int q = blockIdx.x;
+  const int n = count[q] * kPfBlock;
+  if (flags[q] || n < k) {
+    if (threadIdx.x == 0) flags[q] = 1;
+    return;
+  }
+  const float* cs = cand + (int64_t)q * cap * kPfBlock;
+  auto key = [&](int i) {
+    const float d = cs[i];
+    return __float_as_uint(d) == 0xffffffffu ? 0u : bf_key(d);
+  };
+  uint32_t T;
+  int above, at;
+  wg_select<3>(key, n, k, hist, T, above, at);
+  if (above + at != k) {
+    if (threadIdx.x == 0) flags[q] = 1;
+    return;
+  }
+  if (threadIdx.x == 0) cnt = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += kTopThreads)
+    if (key(i) >= T) {
+      const int slot = atomicAdd(&cnt, 1);
+      if (slot < k) {
+        out_idx[(int64_t)q * k + slot] = list[(int64_t)q * cap + i / kPfBlock] * kPfBlock + i % kPfBlock;
+        out_dist[(int64_t)q * k + slot] = cs[i];
+      }
+    }
+}
+
 __global__ void k_bf_fill_i32(int32_t* p, int64_t n, int32_t v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -554,7 +1150,7 @@ namespace sgk {
 hipError_t bf_build(int mode, const float* src, int64_t ld, int n, int dim, int row0, int N, void* grp, void* tail,
                     bool normalize, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  const unsigned nb = nblocks(n, kBfThreads);
+  const unsigned nb = nblocks(n, kBuildRows);
   const int nz = normalize ? 1 : 0;
   switch (mode) {
     case kBfF32:
@@ -654,6 +1250,96 @@ hipError_t bf_select(const float* scores, int64_t ld_scores, int N, int nq, int 
     hipLaunchKernelGGL(k_bf_radix, grid, dim3(kBfThreads), 0, s, scores, ld_scores, N, digit, state, hist);
   hipLaunchKernelGGL(k_bf_collect, grid, dim3(kBfThreads), 0, s, scores, ld_scores, N, k, state, out_idx, out_dist);
   hipLaunchKernelGGL(k_bf_stream, dim3(nq), dim3(64), 0, s, scores, ld_scores, N, k, state, out_idx, out_dist);
+  return hipGetLastError();
+}
+
+hipError_t bf_vnorm(int mode, const void* grp, const void* tail, int N, int dim, uint32_t* vmax, hipStream_t s) {
+  if (N <= 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_bf_fill_i32, dim3(1), dim3(64), 0, s, reinterpret_cast<int32_t*>(vmax), (int64_t)1, 0);
+  const dim3 grid(nblocks(N, kBfThreads)), blk(kBfThreads);
+  switch (mode) {
+    case kBfF32:
+      hipLaunchKernelGGL(k_bf_vnorm<float>, grid, blk, 0, s, static_cast<const float*>(grp),
+                         static_cast<const float*>(tail), N, dim, vmax);
+      break;
+    case kBfI8:
+      hipLaunchKernelGGL(k_bf_vnorm<int8_t>, grid, blk, 0, s, static_cast<const int8_t*>(grp),
+                         static_cast<const int8_t*>(tail), N, dim, vmax);
+      break;
+    case kBfI16:
+      hipLaunchKernelGGL(k_bf_vnorm<int16_t>, grid, blk, 0, s, static_cast<const int16_t*>(grp),
+                         static_cast<const int16_t*>(tail), N, dim, vmax);
+      break;
+    default:
+      return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+namespace {
+int pf_ksteps(int dim) { return ((dim >> 3) + 1) / 2 + ((dim & 7) ? 1 : 0); }
+
+template <typename T, int CT>
+hipError_t approx_t(const void* grp, const void* tail, int N, int dim, float vscale, const _Float16* qfrag, int nq,
+                    float* blockmax, int nb, hipStream_t s) {
+  constexpr int PF = sizeof(T) == 1 ? 12 : sizeof(T) == 2 ? 8 : 6;
+  constexpr int waves = kPfThreads<CT> / 64, most = 256 * (CT == 2 ? 1 : 3);
+  const int wgs = (nb + waves - 1) / waves;
+  const size_t lds = (size_t)pf_ksteps(dim) * CT * 1024;
+  hipLaunchKernelGGL((k_bf_approx<T, CT, PF>), dim3(wgs < most ? wgs : most), dim3(kPfThreads<CT>), lds, s,
+                     static_cast<const T*>(grp), static_cast<const T*>(tail), N, dim, vscale, qfrag, nq, blockmax, nb);
+  return hipGetLastError();
+}
+}  // namespace
+
+bool bf_prefilter_ok(int N, int dim, int k, float vnorm) {
+  const int nb = (N + kBfBlock - 1) / kBfBlock;
+  return N <= (1 << 30) && dim >= 16 && (size_t)pf_ksteps(dim) * 1024 <= kBfPfLds && nb >= 2 * bf_prefilter_cap(k) &&
+         vnorm >= 1.0e-30f && vnorm <= 1.0e30f;
+}
+
+int bf_prefilter_queries(int dim) { return (size_t)pf_ksteps(dim) * 2048 <= kBfPfLds ? 64 : 32; }
+
+hipError_t bf_prefilter(int mode, const void* grp, const void* tail, int N, int dim, float vnorm, float* queries,
+                        int nq, bool normalize, int k, const sg_bf_work& w, hipStream_t s) {
+  if (nq <= 0 || nq > bf_prefilter_queries(dim) || !bf_prefilter_ok(N, dim, k, vnorm)) return hipErrorInvalidValue;
+  const int ct = nq > 32 ? 2 : 1, nb = (N + kBfBlock - 1) / kBfBlock, cap = bf_prefilter_cap(k);
+  // Stored norm in the units of the fp16 operand: codes as they are (the norm
+  // is in dequantized units), floats scaled by a power of two to a largest
+  // norm in [128, 256).
+  float vscale = 1.0f, vs = vnorm;
+  if (mode == kBfF32) {
+    int e = 0;
+    (void)frexpf(vnorm, &e);
+    vscale = ldexpf(1.0f, 8 - e);
+    vs = vnorm * vscale;
+  } else {
+    vs = vnorm * (mode == kBfI8 ? 127.0f : 32767.0f);
+  }
+  hipLaunchKernelGGL(k_bf_prep, dim3(32 * ct), dim3(64), (sizeof(float) + sizeof(double)) * (size_t)((dim + 15) & ~15), s, queries, nq, dim,
+                     normalize ? 1 : 0, vs * 1.01f, mode == kBfI8 ? 1 : 0, ct, w.qfrag, w.eps, w.flags);
+  hipError_t e = hipErrorInvalidValue;
+  switch (mode) {
+#define SG_PF(MODE, T)                                                                                           \
+  case MODE:                                                                                                     \
+    e = ct == 2 ? approx_t<T, 2>(grp, tail, N, dim, vscale, w.qfrag, nq, w.blockmax, nb, s)                      \
+                : approx_t<T, 1>(grp, tail, N, dim, vscale, w.qfrag, nq, w.blockmax, nb, s);                     \
+    if (e != hipSuccess) return e;                                                                               \
+    hipLaunchKernelGGL(k_bf_blocks, dim3(nq), dim3(kTopThreads), 0, s, w.blockmax, nb, k, w.eps, cap, w.list,    \
+                       w.count, w.flags);                                                                        \
+    hipLaunchKernelGGL(k_bf_rescore<T>, dim3(nblocks(cap, kBfThreads / 64), nq), dim3(kBfThreads), 0, s,         \
+                       static_cast<const T*>(grp), static_cast<const T*>(tail), N, dim, queries, w.list, w.count, \
+                       cap, w.cand);                                                                             \
+    break;
+    SG_PF(kBfF32, float)
+    SG_PF(kBfI8, int8_t)
+    SG_PF(kBfI16, int16_t)
+#undef SG_PF
+    default:
+      return e;
+  }
+  hipLaunchKernelGGL(k_bf_top, dim3(nq), dim3(kTopThreads), 0, s, w.cand, w.list, w.count, cap, k, w.out_idx,
+                     w.out_dist, w.flags);
   return hipGetLastError();
 }
 

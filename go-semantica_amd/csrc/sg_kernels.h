@@ -278,4 +278,29 @@ hipError_t bf_score(int mode, const void* grp, const void* tail, int N, int dim,
 hipError_t bf_select(const float* scores, int64_t ld_scores, int N, int nq, int k, int32_t* state, uint32_t* hist,
                      int32_t* out_idx, float* out_dist, hipStream_t s);
 
+// ---- prefiltered search (k_search.hip, "prefiltering") ----
+// Largest L2 norm of the stored vectors (dequantized units), as float bits in
+// *vmax (device); +inf when one is not finite.
+hipError_t bf_vnorm(int mode, const void* grp, const void* tail, int N, int dim, uint32_t* vmax, hipStream_t s);
+constexpr int kBfBlock = 64;            // vectors per block
+constexpr size_t kBfPfLds = 144 << 10;  // LDS for the queries' fragments
+inline int bf_prefilter_cap(int k) { return 4 * k + 64; }  // listed blocks per query
+bool bf_prefilter_ok(int N, int dim, int k, float vnorm);
+int bf_prefilter_queries(int dim);  // queries per call
+struct sg_bf_work {
+  _Float16* qfrag;   // 64 x (dim rounded up to 32) + 1024
+  float* eps;        // [nq]
+  float* blockmax;   // [nq][blocks]
+  int32_t* list;     // [nq][cap]
+  int32_t* count;    // [nq]
+  float* cand;       // [nq][cap * kBfBlock]
+  int32_t* out_idx;  // [nq][k]
+  float* out_dist;   // [nq][k]
+  int32_t* flags;    // [nq]: 1 = not decided, run the query through bf_score / bf_select
+};
+// queries [nq][dim]: normalized in place when `normalize` (bf_normalize's
+// arithmetic).  out_idx / out_dist as bf_select's, for the unflagged queries.
+hipError_t bf_prefilter(int mode, const void* grp, const void* tail, int N, int dim, float vnorm, float* queries,
+                        int nq, bool normalize, int k, const sg_bf_work& w, hipStream_t s);
+
 }  // namespace sgk

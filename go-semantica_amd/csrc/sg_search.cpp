@@ -33,11 +33,13 @@ struct sg_index {
   std::vector<int32_t> ids;
   std::unordered_map<int32_t, int> pos;
   DevBuf grp, tail;                                  // the vectors
-  DevBuf stage, queries, scores, state, hist, oidx, odist;  // call workspace
+  float vnorm = 0.0f;  // largest stored L2 norm (sgk::bf_vnorm); 0: none
+  DevBuf stage, queries, scores, state, hist, out;  // call workspace; out: [idx | dist | flags]
+  DevBuf pf, redo;                                  // prefiltered search: its workspace; undecided queries
   HostBuf h_in, h_out;
   std::mutex mu;
   ~sg_index() {
-    for (DevBuf* b : {&grp, &tail, &stage, &queries, &scores, &state, &hist, &oidx, &odist}) b->release();
+    for (DevBuf* b : {&grp, &tail, &stage, &queries, &scores, &state, &hist, &out, &pf, &redo}) b->release();
     h_in.release();
     h_out.release();
   }
@@ -79,6 +81,18 @@ int make_index(sg_ctx* ctx, int dim, int mode, const int32_t* ids, int n, sg_ind
     return r;
   }
   *out = x;
+  return SG_OK;
+}
+
+// The stored vectors' largest norm, once they are in place (synchronizes s).
+int finish_index(sg_index* x, hipStream_t s) {
+  if (x->count == 0) return SG_OK;
+  uint32_t bits = 0;
+  SG_TRY(x->state.ensure(sizeof(int32_t) * 8));
+  SG_HIP(sgk::bf_vnorm(x->mode, x->grp.p, x->tail.p, x->count, x->dim, x->state.as<uint32_t>(), s));
+  SG_HIP(hipMemcpyAsync(&bits, x->state.p, sizeof bits, hipMemcpyDeviceToHost, s));
+  SG_HIP(hipStreamSynchronize(s));
+  memcpy(&x->vnorm, &bits, sizeof bits);
   return SG_OK;
 }
 
@@ -151,6 +165,7 @@ int sg_index_build(sg_ctx* ctx, int32_t dim, int32_t quantization, const int32_t
     if (e != hipSuccess) r = fail(SG_ERR_DEVICE, "index build: %s", hipGetErrorString(e));
   }
   x->stage.release();
+  if (r == SG_OK) r = finish_index(x, s);
   if (r != SG_OK) {
     delete x;
     return r;
@@ -171,10 +186,11 @@ int sg_index_build_device(sg_ctx* ctx, int32_t dim, int32_t quantization, const 
   sg_index* x = nullptr;
   SG_TRY(make_index(ctx, dim, quantization, ids, n, &x));
   hipError_t e = sgk::bf_build(quantization, d_vectors, ld, n, dim, 0, n, x->grp.p, x->tail.p, true, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  if (e != hipSuccess) {
+  const int r = e == hipSuccess ? finish_index(x, s) : fail(SG_ERR_DEVICE, "index build: %s", hipGetErrorString(e));
+  if (r != SG_OK) {
+    (void)hipStreamSynchronize(s);
     delete x;
-    return fail(SG_ERR_DEVICE, "index build: %s", hipGetErrorString(e));
+    return r;
   }
   *out = x;
   return SG_OK;
@@ -219,6 +235,7 @@ int sg_index_deserialize(sg_ctx* ctx, const void* data, size_t size, sg_index** 
     if (e != hipSuccess) r = fail(SG_ERR_DEVICE, "index upload: %s", hipGetErrorString(e));
   }
   x->stage.release();
+  if (r == SG_OK) r = finish_index(x, s);
   if (r != SG_OK) {
     delete x;
     return r;
@@ -310,48 +327,107 @@ int sg_index_search(sg_index* x, const float* queries, int32_t n_queries, int32_
   }
   SG_HIP(hipSetDevice(sgi::ctx_device(x->ctx)));
   hipStream_t s = sgi::ctx_stream(x->ctx, stream);
-  const int qb = (int)std::max<size_t>(1, std::min<size_t>((size_t)n_queries, kScoreBytes / (sizeof(float) * N)));
+  const bool pre = sgk::bf_prefilter_ok(N, dim, k, x->vnorm);
+  const size_t full_qb = std::max<size_t>(1, std::min<size_t>((size_t)n_queries, kScoreBytes / (sizeof(float) * N)));
+  int qb = (int)full_qb;
+  if (pre) {
+    const size_t per = sizeof(float) * (size_t)sgk::bf_prefilter_cap(k) * sgk::kBfBlock;
+    qb = std::min(std::min(n_queries, sgk::bf_prefilter_queries(dim)), (int)std::max<size_t>(1, kScoreBytes / per));
+  }
   SG_TRY(x->queries.ensure(sizeof(float) * (size_t)qb * dim));
-  SG_TRY(x->scores.ensure(sizeof(float) * (size_t)qb * N));
-  SG_TRY(x->state.ensure(sizeof(int32_t) * 8 * (size_t)qb));
-  SG_TRY(x->hist.ensure(sizeof(uint32_t) * 256 * (size_t)qb));
-  SG_TRY(x->oidx.ensure(sizeof(int32_t) * (size_t)qb * k));
-  SG_TRY(x->odist.ensure(sizeof(float) * (size_t)qb * k));
+  SG_TRY(x->out.ensure(sizeof(int32_t) * ((size_t)qb * k * 2 + qb)));
   SG_TRY(x->h_in.ensure(sizeof(float) * (size_t)qb * dim));
-  SG_TRY(x->h_out.ensure((sizeof(int32_t) + sizeof(float)) * (size_t)qb * k));
+  SG_TRY(x->h_out.ensure(sizeof(int32_t) * ((size_t)qb * k * 2 + qb)));
   struct Res {
     int32_t id;
     float dist;
   };
   std::vector<Res> res((size_t)k);
+  // One query's k positions and scores, in the reference's final order.
+  auto emit = [&](int q, const int32_t* hi, const float* hd) {
+    for (int j = 0; j < k; j++) {
+      const int32_t p = hi[j];
+      if (p < 0 || p >= N) return fail(SG_ERR_DEVICE, "top-k selection left slot %d of query %d empty", j, q);
+      res[j] = Res{x->ids[p], hd[j]};
+    }
+    std::sort(res.begin(), res.end(), [](const Res& a, const Res& b) {
+      return a.dist == b.dist ? a.id < b.id : a.dist > b.dist;  // index.go:133-137
+    });
+    for (int j = 0; j < k; j++) {
+      out_ids[(size_t)q * top_k + j] = res[j].id;
+      out_dist[(size_t)q * top_k + j] = res[j].dist;
+    }
+    n_found[q] = k;
+    return SG_OK;
+  };
+  // Every score of nq (normalized) queries on the device, then the selection:
+  // positions and scores to x->h_out as [idx | dist].
+  auto full = [&](const float* queries_d, int nq) {
+    SG_TRY(x->scores.ensure(sizeof(float) * (size_t)nq * N));
+    SG_TRY(x->state.ensure(sizeof(int32_t) * 8 * (size_t)nq));
+    SG_TRY(x->hist.ensure(sizeof(uint32_t) * 256 * (size_t)nq));
+    int32_t* oi = x->out.as<int32_t>();
+    SG_HIP(sgk::bf_score(x->mode, x->grp.p, x->tail.p, N, dim, queries_d, nq, x->scores.as<float>(), N, s));
+    SG_HIP(sgk::bf_select(x->scores.as<float>(), N, N, nq, k, x->state.as<int32_t>(), x->hist.as<uint32_t>(), oi,
+                          reinterpret_cast<float*>(oi + (size_t)nq * k), s));
+    SG_HIP(hipMemcpyAsync(x->h_out.p, oi, sizeof(int32_t) * (size_t)nq * k * 2, hipMemcpyDeviceToHost, s));
+    SG_HIP(hipStreamSynchronize(s));
+    return SG_OK;
+  };
+  int32_t* hi = x->h_out.as<int32_t>();
   for (int q0 = 0; q0 < n_queries; q0 += qb) {
     const int nq = std::min(qb, n_queries - q0);
+    float* qd = x->queries.as<float>();
     memcpy(x->h_in.p, queries + (size_t)q0 * dim, sizeof(float) * (size_t)nq * dim);
-    SG_HIP(hipMemcpyAsync(x->queries.p, x->h_in.p, sizeof(float) * (size_t)nq * dim, hipMemcpyHostToDevice, s));
-    if (normalize) SG_HIP(sgk::bf_normalize(x->queries.as<float>(), nq, dim, s));
-    SG_HIP(sgk::bf_score(x->mode, x->grp.p, x->tail.p, N, dim, x->queries.as<float>(), nq, x->scores.as<float>(), N,
-                         s));
-    SG_HIP(sgk::bf_select(x->scores.as<float>(), N, N, nq, k, x->state.as<int32_t>(), x->hist.as<uint32_t>(),
-                          x->oidx.as<int32_t>(), x->odist.as<float>(), s));
-    int32_t* hi = x->h_out.as<int32_t>();
-    float* hd = reinterpret_cast<float*>(hi + (size_t)nq * k);
-    SG_HIP(hipMemcpyAsync(hi, x->oidx.p, sizeof(int32_t) * (size_t)nq * k, hipMemcpyDeviceToHost, s));
-    SG_HIP(hipMemcpyAsync(hd, x->odist.p, sizeof(float) * (size_t)nq * k, hipMemcpyDeviceToHost, s));
+    SG_HIP(hipMemcpyAsync(qd, x->h_in.p, sizeof(float) * (size_t)nq * dim, hipMemcpyHostToDevice, s));
+    if (!pre) {
+      if (normalize) SG_HIP(sgk::bf_normalize(qd, nq, dim, s));
+      SG_TRY(full(qd, nq));
+      for (int q = 0; q < nq; q++)
+        SG_TRY(emit(q0 + q, hi + (size_t)q * k, reinterpret_cast<float*>(hi + (size_t)nq * k) + (size_t)q * k));
+      continue;
+    }
+    // Prefiltered: the workspace's parts, then the output's.
+    const size_t nb = ((size_t)N + sgk::kBfBlock - 1) / sgk::kBfBlock, cap = (size_t)sgk::bf_prefilter_cap(k);
+    const size_t frag = (size_t)64 * ((dim + 31) & ~31) + 64 * 32;  // halves
+    size_t off = 0;
+    auto part = [&](size_t bytes) {
+      const size_t o = off;
+      off += (bytes + 255) & ~(size_t)255;
+      return o;
+    };
+    const size_t o_frag = part(sizeof(_Float16) * frag), o_eps = part(sizeof(float) * qb),
+                 o_bm = part(sizeof(float) * qb * nb), o_list = part(sizeof(int32_t) * qb * cap),
+                 o_cnt = part(sizeof(int32_t) * qb), o_cand = part(sizeof(float) * qb * cap * sgk::kBfBlock);
+    SG_TRY(x->pf.ensure(off));
+    uint8_t* pw = x->pf.as<uint8_t>();
+    int32_t* oi = x->out.as<int32_t>();
+    int32_t* flags = oi + (size_t)nq * k * 2;
+    const sgk::sg_bf_work w{reinterpret_cast<_Float16*>(pw + o_frag), reinterpret_cast<float*>(pw + o_eps),
+                            reinterpret_cast<float*>(pw + o_bm), reinterpret_cast<int32_t*>(pw + o_list),
+                            reinterpret_cast<int32_t*>(pw + o_cnt), reinterpret_cast<float*>(pw + o_cand), oi,
+                            reinterpret_cast<float*>(oi + (size_t)nq * k), flags};
+    SG_HIP(sgk::bf_prefilter(x->mode, x->grp.p, x->tail.p, N, dim, x->vnorm, qd, nq, normalize != 0, k, w, s));
+    SG_HIP(hipMemcpyAsync(hi, oi, sizeof(int32_t) * ((size_t)nq * k * 2 + nq), hipMemcpyDeviceToHost, s));
     SG_HIP(hipStreamSynchronize(s));
+    std::vector<int> again;
+    const int32_t* hf = hi + (size_t)nq * k * 2;
     for (int q = 0; q < nq; q++) {
-      for (int j = 0; j < k; j++) {
-        const int32_t p = hi[(size_t)q * k + j];
-        if (p < 0 || p >= N) return fail(SG_ERR_DEVICE, "top-k selection left slot %d of query %d empty", j, q0 + q);
-        res[j] = Res{x->ids[p], hd[(size_t)q * k + j]};
-      }
-      std::sort(res.begin(), res.end(), [](const Res& a, const Res& b) {
-        return a.dist == b.dist ? a.id < b.id : a.dist > b.dist;  // index.go:133-137
-      });
-      for (int j = 0; j < k; j++) {
-        out_ids[(size_t)(q0 + q) * top_k + j] = res[j].id;
-        out_dist[(size_t)(q0 + q) * top_k + j] = res[j].dist;
-      }
-      n_found[q0 + q] = k;
+      if (hf[q])
+        again.push_back(q);
+      else
+        SG_TRY(emit(q0 + q, hi + (size_t)q * k, reinterpret_cast<float*>(hi + (size_t)nq * k) + (size_t)q * k));
+    }
+    // Undecided queries (already normalized in place): every score.
+    for (size_t a = 0; a < again.size(); a += full_qb) {
+      const int m = (int)std::min(full_qb, again.size() - a);
+      SG_TRY(x->redo.ensure(sizeof(float) * (size_t)m * dim));
+      for (int i = 0; i < m; i++)
+        SG_HIP(hipMemcpyAsync(x->redo.as<float>() + (size_t)i * dim, qd + (size_t)again[a + i] * dim,
+                              sizeof(float) * dim, hipMemcpyDeviceToDevice, s));
+      SG_TRY(full(x->redo.as<float>(), m));
+      for (int i = 0; i < m; i++)
+        SG_TRY(emit(q0 + again[a + i], hi + (size_t)i * k, reinterpret_cast<float*>(hi + (size_t)m * k) + (size_t)i * k));
     }
   }
   return SG_OK;

@@ -283,3 +283,68 @@ def test_large_index(gpu_ctx):
             assert np.array_equal(gi[q], wi) and np.array_equal(gd[q].view(np.uint32), wd.view(np.uint32))
     finally:
         idx.close()
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("dim,n,nq,k", [
+    (16, 20011, 1, 10),     # one k-step; one query
+    (23, 20011, 33, 1),     # odd group count (2) and a 7-element tail; two column tiles
+    (136, 17664, 40, 20),   # odd group count (17), whole blocks only
+    (257, 13312, 65, 10),   # a 1-element tail; the smallest index taken at k = 10; two passes
+    (768, 26001, 64, 37),
+    (1300, 9000, 34, 1),    # fragments of 32 queries fill the LDS: two passes of one column tile
+])
+def test_prefiltered_search_matches_oracle(gpu_ctx, mode, dim, n, nq, k):
+    """Indexes large enough for the matrix-core prefilter (at least twice the
+    listed-block capacity): ids and distances identical to the oracle's, over
+    clustered vectors (many scores close to the k-th), with queries that are
+    stored vectors, and with ones the prefilter hands back: zero, not finite
+    in its fp16 scaling (1e-35, 1e35), a tie straddling the k-th place (a
+    vector stored twice and searched for with k = 1)."""
+    rng = np.random.default_rng(dim * 7 + mode)
+    topics = rng.standard_normal((12, dim)).astype(np.float32)
+    vecs = (0.3 * rng.standard_normal((n, dim)) + topics[rng.integers(0, 12, n)]).astype(np.float32)
+    vecs[n - 1] = vecs[5]
+    ids = rng.permutation(3 * n)[:n].astype(np.int32)
+    idx = _build(gpu_ctx, ids, vecs, mode)
+    q = (topics[rng.integers(0, 12, nq)] + 0.4 * rng.standard_normal((nq, dim))).astype(np.float32)
+    q[0] = vecs[5]
+    if nq > 8:
+        q[3] = 0.0
+        q[5] = vecs[n // 2]
+        q[6] = -vecs[7]
+    say(f"prefilter mode={MODE_NAMES[mode]} dim={dim} n={n} q={nq} k={k}")
+    _check(idx, vecs, ids, mode, q, k, False, "normalized by the search")
+    q[nq - 1] *= np.float32(1e-35) if mode else np.float32(1e35)
+    _check(idx, vecs, ids, mode, q, k, True, "as given")
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_prefilter_hands_back_crowded_queries(gpu_ctx, mode):
+    """Vectors so alike that every block can hold one of the k best: more
+    blocks than the list takes, so the queries run through the full scoring."""
+    rng = np.random.default_rng(91 + mode)
+    n, dim, k = 20000, 64, 10
+    base = rng.standard_normal(dim)
+    vecs = (base + 1e-5 * rng.standard_normal((n, dim))).astype(np.float32)
+    ids = np.arange(n, dtype=np.int32)
+    q = np.stack([base, base + 0.1 * rng.standard_normal(dim), rng.standard_normal(dim)]).astype(np.float32)
+    say(f"crowded mode={MODE_NAMES[mode]}")
+    _check(_build(gpu_ctx, ids, vecs, mode), vecs, ids, mode, q, k, False, "crowded")
+
+
+@pytest.mark.parametrize("dim,n", [(1, 3), (7, 64), (64, 65), (71, 200), (200, 129)])
+@pytest.mark.parametrize("mode", MODES)
+def test_build_tiles_match_oracle(gpu_ctx, mode, dim, n):
+    """The tiled index build at the edges of its 64 x 64 tiles: stored codes
+    byte-exact (serialized), a zero vector and one with an element past 1e19
+    (its float32 square overflows) among them."""
+    from semantica_gpu import search
+    rng = np.random.default_rng(dim + n + mode)
+    vecs = rng.standard_normal((n, dim)).astype(np.float32)
+    vecs[1] = 0.0
+    vecs[2, 0] = 1e20
+    ids = rng.permutation(5 * n)[:n].astype(np.int32)
+    raw = search.Serializer().serialize(_build(gpu_ctx, ids, vecs, mode))
+    want = o.bf_quantize(o.bf_normalize(vecs), mode)
+    assert raw[20 + 4 * n:] == np.ascontiguousarray(want).tobytes()
