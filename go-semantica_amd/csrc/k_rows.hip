@@ -179,12 +179,16 @@ __device__ __forceinline__ void store_codes4(int8_t* p, const float (&c)[4]) {
 // One row per wave (4 rows per workgroup): the row's scale and reciprocal are
 // computed once, then the wave walks the row in coalesced float4 slots.  The
 // codes go to the block-major GEMM operand qb [cols/32][a_rows][32] (qb !=
-// null) or row-major to qi [rows][cols].
+// null) or row-major to qi [rows][cols]; the sequences' scales to seq_scale
+// [n_seq] when it is not null (the first workgroup writes them).
 __global__ __launch_bounds__(kThreads) void k_quantize(const float* __restrict__ x, int ldx, int rows, int cols,
                                                        const int32_t* __restrict__ row_seq,
                                                        const float* __restrict__ amax, int8_t* __restrict__ qb,
                                                        int a_rows, int8_t* __restrict__ qi,
-                                                       float* __restrict__ row_scale) {
+                                                       float* __restrict__ row_scale, int n_seq,
+                                                       float* __restrict__ seq_scale) {
+  if (seq_scale && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < n_seq; i += kThreads) seq_scale[i] = amax[i] == 0.0f ? 1.0f : amax[i] / 127.0f;
   const int row = blockIdx.x * (kThreads / SG_WAVE) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(kThreads) void k_quantize(const float* __restrict__
     scale = m / 127.0f;
     inv = 1.0f / scale;
   }
-  if (lane == 0) row_scale[row] = scale;
+  if (row_scale && lane == 0) row_scale[row] = scale;
   const float* xr = x + (int64_t)row * ldx;
   for (int c4 = lane; c4 < (cols >> 2); c4 += SG_WAVE) {
     const f32x4_t v = *reinterpret_cast<const f32x4_t*>(xr + 4 * c4);
@@ -283,13 +287,6 @@ __global__ __launch_bounds__(kThreads) void k_quantize_blocked(const float* __re
     for (int t = 0; t < 4; t++) cv[t] = sg_quant_code(v[c][t], inv);
     store_codes4(qr + (int64_t)c * a_rows * 32, cv);
   }
-}
-
-__global__ void k_seq_scales(const float* __restrict__ amax, int n, float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float m = amax[i];
-  out[i] = m == 0.0f ? 1.0f : m / 127.0f;
 }
 
 // --------------------------------------------------------------- RMSNorm --
@@ -626,22 +623,59 @@ __global__ __launch_bounds__(kThreads) void k_gelu_mul(float* __restrict__ g, in
 
 // Per-row max|x| folded into the row's sequence maximum (absMaxScalar,
 // quantize.go:80-90, over a whole sequence).
-__global__ __launch_bounds__(kThreads) void k_absmax_rows(const float* __restrict__ x, int ldx, int cols,
+// The sequences' max|x| into amax (zeroed before), a wave per kMaxRows rows with
+// the loads of 5 x 64 columns' float4s of all its rows in flight.  One atomic
+// per workgroup of one sequence: the sequences' maxima share a cache line and
+// its atomics go one after another, 13 ns each (one per row made 2048 rows of
+// 768 take 26 us, more than the quantization itself).
+constexpr int kMaxRows = 4, kMaxBatch = 5;
+__global__ __launch_bounds__(kThreads) void k_absmax_rows(const float* __restrict__ x, int rows, int cols,
                                                           const int32_t* __restrict__ row_seq,
                                                           float* __restrict__ amax) {
-  __shared__ float red[kThreads / SG_WAVE];
-  const float* xr = x + (int64_t)blockIdx.x * ldx;
-  float m = 0.0f;
-  for (int c = threadIdx.x; c < cols; c += kThreads) m = fmaxf(m, fabsf(xr[c]));
-  m = sg_wave_max(m);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float mm = red[0];
-    for (int i = 1; i < kThreads / SG_WAVE; i++) mm = fmaxf(mm, red[i]);
-    sg_atomic_max_nonneg(amax + row_seq[blockIdx.x], mm);
+  constexpr int kWaves = kThreads / SG_WAVE;
+  __shared__ float red[kWaves];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int b0 = blockIdx.x * kWaves * kMaxRows, last = min(b0 + kWaves * kMaxRows, rows) - 1;
+  const int r0 = b0 + wave * kMaxRows, n4 = cols >> 2;
+  float m[kMaxRows];
+#pragma unroll
+  for (int i = 0; i < kMaxRows; i++) m[i] = 0.0f;
+  if (r0 < rows) {
+    for (int c = lane; c < n4; c += kMaxBatch * SG_WAVE) {
+      f32x4_t v[kMaxBatch][kMaxRows];
+#pragma unroll
+      for (int b = 0; b < kMaxBatch; b++)
+#pragma unroll
+        for (int i = 0; i < kMaxRows; i++)  // past the last column or row: the last one again
+          v[b][i] = *reinterpret_cast<const f32x4_t*>(x + (int64_t)min(r0 + i, rows - 1) * cols +
+                                                      4 * min(c + b * SG_WAVE, n4 - 1));
+#pragma unroll
+      for (int b = 0; b < kMaxBatch; b++)
+#pragma unroll
+        for (int i = 0; i < kMaxRows; i++)
+#pragma unroll
+          for (int t = 0; t < 4; t++) m[i] = fmaxf(m[i], fabsf(v[b][i][t]));
+    }
+  }
+  if (row_seq[b0] == row_seq[last]) {  // the whole workgroup (uniform)
+    const float w = sg_wave_max(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
+    if (lane == 0) red[wave] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      float mm = red[0];
+#pragma unroll
+      for (int i = 1; i < kWaves; i++) mm = fmaxf(mm, red[i]);
+      sg_atomic_max_nonneg(amax + row_seq[b0], mm);
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < kMaxRows; i++) {
+    const float w = sg_wave_max(m[i]);
+    if (lane == 0 && r0 + i < rows) sg_atomic_max_nonneg(amax + row_seq[r0 + i], w);
   }
 }
+static_assert(kMaxRows == 4, "the workgroup's fold");
 
 // ---------------------------------------------------------- pool and L2 --
 
@@ -847,7 +881,7 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
     }
   }
   hipLaunchKernelGGL(k_quantize, dim3(blocks_for(rows, kThreads / SG_WAVE)), dim3(kThreads), 0, s, x, ldx, rows, cols,
-                     row_seq, amax, q8, a_rows, q8 ? nullptr : i8, row_scale);
+                     row_seq, amax, q8, a_rows, q8 ? nullptr : i8, row_scale, 0, nullptr);
   return hipGetLastError();
 }
 
@@ -866,11 +900,6 @@ hipError_t norm_quantize(const float* h, const float* w, float eps, int T, int d
   SG_DISPATCH_NPL(d, NPL,
                   hipLaunchKernelGGL(k_norm_quantize<NPL / 4>, dim3(blocks_for(T, kRowsPerBlock)), dim3(kThreads), 0,
                                      s, h, w, eps, T, row_seq, amax, q8, a_rows, row_scale));
-  return hipGetLastError();
-}
-
-hipError_t seq_scales(const float* amax, int n_seq, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_seq_scales, dim3(blocks_for(n_seq, 256)), dim3(256), 0, s, amax, n_seq, out);
   return hipGetLastError();
 }
 
@@ -943,10 +972,15 @@ hipError_t stream_probe(int kind, const float* a, const float* b, void* c, int64
   return hipGetLastError();
 }
 
-hipError_t absmax_rows(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, float* amax,
-                       hipStream_t s) {
-  if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_absmax_rows, dim3(rows), dim3(kThreads), 0, s, x, ldx, cols, row_seq, amax);
+hipError_t quantize_seqs(const float* x, int rows, int cols, const int32_t* row_seq, int n_seq, float* amax, int8_t* q,
+                         float* seq_scale, hipStream_t s) {
+  if (rows < 0 || cols <= 0 || cols % 4 || n_seq <= 0) return hipErrorInvalidValue;
+  if (rows > 0)
+    hipLaunchKernelGGL(k_absmax_rows, dim3(blocks_for(rows, kThreads / SG_WAVE * kMaxRows)), dim3(kThreads), 0, s, x,
+                       rows, cols, row_seq, amax);
+  // (rows == 0: the scales of the empty sequences)
+  hipLaunchKernelGGL(k_quantize, dim3(rows > 0 ? blocks_for(rows, kThreads / SG_WAVE) : 1), dim3(kThreads), 0, s, x, cols, rows, cols,
+                     row_seq, amax, nullptr, 0, q, nullptr, n_seq, seq_scale);
   return hipGetLastError();
 }
 

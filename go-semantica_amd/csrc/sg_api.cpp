@@ -1101,15 +1101,18 @@ int sg_quantize_act(sg_ctx* ctx, const float* x, int32_t rows, int32_t cols, con
   std::lock_guard<std::mutex> lk(ctx->mu);
   SG_TRY(set_device(ctx));
   hipStream_t s = pick(ctx, stream);
-  Meta meta;
-  SG_TRY(stage_meta(off, n_seq, 1, ctx->meta_h, ctx->meta_d, s, meta));
-  SG_TRY(ctx->amax.ensure(sizeof(float) * ((size_t)n_seq + (size_t)rows)));
-  float* amax = ctx->amax.as<float>();
-  float* row_scale = amax + n_seq;
-  SG_HIP(sgk::fill_f32(amax, 0.0f, n_seq, s));
-  SG_HIP(sgk::absmax_rows(x, cols, rows, cols, meta.row_seq, amax, s));
-  SG_HIP(sgk::quantize(x, cols, rows, cols, meta.row_seq, amax, nullptr, 0, q_out, row_scale, s));
-  SG_HIP(sgk::seq_scales(amax, n_seq, scale_out, s));
+  // [row_seq | a zero per sequence], one copy: the maxima need no fill launch.
+  const size_t bytes = sizeof(int32_t) * ((size_t)rows + (size_t)n_seq);
+  SG_TRY(ctx->meta_h.ensure(bytes));
+  SG_TRY(ctx->meta_d.ensure(bytes));
+  int32_t* rs = ctx->meta_h.as<int32_t>();
+  for (int i = 0; i < n_seq; i++) std::fill(rs + off[i], rs + off[i + 1], i);
+  std::fill(rs + rows, rs + rows + n_seq, 0);
+  SG_HIP(hipMemcpyAsync(ctx->meta_d.p, rs, bytes, hipMemcpyHostToDevice, s));
+  SG_TRY(ctx->meta_h.record(s));
+  int32_t* row_seq = ctx->meta_d.as<int32_t>();
+  SG_HIP(sgk::quantize_seqs(x, rows, cols, row_seq, n_seq, reinterpret_cast<float*>(row_seq + rows), q_out, scale_out,
+                            s));
   SG_HIP(hipStreamSynchronize(s));
   return SG_OK;
 }

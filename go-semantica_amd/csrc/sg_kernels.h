@@ -96,9 +96,11 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
 hipError_t norm_quantize(const float* h, const float* w, float eps, int T, int d, const int32_t* row_seq,
                          const float* amax, int8_t* q8, int a_rows, float* row_scale, hipStream_t s,
                          const float* rmax = nullptr, const int32_t* seq_off = nullptr);
-hipError_t absmax_rows(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, float* amax,
-                       hipStream_t s);
-hipError_t seq_scales(const float* amax, int n_seq, float* out, hipStream_t s);
+// Per-sequence symmetric quantization of x[rows][cols] from scratch: codes
+// row-major q[rows][cols], scales seq_scale[n_seq].  amax [n_seq]: zeros on
+// entry, the sequences' max|x| on return.
+hipError_t quantize_seqs(const float* x, int rows, int cols, const int32_t* row_seq, int n_seq, float* amax, int8_t* q,
+                         float* seq_scale, hipStream_t s);
 // RMSNorm rows in the reference's order; amax (optional) collects per-sequence max|y|.
 hipError_t rmsnorm(float* dst, const float* src, const float* w, int rows, int n, float eps,
                    const int32_t* row_seq, float* amax, hipStream_t s);

@@ -374,6 +374,32 @@ def test_quantize_per_sequence_bit_exact(gpu_ctx, oracle, cols):
         assert np.array_equal(qg[off[i]:off[i + 1]], qo), i
 
 
+@pytest.mark.parametrize("lens", [[1], [15], [16], [17, 0], [8, 8, 1], [63, 65, 64]])
+@pytest.mark.parametrize("cols", [4, 256, 1276, 1284, 2564])
+def test_quantize_maxima_edges(gpu_ctx, oracle, lens, cols):
+    """Row and column remainders of the maxima's workgroups (16 rows, 1280
+    columns), the sequence's largest value in its last row and column."""
+    import torch
+    from semantica_gpu import kernels
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    say(f"quantize maxima lens={lens} cols={cols}")
+    x = np.random.default_rng(cols).standard_normal((int(off[-1]), cols)).astype(np.float32)
+    for i, n in enumerate(lens):
+        if n:
+            x[off[i + 1] - 1, cols - 1] = -10.0 - i
+    q = torch.empty(x.shape, dtype=torch.int8, device="cuda")
+    sc = torch.empty(len(lens), dtype=torch.float32, device="cuda")
+    kernels.quantize_symmetric_int8(gpu_ctx, dev(x), off, q, sc)
+    qg, sg = host(q), host(sc)
+    for i, n in enumerate(lens):
+        if n == 0:
+            assert sg[i] == 1.0
+            continue
+        qo, so = oracle.quantize(x[off[i]:off[i + 1]])
+        assert sg[i] == so, i
+        assert np.array_equal(qg[off[i]:off[i + 1]], qo), i
+
+
 def _near_ties(m):
     """Values x (|x| < m) whose float32 product with the kernel's inv =
     1/(m/127) lands exactly on k + 1/2, while the exact product (what the
