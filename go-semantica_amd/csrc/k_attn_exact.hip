@@ -30,7 +30,6 @@ namespace {
 constexpr int kXT = 64;     // query rows and key rows per score tile
 constexpr int kXD = 32;     // head dims staged in LDS per step (four 8-lane steps)
 constexpr int kXHd = 256;   // head_dim
-constexpr int kXRows = 32;  // query rows per P.V workgroup
 constexpr int kXKeys = 64;  // keys per P.V LDS stage
 
 // One 64 x 64 tile of one (sequence, head): 256 threads, thread (tx, ty) the
@@ -230,83 +229,126 @@ __global__ __launch_bounds__(256) void k_exact_softmax(float* __restrict__ P, in
   }
 }
 
-// out[r][h*256 + d] for 32 query rows of one (sequence, head): thread d, one
-// chain per row over the keys in order.  The weights of 64 keys are staged in
-// LDS per step; V's row j is one coalesced 1-KB read shared by the 32 rows.
-__global__ __launch_bounds__(256) void k_exact_pv(const float* __restrict__ P, int ldp, const float* __restrict__ v,
-                                                  int ldv, const int32_t* __restrict__ seq_off, int H, int group,
-                                                  float* __restrict__ out, int ldo, int T, float* __restrict__ amax) {
+// out[r][h*256 + d]: a wave takes kPvRows query rows of one (sequence, head) and
+// all 256 dims, four consecutive dims per lane, one chain per (row, dim) over
+// the keys in order.  The wave stages its rows' weights of 64 keys in an LDS
+// slice of its own (the next 64 in flight meanwhile, no workgroup barrier) and
+// reads them by broadcast; V's row j is one coalesced 1-KB read, 8 keys' rows in
+// flight under the 8 before.  Bound by the VALU (a multiplication and an
+// addition per row, dim and key, which the reference rounds separately): one
+// broadcast read of 4 weights serves 32 of these instructions.  (With a
+// dim per lane and 32 rows it served 8, and every 4 keys waited for V: 132 us
+// for 20 sequences of 32 to 400 tokens, 74 us now.)
+constexpr int kPvRows = 8, kPvWaves = 2, kPvKeys = 8;
+
+// The keys of one (sequence, head), in order, for a wave's rows.  SKIP: the
+// reference's skip of keys of weight 0 (attention.go:344-363).
+template <bool SKIP>
+__device__ __forceinline__ void pv_rows(const float* __restrict__ prow, int ldp, int rows, const float* __restrict__ vp,
+                                        int ldv, int S, float (*__restrict__ ps)[kXKeys], int lane,
+                                        f32x4_t (&acc)[kPvRows]) {
+#pragma unroll
+  for (int i = 0; i < kPvRows; i++) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float w[kPvRows];
+  auto weights = [&](int j0) {  // rows past `rows` repeat the last one
+    const int j = min(j0 + lane, S - 1);
+#pragma unroll
+    for (int i = 0; i < kPvRows; i++) w[i] = prow[(int64_t)min(i, rows - 1) * ldp + j];
+  };
+  f32x4_t cur[kPvKeys], nxt[kPvKeys];
+  auto values = [&](f32x4_t (&r)[kPvKeys], int j) {  // keys past the end: the last one's (their weight is 0)
+#pragma unroll
+    for (int u = 0; u < kPvKeys; u++) {
+      const float* vr = vp + (int64_t)min(j + u, S - 1) * ldv;
+      r[u] = f32x4_t{vr[0], vr[1], vr[2], vr[3]};
+    }
+  };
+  f32x4_t pw[2][kPvRows];  // four keys' weights, the next four's being read
+  auto quad = [&](f32x4_t (&r)[kPvRows], int jb) {
+#pragma unroll
+    for (int i = 0; i < kPvRows; i++) r[i] = *reinterpret_cast<const f32x4_t*>(&ps[i][jb]);
+  };
+  weights(0);
+  values(cur, 0);
+  for (int j0 = 0; j0 < S; j0 += kXKeys) {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < kPvRows; i++) ps[i][lane] = j0 + lane < S ? w[i] : 0.0f;
+    __builtin_amdgcn_wave_barrier();
+    weights(j0 + kXKeys);
+    const int nk = min(kXKeys, S - j0);
+    quad(pw[0], 0);
+    for (int jb = 0; jb < nk; jb += kPvKeys) {
+      values(nxt, j0 + jb + kPvKeys);
+#pragma unroll
+      for (int g = 0; g < kPvKeys / 4; g++) {
+        quad(pw[(g + 1) & 1], min(jb + 4 * (g + 1), kXKeys - 4));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kPvRows; i++)
+#pragma unroll
+          for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+              const float p = cur[4 * g + u][t] * pw[g & 1][i][u];  // VecScaleF32: one rounding
+              if (!SKIP || pw[g & 1][i][u] != 0.0f) acc[i][t] = acc[i][t] + p;  // VecAddF32
+            }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int u = 0; u < kPvKeys; u++) cur[u] = nxt[u];
+    }
+  }
+}
+
+__global__ __launch_bounds__(kPvWaves * 64) void k_exact_pv(const float* __restrict__ P, int ldp,
+                                                            const float* __restrict__ v, int ldv,
+                                                            const int32_t* __restrict__ seq_off, int H, int group,
+                                                            float* __restrict__ out, int ldo, int T,
+                                                            float* __restrict__ amax) {
   const int s = blockIdx.y / H, h = blockIdx.y % H;
   const int r0 = seq_off[s], S = seq_off[s + 1] - r0;
-  const int i0 = blockIdx.x * kXRows;
-  if (i0 >= S) return;  // uniform, before any barrier
-  const int kvh = h / group, d = threadIdx.x;
-  __shared__ __attribute__((aligned(16))) float ps[kXRows][kXKeys];
-  float acc[kXRows];
+  if ((int)blockIdx.x * kPvWaves * kPvRows >= S) return;  // uniform, before any barrier
+  __shared__ __attribute__((aligned(16))) float ps[kPvWaves][kPvRows][kXKeys];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i0 = (blockIdx.x * kPvWaves + wave) * kPvRows, rows = min(kPvRows, S - i0);
+  float m = 0.0f;
+  if (rows > 0) {
+    const float* prow = P + ((int64_t)h * T + r0 + i0) * ldp;
+    const float* vp = v + (int64_t)r0 * ldv + (h / group) * kXHd + 4 * lane;
+    f32x4_t acc[kPvRows];
+    pv_rows<false>(prow, ldp, rows, vp, ldv, S, ps[wave], lane, acc);
+    // The reference skips keys of weight 0.  With v finite that changes nothing:
+    // the product is +-0, and o + (+-0) = o, since o starts at +0 and a sum is -0
+    // only when both terms are.  An infinite or NaN product leaves o infinite or
+    // NaN for good, so only then the rows are summed again with the skip.
+    bool finite = true;
 #pragma unroll
-  for (int i = 0; i < kXRows; i++) acc[i] = 0.0f;
-  const float* vcol = v + (int64_t)r0 * ldv + kvh * kXHd + d;
-  for (int j0 = 0; j0 < S; j0 += kXKeys) {
-    // 32 rows x 64 keys of weights (zeros past the sequence's rows or keys)
+    for (int i = 0; i < kPvRows; i++)
 #pragma unroll
-    for (int e = threadIdx.x; e < kXRows * kXKeys; e += 256) {
-      const int i = e / kXKeys, jj = e % kXKeys;
-      float pv = 0.0f;
-      if (i0 + i < S && j0 + jj < S) pv = P[((int64_t)h * T + r0 + i0 + i) * ldp + j0 + jj];
-      ps[i][jj] = pv;
-    }
-    __syncthreads();
-    const int nk = min(kXKeys, S - j0);
-    // Keys in batches of 4: their V loads go out together, and each row's 4
-    // weights are one LDS read.  Keys past nk carry weight 0 in ps and a
-    // clamped (in-range) V row, so they take the skip like any zero weight.
-    for (int jb = 0; jb < nk; jb += 4) {
-      float vj[4];
+      for (int t = 0; t < 4; t++) finite = finite && __builtin_isfinite(acc[i][t]);
+    if (__ballot(!finite)) pv_rows<true>(prow, ldp, rows, vp, ldv, S, ps[wave], lane, acc);
+    float* o = out + (int64_t)(r0 + i0) * ldo + h * kXHd + 4 * lane;
 #pragma unroll
-      for (int u = 0; u < 4; u++) vj[u] = vcol[(int64_t)(j0 + min(jb + u, nk - 1)) * ldv];
-      // The reference skips keys of weight 0.  With v finite that changes
-      // nothing: the product is +-0, and o + (+-0) = o, since o starts at +0 and
-      // a sum is -0 only when both terms are.  So the skip is taken only when
-      // this wave's values of the batch include an infinity or a NaN.
-      const bool finite = __builtin_isfinite(vj[0]) && __builtin_isfinite(vj[1]) && __builtin_isfinite(vj[2]) &&
-                          __builtin_isfinite(vj[3]);
-      if (__ballot(!finite) == 0 && jb + 4 <= nk) {
+    for (int i = 0; i < kPvRows; i++)
+      if (i < rows) {
 #pragma unroll
-        for (int i = 0; i < kXRows; i++) {
-          const f32x4_t pw = *reinterpret_cast<const f32x4_t*>(&ps[i][jb]);
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const float t = vj[u] * pw[u];  // VecScaleF32: one rounding
-            acc[i] = acc[i] + t;            // VecAddF32
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < kXRows; i++) {
-          const f32x4_t pw = *reinterpret_cast<const f32x4_t*>(&ps[i][jb]);
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            const float t = vj[u] * pw[u];
-            if (pw[u] != 0.0f) acc[i] = acc[i] + t;
-          }
+        for (int t = 0; t < 4; t++) {
+          o[(int64_t)i * ldo + t] = acc[i][t];
+          m = fmaxf(m, fabsf(acc[i][t]));
         }
       }
-    }
-    __syncthreads();
   }
-  float m = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kXRows; i++)
-    if (i0 + i < S) {
-      out[(int64_t)(r0 + i0 + i) * ldo + h * kXHd + d] = acc[i];
-      m = fmaxf(m, fabsf(acc[i]));
-    }
   if (amax) {  // the sequence's max|o| for the quantizer: one atomic per workgroup
-    __shared__ float red[4];
+    __shared__ float red[kPvWaves];
     m = sg_wave_max(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    if (lane == 0) red[wave] = m;
     __syncthreads();
-    if (threadIdx.x == 0) sg_atomic_max_nonneg(amax + s, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int i = 1; i < kPvWaves; i++) m = fmaxf(m, red[i]);
+      sg_atomic_max_nonneg(amax + s, m);
+    }
   }
 }
 
@@ -339,7 +381,7 @@ hipError_t attention_exact(const float* q, int ldq, const float* k, const float*
                      T, H);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_exact_pv, dim3(ceil_div(max_len, kXRows), n_seq * H), dim3(256), 0, s, P, ldp, v, ldkv,
+  hipLaunchKernelGGL(k_exact_pv, dim3(ceil_div(max_len, kPvWaves * kPvRows), n_seq * H), dim3(kPvWaves * 64), 0, s, P, ldp, v, ldkv,
                      seq_off, H, group, out, ldo, T, amax);
   return hipGetLastError();
 }
