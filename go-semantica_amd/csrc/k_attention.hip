@@ -231,27 +231,35 @@ static_assert(kScoreBytes == kWaves * 2048, "spill tile layout");
 // A tile's LDS stage is its 32 KB of fragments as they lie in memory, so a copy
 // is 1 KB to 1 KB and a fragment read is the wave's lanes in order (no bank
 // conflicts, an immediate offset per fragment).
-template <bool QPRE, bool SPILL>
-__global__ __launch_bounds__(kNT, 2) void k_attn_rs(
-    const _Float16* __restrict__ qf, const _Float16* __restrict__ kf, const _Float16* __restrict__ vf, int n_tiles, float* __restrict__ out, int ldo,
-    const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff, const sg_item* __restrict__ items,
-    int G, float sscale, float* __restrict__ amax, sg_attn_qpre qp, sg_attn_qout qo, sg_attn_spill sp) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kRing * kTileBytes];
-  __shared__ __attribute__((aligned(16))) unsigned char slds[SPILL ? kRing * kScoreBytes : 16];
-  __shared__ float red[kWaves];
+//
+// Split items.  A launch of fewer workgroups than CUs takes as long as its
+// longest sequence's; `n_split` of its items (the first ones: the longest) then
+// run as two workgroups of four chunks, a wave per SIMD each, and take 0.8 of
+// an item's time (one K or V stream for half of the MFMAs, nothing to overlap a
+// wave's softmax with).  us per launch, unsplit / split: 6 x 512 tokens 50 / 40,
+// 5 x 1024 95 / 77, 2 x 2048 175 / 134, 40 x 128 20 / 17; more than 256 workgroups
+// of halves lose (16 x 512: 55 / 77), so only as many items are split as there
+// are idle CUs.
+template <bool QPRE, bool SPILL, int W>
+__device__ __forceinline__ void attn_rs_item(
+    unsigned char* lds, unsigned char* slds, float* red, const sg_item& it, int half,
+    const _Float16* __restrict__ qf, const _Float16* __restrict__ kf, const _Float16* __restrict__ vf, int n_tiles,
+    float* __restrict__ out, int ldo, const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff, int G,
+    float sscale, float* __restrict__ amax, const sg_attn_qpre& qp, const sg_attn_qout& qo, const sg_attn_spill& sp) {
   typedef __attribute__((address_space(3))) void* lds_ptr;
 
-  const sg_item it = items[blockIdx.x];
   const int kvh = blockIdx.y;
   const int r0 = seq_off[it.seq];
   const int S = seq_off[it.seq + 1] - r0;
   const int vo = voff[it.seq];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6) & (kWaves - 1);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6) & (W - 1);
+  const int wi = half * W + w;  // the wave's chunk of the item
   const int ln = lane & 15, g4 = lane >> 4;
   const int nqb = (S + kQW - 1) / kQW;
   const int nt = (S + kBK - 1) / kBK;  // <= kRegTiles unless SPILL (the host checks the longest sequence)
-  const int c = it.c0 + w;
+  if (W != kWaves && it.c0 + half * W >= G * nqb) return;  // workgroup-uniform, before any barrier
+  const int c = it.c0 + wi;
   const bool active = c < G * nqb;  // wave-uniform
   const int hg = active ? c / nqb : 0;
   const int q0 = active ? (c % nqb) * kQW : 0;
@@ -261,16 +269,17 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
   const int qr = r0 + min(qrow, S - 1);
 
   // ---- copies ----
-  // Wave w's four copies of an item: pieces 4w .. 4w + 3 of the tile.  Keys past
+  // Wave w's kCopies copies of an item: pieces kCopies * w .. of the tile.  Keys past
   // the sequence's end hold whatever the buffer held; their scores are masked
   // below (V's pad keys are zeros).
   const int64_t tile0 = (int64_t)kvh * n_tiles + (vo >> 5);
   const i32x4_t rk = sg_raw_rsrc(kf + tile0 * sgd::kFragTile);
   const i32x4_t rv = sg_raw_rsrc(vf + tile0 * sgd::kFragTile);
+  constexpr int kCopies = 32 / W;
   auto copy_tile = [&](uint32_t dst, bool isk, int tile) {
-    const uint32_t soff = (uint32_t)tile * kTileBytes + (uint32_t)w * 4096u;
+    const uint32_t soff = (uint32_t)tile * kTileBytes + (uint32_t)w * (kCopies * 1024u);
 #pragma unroll
-    for (int i = 0; i < 4; i++) sg_lds_copy16(dst + 1024u * i, 16u * lane, isk ? rk : rv, soff + 1024u * i);
+    for (int i = 0; i < kCopies; i++) sg_lds_copy16(dst + 1024u * i, 16u * lane, isk ? rk : rv, soff + 1024u * i);
   };
   // SPILL: this workgroup's spilled scores, nt - kRegTiles tiles of
   // kScoreBytes (wave w's 2 KB at w * 2048: lane l's keys 4g4 + r at 16 l,
@@ -287,32 +296,32 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
   auto carries = [&](int src) { return SPILL && src >= nt + kRegTiles - 1 && src < last; };
   auto issue = [&](int item) {
     const int src = item < last ? item : last;
-    const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr)(lds + ((unsigned)item % kRing) * kTileBytes + w * 4096);
+    const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr)(lds + ((unsigned)item % kRing) * kTileBytes + w * (kCopies * 1024));
     copy_tile(dst, src < nt, src < nt ? src : src - nt);
     if (carries(src)) {
-      const uint32_t sd = (uint32_t)(uintptr_t)(lds_ptr)(slds + ((unsigned)item % kRing) * kScoreBytes + w * 2048);
-      const uint32_t so = (uint32_t)((src - nt + 1 - kRegTiles) * kScoreBytes + w * 2048);
+      const uint32_t sd = (uint32_t)(uintptr_t)(lds_ptr)(slds + ((unsigned)item % kRing) * (W * 2048) + w * 2048);
+      const uint32_t so = (uint32_t)((src - nt + 1 - kRegTiles) * kScoreBytes + wi * 2048);
       sg_lds_copy16(sd, 16u * lane, rsp, so);
       sg_lds_copy16(sd + 1024u, 16u * lane + 1024u, rsp, so);
     }
   };
-  // Wait until item i has landed, item i + 1 (4 copies per wave, or 6 when it
-  // carries scores) may still be in flight.
+  // Wait until item i has landed, item i + 1 (kCopies copies per wave, or two more
+  // when it carries scores) may still be in flight.
   auto wait_item = [&](int i) {
     if (carries(i + 1 < last ? i + 1 : last))
-      sg_wait_vmcnt<6>();
+      sg_wait_vmcnt<kCopies + 2>();
     else
-      sg_wait_vmcnt<4>();
+      sg_wait_vmcnt<kCopies>();
   };
   issue(0);
   issue(1);
   half8_t bqh[kHD / 32], bql[kHD / 32];
   // The Q prologue's LDS tiles sit in stage 2, which no copy touches before
   // the first barrier.
-  static_assert(kWaves * (16 * 40 + kHD) * 4 <= kTileBytes, "prologue tiles fit stage 2");
+  static_assert(W * (16 * 40 + kHD) * 4 <= kTileBytes, "prologue tiles fit stage 2");
   q_operand<QPRE>(bqh, bql, QPRE ? nullptr : qf + q_subtile(head, n_tiles, vo, q0), qp, qr, qr - r0, head, ln, g4, lane,
                   reinterpret_cast<float*>(lds + 2 * kTileBytes) + w * (16 * 40),
-                  reinterpret_cast<float*>(lds + 2 * kTileBytes) + kWaves * (16 * 40) + w * kHD);
+                  reinterpret_cast<float*>(lds + 2 * kTileBytes) + W * (16 * 40) + w * kHD);
 
   auto key_of = [&](int kt, int st, int r) { return kt + 16 * st + 4 * g4 + r; };
   // ---- pass 1: S^T = K Q^T per tile, kept in registers; row max ----
@@ -403,7 +412,7 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
           m = fmaxf(m, fmaxf(s0[r], s1[r]));
         }
       }
-      float* sp = wspill + (size_t)(t - kRegTiles) * (kScoreBytes / 4) + w * 512 + 4 * lane;
+      float* sp = wspill + (size_t)(t - kRegTiles) * (kScoreBytes / 4) + wi * 512 + 4 * lane;
       *reinterpret_cast<f32x4_t*>(sp) = s0;
       *reinterpret_cast<f32x4_t*>(sp + 256) = s1;
     }
@@ -472,7 +481,7 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
     // Tile t's scores landed with item nt + t - 1 (published by its barrier);
     // the stage is overwritten only after the next barrier.
     for (int t = kRegTiles; t < nt; t++) {
-      const unsigned char* sb = slds + ((unsigned)(nt + t - 1) % kRing) * kScoreBytes + w * 2048 + 16 * lane;
+      const unsigned char* sb = slds + ((unsigned)(nt + t - 1) % kRing) * (W * 2048) + w * 2048 + 16 * lane;
       tile2(*reinterpret_cast<const f32x4_t*>(sb), *reinterpret_cast<const f32x4_t*>(sb + 1024), t);
     }
   }
@@ -503,7 +512,7 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
     if (tid == 0) {
       float mm = red[0];
 #pragma unroll
-      for (int i = 1; i < kWaves; i++) mm = fmaxf(mm, red[i]);
+      for (int i = 1; i < W; i++) mm = fmaxf(mm, red[i]);
       sg_atomic_max_nonneg(amax + it.seq, mm);
     }
     // The workgroup holds the whole sequence (every row of every head; the
@@ -515,7 +524,7 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
     if (qo.q8 && qvalid) {
       float mm = red[0];
 #pragma unroll
-      for (int i = 1; i < kWaves; i++) mm = fmaxf(mm, red[i]);
+      for (int i = 1; i < W; i++) mm = fmaxf(mm, red[i]);
       float scale = 1.0f, inv = 0.0f;
       if (mm != 0.0f) {
         scale = mm / 127.0f;
@@ -533,6 +542,28 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_rs(
         *reinterpret_cast<uint32_t*>(qo.q8 + ((int64_t)(col >> 5) * qo.a_rows + row) * 32 + (col & 31)) = u;
       }
     }
+  }
+}
+
+template <bool QPRE, bool SPILL>
+__global__ __launch_bounds__(kNT, 2) void k_attn_rs(
+    const _Float16* __restrict__ qf, const _Float16* __restrict__ kf, const _Float16* __restrict__ vf, int n_tiles,
+    float* __restrict__ out, int ldo, const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff,
+    const sg_item* __restrict__ items, int n_items, int n_split, int G, float sscale, float* __restrict__ amax,
+    sg_attn_qpre qp, sg_attn_qout qo, sg_attn_spill sp) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kRing * kTileBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char slds[SPILL ? kRing * kScoreBytes : 16];
+  __shared__ float red[kWaves];
+  const int b = blockIdx.x;
+  if (b < 2 * n_split) {  // n_split is a multiple of 8: the halves of an item on one XCD, like the items
+    const int at = (b >> 4) * 8 + (b & 7);
+    // Four waves stay (the others' end counts at barriers).
+    if (at >= n_items || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= kWaves / 2) return;
+    attn_rs_item<QPRE, SPILL, kWaves / 2>(lds, slds, red, items[at], (b >> 3) & 1, qf, kf, vf, n_tiles, out, ldo,
+                                          seq_off, voff, G, sscale, amax, qp, qo, sp);
+  } else {
+    attn_rs_item<QPRE, SPILL, kWaves>(lds, slds, red, items[b - n_split], 0, qf, kf, vf, n_tiles, out, ldo, seq_off,
+                                      voff, G, sscale, amax, qp, qo, sp);
   }
 }
 
@@ -925,11 +956,14 @@ void launch_small(int n_items, int HKV, hipStream_t s, const _Float16* qf, const
 }
 
 template <bool QPRE, bool SPILL>
-void launch_attn(dim3 grid, hipStream_t s, const _Float16* qf, const _Float16* kf,
-                 const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off, const int32_t* voff, const sg_item* items, int G, float sscale, float* amax,
-                 const sg_attn_qpre& qp, const sg_attn_qout& qo, const sg_attn_spill& sp) {
-  hipLaunchKernelGGL((k_attn_rs<QPRE, SPILL>), grid, dim3(kNT), 0, s, qf, kf, vf, n_tiles, out, ldo, seq_off,
-                     voff, items, G, sscale, amax, qp, qo, sp);
+void launch_attn(int n_items, int HKV, int n_split, hipStream_t s, const _Float16* qf, const _Float16* kf,
+                 const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off, const int32_t* voff,
+                 const sg_item* items, int G, float sscale, float* amax, const sg_attn_qpre& qp, const sg_attn_qout& qo,
+                 const sg_attn_spill& sp) {
+  n_split = (n_split + 7) & ~7;  // past n_items: empty workgroups
+  const int nwg = 2 * n_split + (n_items > n_split ? n_items - n_split : 0);
+  hipLaunchKernelGGL((k_attn_rs<QPRE, SPILL>), dim3(nwg, HKV), dim3(kNT), 0, s, qf, kf, vf, n_tiles, out, ldo, seq_off,
+                     voff, items, n_items, n_split, G, sscale, amax, qp, qo, sp);
 }
 }  // namespace
 
@@ -958,8 +992,9 @@ hipError_t attention_small(const _Float16* qf, const _Float16* kf, const _Float1
 hipError_t attention(const _Float16* qf, const _Float16* kf, const _Float16* vf, int n_tiles,
                      float* out, int ldo, const int32_t* seq_off, const int32_t* voff, const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
                      float* amax, int max_len, hipStream_t s, const sg_attn_qpre* qpre,
-                     const sg_attn_qout* qout, const sg_attn_spill* spill) {
+                     const sg_attn_qout* qout, const sg_attn_spill* spill, int n_split) {
   if (n_items <= 0) return hipSuccess;
+  if (n_split < 0 || n_split > n_items) return hipErrorInvalidValue;
   if (hd != kHD || HKV <= 0 || H % HKV || max_len <= 0) return hipErrorInvalidValue;
   // The quantizing epilogue needs the register-scores kernel, one workgroup per
   // sequence (one kv head, every chunk of the sequence in one item) and amax.
@@ -975,7 +1010,6 @@ hipError_t attention(const _Float16* qf, const _Float16* kf, const _Float16* vf,
     return hipErrorInvalidValue;
   const sg_attn_spill sp = spills ? *spill : sg_attn_spill{nullptr, nullptr, 0};
   const float sscale = scale / (kQKScale * kQKScale);
-  const dim3 grid(n_items, HKV);
   sg_attn_qpre qp{};
   if (qpre) {
     if (!qpre->q || !qpre->cos_t || !qpre->sin_t || (qpre->ldq & 3) ||
@@ -986,11 +1020,13 @@ hipError_t attention(const _Float16* qf, const _Float16* kf, const _Float16* vf,
   } else if (!qf) {
     return hipErrorInvalidValue;
   }
-  using fn = void (*)(dim3, hipStream_t, const _Float16*, const _Float16*, const _Float16*, int, float*, int, const int32_t*, const int32_t*, const sg_item*, int, float,
-                      float*, const sg_attn_qpre&, const sg_attn_qout&, const sg_attn_spill&);
+  using fn = void (*)(int, int, int, hipStream_t, const _Float16*, const _Float16*, const _Float16*, int, float*, int,
+                      const int32_t*, const int32_t*, const sg_item*, int, float, float*, const sg_attn_qpre&,
+                      const sg_attn_qout&, const sg_attn_spill&);
   static const fn table[2][2] = {{launch_attn<false, false>, launch_attn<false, true>},
                                  {launch_attn<true, false>, launch_attn<true, true>}};
-  table[qpre != nullptr][spills](grid, s, qf, kf, vf, n_tiles, out, ldo, seq_off, voff, items, H / HKV,
+  if (qout) n_split = 0;  // one workgroup per sequence
+  table[qpre != nullptr][spills](n_items, HKV, n_split, s, qf, kf, vf, n_tiles, out, ldo, seq_off, voff, items, H / HKV,
                                  sscale, amax, qp, qo, sp);
   return hipGetLastError();
 }

@@ -74,6 +74,7 @@ struct Meta {
   sg_item* vtiles = nullptr; // V^T split tiles (sequence, first key)
   int32_t* spill_off = nullptr;  // [n_seq] first attention spill tile of each sequence
   int spill_total = 0;           // attention spill tiles per kv head
+  int n_split = 0;               // attention items to run as two workgroups (one kv head, alone on the GPU)
 };
 
 // Attention workgroups of one sequence: G*ceil(S/16) chunks, kAttnChunks each.
@@ -95,6 +96,7 @@ int seq_groups(int S, int G) {
 // the list interleaves the bins: all workgroups of a sequence then share one
 // L2 copy of its K and V^T.
 constexpr int kAttnLptItems = 512;  // two rounds of attention workgroups on 256 CUs
+constexpr int kAttnCus = 256;
 
 int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev, hipStream_t s, Meta& m) {
   constexpr int kXcd = 8;
@@ -170,6 +172,17 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
       std::stable_sort(it, it + n_items, [&](const sg_item& a, const sg_item& b) {
         return off[a.seq + 1] - off[a.seq] > off[b.seq + 1] - off[b.seq];
       });
+  }
+  // Idle CUs take half of the longest items (k_attn_rs, "split items").  With
+  // too few of them for every item, the longest one left whole sets the time:
+  // no split unless it is a tenth shorter than the longest.
+  m.n_split = 0;
+  if (2 * n_items <= kAttnCus) {
+    m.n_split = n_items;
+  } else if (n_items < kAttnCus) {
+    const int sp8 = (kAttnCus - n_items) & ~7;
+    auto len = [&](int i) { return off[it[i].seq + 1] - off[it[i].seq]; };
+    if (sp8 > 0 && 10 * len(sp8) <= 9 * len(0)) m.n_split = sp8;
   }
   SG_HIP(hipMemcpyAsync(dev.p, host.p, bytes, hipMemcpyHostToDevice, s));
   SG_TRY(host.record(s));
@@ -514,9 +527,10 @@ bool attn_small(const sg_model* m, const Meta& meta) {
 // embedding first when l0 == 0, the pooled embeddings into d_out after the
 // last layer.  stop >= 0: return after `stop` layers with the residual stream
 // copied to d_out (when non-null).  tr: per-layer copies of the first `stop`
-// layers.
+// layers.  alone: no other group's kernels run beside these (idle CUs stay
+// idle).
 int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta, int out_dim, float* d_out,
-                hipStream_t s, int l0, int l1, int stop = -1, const Trace* tr = nullptr) {
+                hipStream_t s, int l0, int l1, bool alone, int stop = -1, const Trace* tr = nullptr) {
   const sg_model_config& c = m->cfg;
   const int T = meta.T, ns = meta.n_seq, d = c.embed_dim, ff = c.interm_dim, L = c.num_layers;
   const int qd = m->qd, kvd = m->kvd, nqkv = m->nqkv;
@@ -623,7 +637,8 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
                                                m->attn_scale, cmax, meta.max_len, s)
                         : sgk::attention(nullptr, kf, vf, n_tiles, att, qd, meta.seq_off, meta.voff, meta.items, meta.n_items,
                                          c.num_heads, c.num_kv_heads, m->hd, m->attn_scale, site(l, 1), meta.max_len,
-                                         s, &qpre, q_attn ? &qout : nullptr, &spill));
+                                         s, &qpre, q_attn ? &qout : nullptr, &spill,
+                                         alone && c.num_kv_heads == 1 ? meta.n_split : 0));
     }
     if (tr && tr->att) SG_HIP(tap(tr->att, att, l, qd));
     if (!(q_attn && m->attn_mode != SG_ATTN_EXACT))
@@ -804,7 +819,7 @@ int forward_device_locked(sg_model* m, const int32_t* d_tokens, const int32_t* o
   }
   int rc = SG_OK;
   if (G == 1) {
-    rc = run_forward(m, w0, d_tokens, meta[0], out_dim, d_out, s, 0, L, stop, tr);
+    rc = run_forward(m, w0, d_tokens, meta[0], out_dim, d_out, s, 0, L, true, stop, tr);
   } else {
     // Each group's ~20 launches per layer go out from a host thread of its
     // own (the calling thread takes the first group): one thread issuing every
@@ -815,7 +830,7 @@ int forward_device_locked(sg_model* m, const int32_t* d_tokens, const int32_t* o
       int r = set_device(m->ctx);
       if (r == SG_OK)
         r = run_forward(m, m->lanes[g], d_tokens + off[b[g]], meta[g], out_dim, d_out + (size_t)b[g] * out_dim,
-                        st[g], 0, L);
+                        st[g], 0, L, false);
       if (r == SG_OK && g > 0 && hipEventRecord(m->lanes[g].done, st[g]) != hipSuccess)
         r = fail(SG_ERR_DEVICE, "hipEventRecord failed (sequence group %d)", g);
       lrc[g] = r;
@@ -1389,7 +1404,7 @@ int sg_attention(sg_ctx* ctx, float* out, const float* q, int32_t ldq, const flo
                             meta.spill_total};
   SG_HIP(sgk::attention(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items,
                         meta.n_items, n_heads, n_kv_heads, head_dim, scale, nullptr,
-                        meta.max_len, s, nullptr, nullptr, &spill));
+                        meta.max_len, s, nullptr, nullptr, &spill, n_kv_heads == 1 ? meta.n_split : 0));
   SG_HIP(hipStreamSynchronize(s));
   return SG_OK;
 }

@@ -52,7 +52,8 @@ __device__ __forceinline__ void sg_lds_copy16(uint32_t lds_addr, uint32_t voff, 
 // __builtin_amdgcn_make_buffer_rsrc builds it (word 3: gfx9 raw buffer).
 __device__ __forceinline__ i32x4_t sg_raw_rsrc(const void* base) {
   const uint64_t a = reinterpret_cast<uint64_t>(base);
-  return i32x4_t{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), 0x7fffffff, 0x00020000};
+  return i32x4_t{__builtin_amdgcn_readfirstlane((int)(uint32_t)a), __builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
+                 0x7fffffff, 0x00020000};
 }
 
 #define SG_WAVE 64

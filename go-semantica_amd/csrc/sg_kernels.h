@@ -212,11 +212,12 @@ hipError_t kv_prep(const float* k, const float* v, int ldkv, const float* kw, in
 // with qknorm_rope's arithmetic) and qf is ignored.  max_len: the
 // longest sequence of the launch.  Pass 1's scores stay in registers up to
 // kAttnRegKeys keys; a longer sequence keeps the rest in spill (required
-// when max_len exceeds kAttnRegKeys).  A sequence gives the same bits
+// when max_len exceeds kAttnRegKeys).  The first n_split items run as two
+// workgroups of half the chunks (not with qout), the same bits.  A sequence gives the same bits
 // whatever the launch's max_len.
 hipError_t attention(const _Float16* qf, const _Float16* kf, const _Float16* vf, int n_tiles, float* out, int ldo, const int32_t* seq_off, const int32_t* voff, const sg_item* items, int n_items, int H, int HKV, int hd, float scale,
                      float* amax, int max_len, hipStream_t s, const sg_attn_qpre* qpre = nullptr,
-                     const sg_attn_qout* qout = nullptr, const sg_attn_spill* spill = nullptr);
+                     const sg_attn_qout* qout = nullptr, const sg_attn_spill* spill = nullptr, int n_split = 0);
 // The same for launches too small to fill the GPU (attn_small_form), with Q
 // pre-split: the same bits as attention(), no spill buffer.  cmax (optional)
 // receives each chunk's max|out|, sequence i's chunks (kv head by kv head) from

@@ -616,6 +616,33 @@ def test_attention_register_scores_match_spilling_launch(gpu_ctx):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("lens", [[512] * 5 + [200], [16] * 66, [21, 85] * 20, [700] * 4,
+                                  [1100, 900, 700, 600, 500, 400, 200], [300] * 11 + [33] * 39])
+def test_attention_split_items_match_whole(gpu_ctx, lens):
+    """65 to 255 items: all, or as many of the longest as there are idle CUs,
+    run as two workgroups of half the chunks (register-held and spilled scores,
+    items with fewer than eight or four chunks).  The same bits as in a launch
+    with enough companions that none is split."""
+    import torch
+    from semantica_gpu import kernels
+    items = sum(-(-3 * -(-n // 16) // 8) for n in lens)
+    assert 64 < items < 256
+    more = lens + [512] * (1 + (256 - items) // 12)
+    off = np.concatenate([[0], np.cumsum(more)]).astype(np.int32)
+    T0, T = sum(lens), sum(more)
+    say(f"attention split items={items} lens={lens}")
+    rng = np.random.default_rng(T0)
+    q = (rng.standard_normal((T, 768)) * rng.uniform(0.5, 1.5, 768)).astype(np.float32)
+    k = (rng.standard_normal((T, 256)) * rng.uniform(0.5, 1.5, 256)).astype(np.float32)
+    v = (rng.standard_normal((T, 256)) * 2).astype(np.float32)
+    out_a = torch.empty((T0, 768), dtype=torch.float32, device="cuda")
+    out_b = torch.empty((T, 768), dtype=torch.float32, device="cuda")
+    kernels.attention(gpu_ctx, out_a, dev(q[:T0]), dev(k[:T0]), dev(v[:T0]), 3, 1, 256, off[:len(lens) + 1])
+    kernels.attention(gpu_ctx, out_b, dev(q), dev(k), dev(v), 3, 1, 256, off)
+    a, b = host(out_a), host(out_b)[:T0]
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_attention_clamped_keys_are_exact_zero(gpu_ctx, oracle):
     """A key 25 above the rest (after scaling) gives the others weight exactly
     0 (fastExp's -10 clamp), so the output is exactly that key's V row."""
