@@ -68,6 +68,7 @@ struct Meta {
   int32_t* row_seq = nullptr;
   int32_t* row_pos = nullptr;
   int32_t* row_key = nullptr;  // the row's key in the padded key numbering
+  int32_t* row_slot = nullptr;  // row_seq * kSlot: the row's sequence in a maxima array with a cache line each
   int32_t* seq_off = nullptr;
   int32_t* voff = nullptr;   // [n_seq + 1] first padded key of each sequence
   sg_item* items = nullptr;  // attention workgroups (sequence, first chunk)
@@ -83,7 +84,7 @@ int seq_groups(int S, int G) {
   return (chunks + sgk::kAttnChunks - 1) / sgk::kAttnChunks;
 }
 
-// Fills `host` with [row_seq | row_pos | row_key | seq_off | voff | items | vtiles |
+// Fills `host` with [row_seq | row_pos | row_key | row_slot | seq_off | voff | items | vtiles |
 // spill_off] and
 // copies it to `dev` on stream s, asynchronously: kernels launched on s after
 // this see the metadata, and the next stage_meta waits for the copy before it
@@ -95,6 +96,10 @@ int seq_groups(int S, int G) {
 // sequences are binned to XCDs (largest first, onto the least-loaded bin) and
 // the list interleaves the bins: all workgroups of a sequence then share one
 // L2 copy of its K and V^T.
+// The gate/up GEMM folds every workgroup's max|g| into its sequences' by atomics,
+// 13 ns each, one after another within a cache line: 13 sequences of 5-60 tokens
+// in one line made the launch 17.9 us, a line per sequence 16.3.
+constexpr int kSlot = 32;  // floats
 constexpr int kAttnLptItems = 512;  // two rounds of attention workgroups on 256 CUs
 constexpr int kAttnCus = 256;
 
@@ -110,7 +115,7 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
     n_spill += (int64_t)seq_groups(S, G) * sgk::attention_spill_tiles(S);
   }
   if (n_spill > INT32_MAX) return fail(SG_ERR_INVALID, "batch too large for the attention spill layout");
-  const size_t bytes = sizeof(int32_t) * ((size_t)3 * T + 2 * (n_seq + 1)) +
+  const size_t bytes = sizeof(int32_t) * ((size_t)4 * T + 2 * (n_seq + 1)) +
                        sizeof(sg_item) * ((size_t)n_items + n_vt) + sizeof(int32_t) * (size_t)n_seq + 64;
   SG_TRY(host.ensure(bytes));
   SG_TRY(dev.ensure(bytes));
@@ -118,7 +123,8 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
   int32_t* rs = h;
   int32_t* rp = rs + T;
   int32_t* rk = rp + T;
-  int32_t* so = rk + T;
+  int32_t* rl = rk + T;
+  int32_t* so = rl + T;
   int32_t* vo = so + n_seq + 1;
   sg_item* it = reinterpret_cast<sg_item*>(vo + n_seq + 1);
   sg_item* vt = it + n_items;
@@ -133,6 +139,7 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
       rs[r] = i;
       rp[r] = r - off[i];
       rk[r] = vo[i] + r - off[i];
+      rl[r] = i * kSlot;
     }
     for (int k0 = 0; k0 < S; k0 += 32) vt[nv++] = sg_item{i, k0};
     sp[i] = ns;
@@ -205,7 +212,8 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
   m.row_seq = d;
   m.row_pos = d + T;
   m.row_key = d + 2 * (size_t)T;
-  m.seq_off = d + 3 * (size_t)T;
+  m.row_slot = d + 3 * (size_t)T;
+  m.seq_off = d + 4 * (size_t)T;
   m.voff = m.seq_off + n_seq + 1;
   m.items = reinterpret_cast<sg_item*>(m.voff + n_seq + 1);
   m.vtiles = m.items + n_items;
@@ -502,7 +510,8 @@ int validate_config(const sg_model_config& c) {
   } while (0)
 
 // The per-layer launch sequence.  amax sites per layer: 0 pre-attention
-// norm, 1 attention output, 2 pre-FFN norm, 3 GELU*up; each [n_seq].
+// norm, 1 attention output, 2 pre-FFN norm, each [n_seq]; GELU*up has its own,
+// by row_slot.
 // Work figures are the algorithmic ones: 2*M*N*K int8 ops per GEMM,
 // 4*H*hd*S^2 flops per sequence for attention, and bytes read + written at
 // the reference's dtypes (fp32 activations, int8 quantized) elsewhere.
@@ -547,7 +556,8 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   const int n_tiles = meta.Tp / 32;
   float* sx = w.sx.as<float>();
   float* amax = w.amax.as<float>();
-  auto site = [&](int l, int k) { return amax + ((size_t)4 * l + k) * ns; };
+  auto site = [&](int l, int k) { return amax + ((size_t)3 * l + k) * ns; };
+  auto gsite = [&](int l) { return amax + (size_t)3 * L * ns + (size_t)l * ns * kSlot; };  // by row_slot
   const float eps = c.norm_eps;
   const double t = T;
   auto gemm_ops = [&](int N, int K) { return 2.0 * t * N * K; };
@@ -586,7 +596,7 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
   _Float16* qf = a_small ? w.qs.as<_Float16>() : nullptr;
 
   if (l0 == 0) {
-    SG_LAUNCH(SG_K_OTHER, 4.0 * 4 * L * ns, sgk::fill_f32(amax, 0.0f, (int64_t)4 * L * ns, s));
+    SG_LAUNCH(SG_K_OTHER, 4.0 * (3 + kSlot) * L * ns, sgk::fill_f32(amax, 0.0f, (int64_t)(3 + kSlot) * L * ns, s));
     // V^T positions past each sequence's end stay zero through the layers
     // (the fused epilogue writes only the sequences' keys).
     if (vt_fused)
@@ -657,8 +667,9 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
     }
     SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(d), norm_q(ly.ffn_norm, site(l, 2)));
     SG_LAUNCH(SG_K_GEMM, gemm_ops(2 * ff, d),
-              sgk::gemm_q8_gelu(a8, ar, ly.wgu, ly.sgu, sx, g, T, ff, d, meta.row_seq, site(l, 3), s, true));
-    SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(ff), quant(g, ff, site(l, 3)));
+              sgk::gemm_q8_gelu(a8, ar, ly.wgu, ly.sgu, sx, g, T, ff, d, meta.row_slot, gsite(l), s, true));
+    SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(ff),
+              sgk::quantize(g, ff, T, ff, meta.row_slot, gsite(l), a8, ar, nullptr, sx, s));
     const bool last = l + 1 == L;
     const float* w_next = last ? m->out_norm : m->layers[l + 1].attn_norm;
     if (sgk::gemm_res_norm_fused(T, d, ly.post_ffw, w_next)) {
@@ -746,7 +757,7 @@ int ensure_workspace(const sg_model* m, Lane& w, const Meta& meta) {
   if (attn_small(m, meta)) SG_TRY(w.qs.ensure(2 * sizeof(_Float16) * (size_t)m->qd * Tp));
   SG_TRY(w.sx.ensure(sizeof(float) * t));
   if (sgk::row_max_form(T, c.embed_dim)) SG_TRY(w.rmax.ensure(sizeof(float) * t));
-  SG_TRY(w.amax.ensure(sizeof(float) * 4 * (size_t)c.num_layers * n_seq));
+  SG_TRY(w.amax.ensure(sizeof(float) * (3 + kSlot) * (size_t)c.num_layers * n_seq));
   SG_TRY(w.ks.ensure(2 * sizeof(_Float16) * (size_t)m->kvd * Tp));
   SG_TRY(w.vt.ensure(2 * sizeof(_Float16) * (size_t)m->kvd * Tp));
   SG_TRY(w.err.ensure(64));
