@@ -665,8 +665,19 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_vnorm(const T* __restrict__ g
   }
   float m = sqrtf(ss);
   if (!(m <= 3.0e38f)) m = __builtin_inff();
+  // One atomic per workgroup, and only if it would raise the maximum: on one
+  // address they go one after another, 13 ns each (one per wave: 25 us for
+  // 100,000 x 256 int16, 11 us now).
+  __shared__ float red[kBfThreads / 64];
   m = sg_wave_max(m);
-  if ((threadIdx.x & 63) == 0) atomicMax(vmax, __float_as_uint(m));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int i = 1; i < kBfThreads / 64; i++) m = fmaxf(m, red[i]);
+    const uint32_t u = __float_as_uint(m);
+    if (u > __hip_atomic_load(vmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(vmax, u);
+  }
 }
 
 // Queries of one pass: normalized in place when asked (builder.go:131-141, as
@@ -674,20 +685,25 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_vnorm(const T* __restrict__ g
 // [256, 512) and rounded to fp16 in the MFMA B operand's order, qfrag [k-step
 // of two 8-element groups][col_tiles][64 lanes][8] (lane 32 h + c: query c of
 // the tile, group 2 s + h; the last k-step's first half holds the tail when
-// dim % 8; zeros elsewhere and for queries past nq).  eps[q] = the bound above
-// in k_bf_approx's units; negative: flagged.  One wave per query.
-__global__ __launch_bounds__(64) void k_bf_prep(float* __restrict__ queries, int nq, int dim, int normalize,
-                                               float vnorm_s, int exact_v, int col_tiles, _Float16* __restrict__ qfrag,
+// dim % 8; zeros elsewhere and for queries past nq).  eps[2 q] = the bound above
+// in k_bf_approx's units, eps[2 q + 1] what takes these to scores.
+// A workgroup per query: one wave took 19 us for 64 queries of 768 dims, four 13.
+constexpr int kPrepThreads = 256;
+__global__ __launch_bounds__(kPrepThreads) void k_bf_prep(float* __restrict__ queries, int nq, int dim, int normalize,
+                                               float vnorm_s, float vunit, int exact_v, int col_tiles, _Float16* __restrict__ qfrag,
                                                float* __restrict__ eps, int32_t* __restrict__ flags) {
   extern __shared__ __attribute__((aligned(16))) float buf[];  // dim rounded up to 16, floats then doubles
   __shared__ float norm;
   __shared__ int scale;
-  const int q = blockIdx.x, lane = threadIdx.x;
+  __shared__ float red[2][kPrepThreads / 64];
+  __shared__ int bad;
+  const int q = blockIdx.x, tid = threadIdx.x, wave = tid >> 6;
   const bool live = q < nq;
   const int dimp = (dim + 15) & ~15;
   float* x = queries + (int64_t)q * dim;
   double* sqs = reinterpret_cast<double*>(buf + dimp);
-  for (int i = lane; i < dimp; i += 64) {
+  if (tid == 0) bad = 0;
+  for (int i = tid; i < dimp; i += kPrepThreads) {
     const float v = live && i < dim ? x[i] : 0.0f;
     const float sq = v * v;
     buf[i] = v;
@@ -695,7 +711,7 @@ __global__ __launch_bounds__(64) void k_bf_prep(float* __restrict__ queries, int
   }
   __syncthreads();
   if (normalize && live) {
-    if (lane == 0) {
+    if (tid == 0) {
       // The float64 sum in index order (the pad's zeros add nothing): a chain of
       // additions, the next 16 squares read under the current 16.
       double sum = 0.0;
@@ -721,7 +737,7 @@ __global__ __launch_bounds__(64) void k_bf_prep(float* __restrict__ queries, int
     __syncthreads();
     const float n = norm;
     if (scale)
-      for (int i = lane; i < dim; i += 64) {
+      for (int i = tid; i < dim; i += kPrepThreads) {
         buf[i] = buf[i] * n;
         x[i] = buf[i];
       }
@@ -729,24 +745,34 @@ __global__ __launch_bounds__(64) void k_bf_prep(float* __restrict__ queries, int
   }
   float m = 0.0f, ss = 0.0f;
   bool finite = true;
-  for (int i = lane; i < dim; i += 64) {
+  for (int i = tid; i < dim; i += kPrepThreads) {
     const float a = fabsf(buf[i]);
     finite = finite && a <= 1.0e30f;
     m = fmaxf(m, a);
   }
-  finite = __ballot(!finite) == 0;
+  if (!finite) bad = 1;
   m = sg_wave_max(m);
+  if ((tid & 63) == 0) red[0][wave] = m;
+  __syncthreads();
+  finite = bad == 0;
+#pragma unroll
+  for (int i = 0; i < kPrepThreads / 64; i++) m = fmaxf(m, red[0][i]);
   const bool ok = live && finite && m >= 1.0e-30f;
   int e = 0;
   if (ok) (void)frexpf(m, &e);  // m = f * 2^e, f in [0.5, 1)
   const float sc = ok ? ldexpf(1.0f, 9 - e) : 0.0f;
-  for (int i = lane; i < dim; i += 64) {
+  for (int i = tid; i < dim; i += kPrepThreads) {
     const float t = buf[i] * sc;
     ss += t * t;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-  if (lane == 0 && live) {
+  if ((tid & 63) == 0) red[1][wave] = ss;
+  __syncthreads();
+  if (tid == 0 && live) {
+    ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kPrepThreads / 64; i++) ss += red[1][i];
     // Per product: fp16 rounding of x (2^-11) and of v unless exact; the two
     // accumulations: at most dim + 32 float32 roundings of up to an ulp (2^-23)
     // each on the matrix cores, dim / 8 + 24 (2^-24) in the reference's order;
@@ -756,12 +782,13 @@ __global__ __launch_bounds__(64) void k_bf_prep(float* __restrict__ queries, int
     const float rel = 4.8829e-4f * (exact_v ? 1.0f : 2.0f) + (float)(dim + 32) * 1.2e-7f +
                       (float)(dim / 8 + 24) * 6.0e-8f + 1.0e-6f;
     const float rd = sqrtf((float)dim) * 3.0e-8f;
-    eps[q] = 1.05f * (rel * xn * vnorm_s + rd * (xn + vnorm_s));
+    eps[2 * q] = 1.05f * (rel * xn * vnorm_s + rd * (xn + vnorm_s));
+    eps[2 * q + 1] = (1.0f / sc) * (1.0f / vunit);  // k_bf_approx's units to scores
     flags[q] = ok ? 0 : 1;
   }
   const int G = dim >> 3, R = dim & 7, ct = q >> 5, c = q & 31;
   const int ks_main = (G + 1) >> 1, ks = ks_main + (R ? 1 : 0);
-  for (int i = lane; i < ks * 2; i += 64) {  // one 8-element piece per lane
+  for (int i = tid; i < ks * 2; i += kPrepThreads) {  // one 8-element piece per thread
     const int s = i >> 1, h = i & 1;
     int src = -1, cnt = 8;
     if (s < ks_main) {
@@ -964,8 +991,9 @@ __device__ __forceinline__ float bf_unkey(uint32_t u) {
 }
 
 // list[q][0 .. count[q]): the blocks that can hold one of query q's k best.
+// Leaves in eps[2 q] the score T - 2 eps, which each of the k best reaches.
 __global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restrict__ blockmax, int nb, int k,
-                                                          const float* __restrict__ eps, int cap,
+                                                          float* __restrict__ eps, int cap,
                                                           int32_t* __restrict__ list, int32_t* __restrict__ count,
                                                           int32_t* __restrict__ flags) {
   __shared__ uint32_t hist[2048 + 64];
@@ -989,7 +1017,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restri
         return bf_key(m);
       },
       (nb + 3) / 4, k, hist, T, above, at);
-  const float cut = bf_unkey(T) - 2.0f * eps[q];
+  const float cut = bf_unkey(T) - 2.0f * eps[2 * q];
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < nb; i += kTopThreads)
@@ -999,52 +1027,99 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restri
     }
   __syncthreads();
   if (threadIdx.x == 0) {
+    eps[2 * q] = cut * eps[2 * q + 1];
     count[q] = cnt <= cap ? cnt : 0;
     if (cnt > cap) flags[q] = 1;
   }
 }
 
+// Half a stored group: four elements as loaded, and as the AVX2 loop's operands.
+template <typename T>
+struct BfHalf;
+template <>
+struct BfHalf<int8_t> {
+  uint32_t w;
+  __device__ void load(const int8_t* p) { w = *reinterpret_cast<const uint32_t*>(p); }
+  __device__ void get(float (&v)[4]) const {
+#pragma unroll
+    for (int l = 0; l < 4; l++) v[l] = (float)(int8_t)(w >> (8 * l)) * BfElem<int8_t>::inv();
+  }
+};
+template <>
+struct BfHalf<int16_t> {
+  uint2 w;
+  __device__ void load(const int16_t* p) { w = *reinterpret_cast<const uint2*>(p); }
+  __device__ void get(float (&v)[4]) const {
+    v[0] = (float)(int16_t)(w.x & 0xffffu) * BfElem<int16_t>::inv();
+    v[1] = (float)(int16_t)(w.x >> 16) * BfElem<int16_t>::inv();
+    v[2] = (float)(int16_t)(w.y & 0xffffu) * BfElem<int16_t>::inv();
+    v[3] = (float)(int16_t)(w.y >> 16) * BfElem<int16_t>::inv();
+  }
+};
+template <>
+struct BfHalf<float> {
+  float4 w;
+  __device__ void load(const float* p) { w = *reinterpret_cast<const float4*>(p); }
+  __device__ void get(float (&v)[4]) const {
+    v[0] = w.x; v[1] = w.y; v[2] = w.z; v[3] = w.w;
+  }
+};
+
 // cand[q][64 i + l]: the score of vector 64 list[q][i] + l in the reference's
-// order (k_bf_score's arithmetic; one query, lane = vector); a wave per listed
-// block.  Vectors past N: NaN bits 0xffffffff, whose key is 0.
+// order (k_bf_score's arithmetic).  Bound by memory latency: a few dozen blocks
+// per query.  So a wave takes half a block, two lanes a vector -- lane 2 v + h
+// keeps the lane sums 4 h .. 4 h + 3 of vector v -- with B groups in flight and
+// the next B behind them; a workgroup takes two blocks and holds its query in
+// LDS.  (A lane per vector with 8 to 16 groups in flight: 14 us for one query
+// over float32 x 512, 32 for 64 over int8 x 768; 7.5 and 22 now.)  Vectors past N: NaN
+// bits 0xffffffff, whose key is 0.
 template <typename T>
 __global__ __launch_bounds__(kBfThreads) void k_bf_rescore(const T* __restrict__ grp, const T* __restrict__ tail, int N,
                                                           int dim, const float* __restrict__ queries,
                                                           const int32_t* __restrict__ list,
                                                           const int32_t* __restrict__ count, int cap,
                                                           float* __restrict__ cand) {
-  constexpr int B = sizeof(T) == 4 ? 8 : 16;  // groups in flight per lane
-  const int q = blockIdx.y, lane = threadIdx.x & 63;
-  const int i = blockIdx.x * (kBfThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (i >= count[q]) return;
-  const int n = list[(int64_t)q * cap + i] * kPfBlock + lane;
+  constexpr int B = sizeof(T) == 4 ? 16 : 32;  // half groups in flight per lane
+  extern __shared__ __attribute__((aligned(16))) float xs[];  // the query's whole groups
+  const int q = blockIdx.y, lane = threadIdx.x & 63, h = lane & 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // The wave's entry is read along with the count (cap is even: in bounds); a
+  // second block past the list repeats the first one.
+  const int i0 = blockIdx.x * (kBfThreads / 128);
+  const int e0 = list[(int64_t)q * cap + i0], e1 = list[(int64_t)q * cap + i0 + 1];
+  const int n_list = count[q];
+  if (i0 >= n_list) return;  // workgroup-uniform
+  const bool second = (wave >> 1) && i0 + 1 < n_list;
+  const int i = i0 + (second ? 1 : 0);
+  const int l = 32 * (wave & 1) + (lane >> 1);  // vector of the block
+  const int n = (second ? e1 : e0) * kPfBlock + l;
   const int nn = min(n, N - 1);
   const int G = dim >> 3, R = dim & 7;
   const float* x = queries + (int64_t)q * dim;
-  float acc[8];
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  const T* gp = grp + (int64_t)nn * 8 + 4 * h;
+  const int64_t gs = (int64_t)N * 8;
+  // No branch between a load and its use: it would sink the loads.
+  BfHalf<T> cur[B], nxt[B];
 #pragma unroll
-  for (int l = 0; l < 8; l++) acc[l] = 0.0f;
-  auto add = [&](const BfRaw<T>& raw, int g) {
-    float v[8];
+  for (int u = 0; u < B; u++) cur[u].load(gp + min(u, G - 1) * gs);
+  for (int e = threadIdx.x; e < 8 * G; e += kBfThreads) xs[e] = x[e];
+  __syncthreads();
+  auto add = [&](const BfHalf<T>& raw, int g) {
+    float v[4];
     raw.get(v);
+    const float4 xv4 = *reinterpret_cast<const float4*>(xs + 8 * g + 4 * h);
+    const float xv[4] = {xv4.x, xv4.y, xv4.z, xv4.w};
 #pragma unroll
-    for (int l = 0; l < 8; l++) {
-      const float xv = x[8 * g + l];
+    for (int t = 0; t < 4; t++) {
       if constexpr (BfElem<T>::kQuant) {
-        const float p = v[l] * xv;
-        acc[l] = acc[l] + p;
+        const float p = v[t] * xv[t];
+        acc[t] = acc[t] + p;
       } else {
-        acc[l] = __builtin_fmaf(v[l], xv, acc[l]);
+        acc[t] = __builtin_fmaf(v[t], xv[t], acc[t]);
       }
     }
   };
-  // Batches of B loads, the next batch in flight under the current one's sums
-  // (no branch between a load and its use: it would sink the loads).
-  const T* gp = grp + (int64_t)nn * 8;
-  const int64_t gs = (int64_t)N * 8;
-  BfRaw<T> cur[B], nxt[B];
-#pragma unroll
-  for (int u = 0; u < B; u++) cur[u].load(gp + min(u, G - 1) * gs);
   int g = 0;
   for (; g + B <= G; g += B) {
 #pragma unroll
@@ -1058,26 +1133,103 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_rescore(const T* __restrict__
 #pragma unroll
   for (int u = 0; u < B; u++)
     if (g + u < G) add(cur[u], g + u);
-  const float sum = bf_finish<T>(acc, G, R, x + 8 * G, tail + (int64_t)nn * R);
-  cand[((int64_t)q * cap + i) * kPfBlock + lane] = n < N ? sum : __uint_as_float(0xffffffffu);
+  float s8[8];
+#pragma unroll
+  for (int t = 0; t < 4; t++) {
+    const float o = __shfl_xor(acc[t], 1);
+    s8[t] = h ? o : acc[t];
+    s8[4 + t] = h ? acc[t] : o;
+  }
+  const float sum = bf_finish<T>(s8, G, R, x + 8 * G, tail + (int64_t)nn * R);
+  if (h == 0) cand[((int64_t)q * cap + i) * kPfBlock + l] = n < N ? sum : __uint_as_float(0xffffffffu);
 }
 
 // The exact top k of the candidates: out_idx/out_dist [q][k] in arbitrary
-// order; a tie straddling the k-th place flags the query.
+// order; a tie straddling the k-th place flags the query.  The candidates that
+// reach cut[2 q] (at least k of them: k_bf_blocks) are few as a rule: gathered in
+// LDS, each is ranked against the others.  (With k or more of them the k best are
+// among them whatever the cut.)  Three radix passes over all
+// candidates, a chain of barriers, took 9.6 us for one query of 150,000 vectors, 5.0 now; they are
+// left for more than kTopRank of them.
+constexpr int kTopRank = kTopThreads, kTopAhead = 2;
 __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict__ cand,
                                                        const int32_t* __restrict__ list,
                                                        const int32_t* __restrict__ count, int cap, int k,
-                                                       int32_t* __restrict__ out_idx, float* __restrict__ out_dist,
-                                                       int32_t* __restrict__ flags) {
+                                                       const float* __restrict__ cut, int32_t* __restrict__ out_idx,
+                                                       float* __restrict__ out_dist, int32_t* __restrict__ flags) {
   __shared__ uint32_t hist[2048 + 64];
-  __shared__ int cnt;
+  __shared__ __attribute__((aligned(16))) uint32_t keys[kTopRank];
+  __shared__ float score[kTopRank];
+  __shared__ int from[kTopRank];
+  __shared__ int cnt, tie;
   const int q = blockIdx.x;
+  // The first candidates are read along with their number (the buffer holds at
+  // least 68 blocks per query).
+  static_assert(sgk::bf_prefilter_cap(1) * kPfBlock >= kTopAhead * kTopThreads, "reads ahead in bounds");
+  float ahead[kTopAhead];
+  int block[kTopAhead];
+#pragma unroll
+  for (int u = 0; u < kTopAhead; u++) {
+    const int i = threadIdx.x + u * kTopThreads;
+    ahead[u] = cand[(int64_t)q * cap * kPfBlock + i];
+    block[u] = list[(int64_t)q * cap + i / kPfBlock];
+  }
   const int n = count[q] * kPfBlock;
   if (flags[q] || n < k) {
     if (threadIdx.x == 0) flags[q] = 1;
     return;
   }
   const float* cs = cand + (int64_t)q * cap * kPfBlock;
+  if (threadIdx.x == 0) cnt = tie = 0;
+  keys[threadIdx.x] = 0u;  // below every score's key
+  __syncthreads();
+  const float least = cut[2 * q];
+  auto take = [&](float d, int at) {
+    if (d >= least) {  // not the NaN past the last vector
+      const int slot = atomicAdd(&cnt, 1);
+      if (slot < kTopRank) {
+        keys[slot] = bf_key(d);
+        score[slot] = d;
+        from[slot] = at;
+      }
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < kTopAhead; u++) {
+    const int i = threadIdx.x + u * kTopThreads;
+    if (i < n) take(ahead[u], block[u] * kPfBlock + i % kPfBlock);
+  }
+  for (int i = threadIdx.x + kTopAhead * kTopThreads; i < n; i += kTopThreads)
+    take(cs[i], list[(int64_t)q * cap + i / kPfBlock] * kPfBlock + i % kPfBlock);
+  __syncthreads();
+  const int m = cnt;
+  if (m >= k && m <= kTopRank) {
+    if ((int)threadIdx.x < m) {
+      const uint32_t u = keys[threadIdx.x];
+      int gt = 0, eq = 0, before = 0;
+      for (int j = 0; j < m; j += 4) {
+        const uint4 o4 = *reinterpret_cast<const uint4*>(&keys[j]);
+        const uint32_t o[4] = {o4.x, o4.y, o4.z, o4.w};
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+          gt += o[t] > u;
+          eq += o[t] == u;
+          before += o[t] == u && j + t < (int)threadIdx.x;
+        }
+      }
+      if (gt < k) {
+        if (gt + eq > k) {
+          tie = 1;
+        } else {
+          out_idx[(int64_t)q * k + gt + before] = from[threadIdx.x];
+          out_dist[(int64_t)q * k + gt + before] = score[threadIdx.x];
+        }
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && tie) flags[q] = 1;
+    return;
+  }
   auto key = [&](int i) {
     const float d = cs[i];
     return __float_as_uint(d) == 0xffffffffu ? 0u : bf_key(d);
@@ -1316,8 +1468,8 @@ hipError_t bf_prefilter(int mode, const void* grp, const void* tail, int N, int 
   } else {
     vs = vnorm * (mode == kBfI8 ? 127.0f : 32767.0f);
   }
-  hipLaunchKernelGGL(k_bf_prep, dim3(32 * ct), dim3(64), (sizeof(float) + sizeof(double)) * (size_t)((dim + 15) & ~15), s, queries, nq, dim,
-                     normalize ? 1 : 0, vs * 1.01f, mode == kBfI8 ? 1 : 0, ct, w.qfrag, w.eps, w.flags);
+  hipLaunchKernelGGL(k_bf_prep, dim3(32 * ct), dim3(kPrepThreads), (sizeof(float) + sizeof(double)) * (size_t)((dim + 15) & ~15), s, queries, nq, dim,
+                     normalize ? 1 : 0, vs * 1.01f, vs / vnorm, mode == kBfI8 ? 1 : 0, ct, w.qfrag, w.eps, w.flags);
   hipError_t e = hipErrorInvalidValue;
   switch (mode) {
 #define SG_PF(MODE, T)                                                                                           \
@@ -1327,7 +1479,8 @@ hipError_t bf_prefilter(int mode, const void* grp, const void* tail, int N, int 
     if (e != hipSuccess) return e;                                                                               \
     hipLaunchKernelGGL(k_bf_blocks, dim3(nq), dim3(kTopThreads), 0, s, w.blockmax, nb, k, w.eps, cap, w.list,    \
                        w.count, w.flags);                                                                        \
-    hipLaunchKernelGGL(k_bf_rescore<T>, dim3(nblocks(cap, kBfThreads / 64), nq), dim3(kBfThreads), 0, s,         \
+    hipLaunchKernelGGL(k_bf_rescore<T>, dim3(nblocks(cap, kBfThreads / 128), nq), dim3(kBfThreads),               \
+                       sizeof(float) * (size_t)(dim & ~7), s,                                                     \
                        static_cast<const T*>(grp), static_cast<const T*>(tail), N, dim, queries, w.list, w.count, \
                        cap, w.cand);                                                                             \
     break;
@@ -1338,8 +1491,8 @@ hipError_t bf_prefilter(int mode, const void* grp, const void* tail, int N, int 
     default:
       return e;
   }
-  hipLaunchKernelGGL(k_bf_top, dim3(nq), dim3(kTopThreads), 0, s, w.cand, w.list, w.count, cap, k, w.out_idx,
-                     w.out_dist, w.flags);
+  hipLaunchKernelGGL(k_bf_top, dim3(nq), dim3(kTopThreads), 0, s, w.cand, w.list, w.count, cap, k, w.eps,
+                     w.out_idx, w.out_dist, w.flags);
   return hipGetLastError();
 }
 

@@ -287,12 +287,12 @@ hipError_t bf_select(const float* scores, int64_t ld_scores, int N, int nq, int 
 hipError_t bf_vnorm(int mode, const void* grp, const void* tail, int N, int dim, uint32_t* vmax, hipStream_t s);
 constexpr int kBfBlock = 64;            // vectors per block
 constexpr size_t kBfPfLds = 144 << 10;  // LDS for the queries' fragments
-inline int bf_prefilter_cap(int k) { return 4 * k + 64; }  // listed blocks per query
+constexpr int bf_prefilter_cap(int k) { return 4 * k + 64; }  // listed blocks per query
 bool bf_prefilter_ok(int N, int dim, int k, float vnorm);
 int bf_prefilter_queries(int dim);  // queries per call
 struct sg_bf_work {
   _Float16* qfrag;   // 64 x (dim rounded up to 32) + 1024
-  float* eps;        // [nq]
+  float* eps;        // [nq][2]: the bound (then the score that the k best reach), its unit
   float* blockmax;   // [nq][blocks]
   int32_t* list;     // [nq][cap]
   int32_t* count;    // [nq]

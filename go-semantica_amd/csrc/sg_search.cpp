@@ -443,7 +443,7 @@ int sg_index_search(sg_index* x, const float* queries, int32_t n_queries, int32_
       off += (bytes + 255) & ~(size_t)255;
       return o;
     };
-    const size_t o_frag = part(sizeof(_Float16) * frag), o_eps = part(sizeof(float) * qb),
+    const size_t o_frag = part(sizeof(_Float16) * frag), o_eps = part(2 * sizeof(float) * qb),
                  o_bm = part(sizeof(float) * qb * nb), o_list = part(sizeof(int32_t) * qb * cap),
                  o_cnt = part(sizeof(int32_t) * qb), o_cand = part(sizeof(float) * qb * cap * sgk::kBfBlock);
     SG_TRY(x->pf.ensure(off));

@@ -333,6 +333,29 @@ def test_prefilter_hands_back_crowded_queries(gpu_ctx, mode):
     _check(_build(gpu_ctx, ids, vecs, mode), vecs, ids, mode, q, k, False, "crowded")
 
 
+@pytest.mark.parametrize("crowd", [12, 900, 1030, 3000])
+@pytest.mark.parametrize("mode", MODES)
+def test_prefilter_ranks_or_selects(gpu_ctx, mode, crowd):
+    """Candidates that reach the cut: fewer than the 1024 that are ranked
+    against each other, and more (radix selection), near the query and side by
+    side; once with a tie inside the k best and once with one that straddles
+    the k-th place."""
+    rng = np.random.default_rng(crowd + mode)
+    n, dim, k = 30000, 40, 10
+    base = rng.standard_normal(dim)
+    vecs = rng.standard_normal((n, dim)).astype(np.float32)
+    vecs[640:640 + crowd] = base + 0.2 * rng.standard_normal((crowd, dim))
+    vecs[7] = vecs[8] = base  # a tie for the first place
+    vecs[9], vecs[20000] = base + 1e-3, base + 1e-3
+    ids = rng.permutation(n).astype(np.int32)
+    idx = _build(gpu_ctx, ids, vecs, mode)
+    q = np.stack([base, base + 0.1 * rng.standard_normal(dim)]).astype(np.float32)
+    say(f"crowd={crowd} mode={MODE_NAMES[mode]}")
+    _check(idx, vecs, ids, mode, q, k, False, "ties inside")
+    _check(idx, vecs, ids, mode, q, 1, False, "tie at the first place")
+    _check(idx, vecs, ids, mode, q, 3, False, "tie at the third place")
+
+
 @pytest.mark.parametrize("dim,n", [(1, 3), (7, 64), (64, 65), (71, 200), (200, 129)])
 @pytest.mark.parametrize("mode", MODES)
 def test_build_tiles_match_oracle(gpu_ctx, mode, dim, n):
