@@ -288,7 +288,7 @@ __device__ __forceinline__ float bf_finish(const float (&l)[8], int G, int R, co
   return sum;
 }
 
-// scores[q][n] for QB queries (rows q0.. of `queries`, already normalized)
+// scores[q][n] for QB queries (rows q0 + QB * blockIdx.y .. of `queries`, already normalized)
 // against every stored vector; lane = vector.  The workgroup stages the
 // queries in LDS, kQChunk dimensions at a time, and every lane reads them by
 // broadcast; each lane issues the loads of kBfBatch groups before using them.
@@ -302,6 +302,7 @@ __global__ __launch_bounds__(kBfThreads) void k_bf_score(const T* __restrict__ g
                                                         int N, int dim, const float* __restrict__ queries, int q0,
                                                         int nq, float* __restrict__ scores, int64_t ld_scores) {
   __shared__ __attribute__((aligned(16))) float qs[QB][kQChunk];
+  q0 += QB * blockIdx.y;
   const int n = blockIdx.x * kBfThreads + threadIdx.x;
   const bool live = n < N;
   const int nn = live ? n : N - 1;  // lanes past the end load a valid vector and store nothing
@@ -525,14 +526,7 @@ __device__ __forceinline__ void bf_min_slot(const float* dist, int k, float& mn,
   mi = idx;
 }
 
-__global__ __launch_bounds__(64) void k_bf_stream(const float* __restrict__ scores, int64_t ld_scores, int N, int k,
-                                                 const int32_t* __restrict__ state, int32_t* __restrict__ out_idx,
-                                                 float* __restrict__ out_dist) {
-  const int q = blockIdx.x;
-  if (state[8 * q + 7] == 0) return;
-  const float* s = scores + (int64_t)q * ld_scores;
-  int32_t* oi = out_idx + (int64_t)q * k;
-  float* od = out_dist + (int64_t)q * k;
+__device__ void bf_stream(const float* __restrict__ s, int N, int k, int32_t* oi, float* od) {
   const int lane = threadIdx.x;
   for (int j = lane; j < k; j += 64) {  // the first k fill the list
     oi[j] = j;
@@ -559,6 +553,14 @@ __global__ __launch_bounds__(64) void k_bf_stream(const float* __restrict__ scor
       live &= __ballot(i < N && d > mn);
     }
   }
+}
+
+__global__ __launch_bounds__(64) void k_bf_stream(const float* __restrict__ scores, int64_t ld_scores, int N, int k,
+                                                 const int32_t* __restrict__ state, int32_t* __restrict__ out_idx,
+                                                 float* __restrict__ out_dist) {
+  const int q = blockIdx.x;
+  if (state[8 * q + 7] == 0) return;
+  bf_stream(scores + (int64_t)q * ld_scores, N, k, out_idx + (int64_t)q * k, out_dist + (int64_t)q * k);
 }
 
 // ------------------------------------------------------------- prefiltering --
@@ -910,13 +912,14 @@ __global__ __launch_bounds__(kPfThreads<CT>, 2) void k_bf_approx(const T* __rest
   }
 }
 
-// The value T of a workgroup's radix select over n keys key(i), i < n: the keys'
+// The value T of a workgroup's radix select over the keys that visit(f) hands to
+// f(valid, key), a whole wave at a time: the keys'
 // top bits (kSelBits0 + kSelBits1 [+ kSelBits2]) of the k-th largest key with
 // the rest zero; above = keys above T's bin, at = keys in it.  hist: 2048 + 64
 // words of LDS.  Every thread of the workgroup calls this.
 constexpr int kTopThreads = 1024;
 template <int PASSES, typename F>
-__device__ __forceinline__ void wg_select(F key, int n, int k, uint32_t* hist, uint32_t& T, int& above, int& at) {
+__device__ __forceinline__ void wg_select(F visit, int k, uint32_t* hist, uint32_t& T, int& above, int& at) {
   __shared__ uint32_t sh_prefix;
   __shared__ int sh_above, sh_at;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -928,13 +931,9 @@ __device__ __forceinline__ void wg_select(F key, int n, int k, uint32_t* hist, u
     const uint32_t mask = p == 0 ? 0u : ~0u << (p == 1 ? 21 : 10);
     for (int i = tid; i < 2048; i += kTopThreads) hist[i] = 0;
     __syncthreads();
-    for (int i0 = 0; i0 < n; i0 += kTopThreads) {
-      const int i = i0 + tid;
+    visit([&](bool valid, uint32_t u) {
       int bin = -1;
-      if (i < n) {
-        const uint32_t u = key(i);
-        if ((u & mask) == prefix) bin = (int)((u >> shift) & ((1u << bits) - 1u));
-      }
+      if (valid && (u & mask) == prefix) bin = (int)((u >> shift) & ((1u << bits) - 1u));
       // Scores crowd into a few bins of the top digit: one addition per
       // distinct bin of the wave there.
       if (p == 0) {
@@ -948,7 +947,7 @@ __device__ __forceinline__ void wg_select(F key, int n, int k, uint32_t* hist, u
       } else if (bin >= 0) {
         atomicAdd(&hist[bin], 1u);
       }
-    }
+    });
     __syncthreads();
     // Suffix counts: thread t owns bins 2t, 2t + 1.
     uint32_t* wsum = hist + 2048;
@@ -985,6 +984,17 @@ __device__ __forceinline__ void wg_select(F key, int n, int k, uint32_t* hist, u
   at = in_bin;
 }
 
+// visit of n keys key(i), i < n.
+template <typename K>
+__device__ __forceinline__ auto each_key(K key, int n) {
+  return [=](auto f) {
+    for (int i0 = 0; i0 < n; i0 += kTopThreads) {
+      const int i = i0 + (int)threadIdx.x;
+      f(i < n, i < n ? key(i) : 0u);
+    }
+  };
+}
+
 // The float whose bf_key is u.
 __device__ __forceinline__ float bf_unkey(uint32_t u) {
   return __uint_as_float((u & 0x80000000u) ? u & 0x7fffffffu : ~u);
@@ -1010,13 +1020,15 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restri
   // for a quarter of the keys.  Its low bits are zero, and the cut's own
   // rounding is covered by eps' slack.
   wg_select<2>(
-      [&](int i) {
-        float m = bm[4 * i];
+      each_key(
+          [=](int i) {
+            float m = bm[4 * i];
 #pragma unroll
-        for (int u = 1; u < 4; u++) m = fmaxf(m, bm[min(4 * i + u, nb - 1)]);
-        return bf_key(m);
-      },
-      (nb + 3) / 4, k, hist, T, above, at);
+            for (int u = 1; u < 4; u++) m = fmaxf(m, bm[min(4 * i + u, nb - 1)]);
+            return bf_key(m);
+          },
+          (nb + 3) / 4),
+      k, hist, T, above, at);
   const float cut = bf_unkey(T) - 2.0f * eps[2 * q];
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
@@ -1230,13 +1242,13 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict_
     if (threadIdx.x == 0 && tie) flags[q] = 1;
     return;
   }
-  auto key = [&](int i) {
+  auto key = [=](int i) {
     const float d = cs[i];
     return __float_as_uint(d) == 0xffffffffu ? 0u : bf_key(d);
   };
   uint32_t T;
   int above, at;
-  wg_select<3>(key, n, k, hist, T, above, at);
+  wg_select<3>(each_key(key, n), k, hist, T, above, at);
   if (above + at != k) {
     if (threadIdx.x == 0) flags[q] = 1;
     return;
@@ -1251,6 +1263,53 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict_
         out_dist[(int64_t)q * k + slot] = cs[i];
       }
     }
+}
+
+// The whole selection over N <= R * 1024 scores in one launch, a workgroup per
+// query with its keys in registers: the radix select, then the scores >= v_k, or
+// (a straddling tie) the first wave's replay of the streaming loop.  The
+// general path is ten launches, four of them grid-wide passes: a
+// query over 2000 x 256 int8 took 91 us with it, 40 with this; 4 over 10,000 x 512
+// 147 and 71; 8 over 30,000 x 256 (k = 100) 174 and 137.  From about 45,000 (64 queries:
+// 440 and 457) the grid-wide passes are the faster ones.
+constexpr int kSelMost = 32;  // keys per thread of the largest instance
+template <int R>
+__global__ __launch_bounds__(kTopThreads) void k_bf_select_wg(const float* __restrict__ scores, int64_t ld_scores, int N,
+                                                             int k, int32_t* __restrict__ out_idx,
+                                                             float* __restrict__ out_dist) {
+  __shared__ uint32_t hist[2048 + 64];
+  __shared__ int cnt;
+  const int q = blockIdx.x, tid = threadIdx.x;
+  const float* s = scores + (int64_t)q * ld_scores;
+  int32_t* oi = out_idx + (int64_t)q * k;
+  float* od = out_dist + (int64_t)q * k;
+  float d[R];
+#pragma unroll
+  for (int u = 0; u < R; u++) d[u] = s[min(u * kTopThreads + tid, N - 1)];
+  if (tid == 0) cnt = 0;
+  uint32_t T;
+  int above, at;
+  wg_select<3>(
+      [&](auto f) {
+#pragma unroll
+        for (int u = 0; u < R; u++) f(u * kTopThreads + tid < N, bf_key(d[u]));
+      },
+      k, hist, T, above, at);
+  if (above + at != k) {  // a tie straddles the k-th place (workgroup-uniform)
+    if (tid < 64) bf_stream(s, N, k, oi, od);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < R; u++) {
+    const int i = u * kTopThreads + tid;
+    if (i < N && bf_key(d[u]) >= T) {
+      const int slot = atomicAdd(&cnt, 1);
+      if (slot < k) {
+        oi[slot] = i;
+        od[slot] = d[u];
+      }
+    }
+  }
 }
 
 __global__ void k_bf_fill_i32(int32_t* p, int64_t n, int32_t v) {
@@ -1272,25 +1331,22 @@ hipError_t score_t(const void* grp, const void* tail, int N, int dim, const floa
   const T* g = static_cast<const T*>(grp);
   const T* t = static_cast<const T*>(tail);
   const unsigned nb = nblocks(N, kBfThreads);
+  // Queries per lane: 8 use a loaded vector best.  A launch of few workgroups is
+  // bound by one workgroup's time instead (a vector's loads and sums in a row),
+  // so there the queries go to as many workgroups as two a CU (the sums are
+  // the same).  With the selection in one launch below: 16 queries over 3000 x 768
+  // int8 168 -> 70 us, 32 over 13,000 x 300 182 -> 92.
+  int most = 8;
+  while (most > 1 && (int64_t)nb * ((nq + most - 1) / most) < 512) most /= 2;
+  if (most < 8 && (int64_t)nb * ((nq + most - 1) / most) > 512) most *= 2;
   for (int q0 = 0; q0 < nq;) {
     const int left = nq - q0;
-    if (left >= 8) {
-      hipLaunchKernelGGL((k_bf_score<T, 8>), dim3(nb, 1), dim3(kBfThreads), 0, s, g, t, N, dim, queries, q0, nq,
-                         scores, ld);
-      q0 += 8;
-    } else if (left >= 4) {
-      hipLaunchKernelGGL((k_bf_score<T, 4>), dim3(nb, 1), dim3(kBfThreads), 0, s, g, t, N, dim, queries, q0, nq,
-                         scores, ld);
-      q0 += 4;
-    } else if (left >= 2) {
-      hipLaunchKernelGGL((k_bf_score<T, 2>), dim3(nb, 1), dim3(kBfThreads), 0, s, g, t, N, dim, queries, q0, nq,
-                         scores, ld);
-      q0 += 2;
-    } else {
-      hipLaunchKernelGGL((k_bf_score<T, 1>), dim3(nb, 1), dim3(kBfThreads), 0, s, g, t, N, dim, queries, q0, nq,
-                         scores, ld);
-      q0 += 1;
-    }
+    int qb = most;
+    while (qb > left) qb /= 2;
+    const int groups = left / qb < 65535 ? left / qb : 65535;
+    const auto f = qb == 8 ? k_bf_score<T, 8> : qb == 4 ? k_bf_score<T, 4> : qb == 2 ? k_bf_score<T, 2> : k_bf_score<T, 1>;
+    hipLaunchKernelGGL(f, dim3(nb, groups), dim3(kBfThreads), 0, s, g, t, N, dim, queries, q0, nq, scores, ld);
+    q0 += qb * groups;
   }
   return hipGetLastError();
 }
@@ -1392,6 +1448,13 @@ hipError_t bf_select(const float* scores, int64_t ld_scores, int N, int nq, int 
                      int32_t* out_idx, float* out_dist, hipStream_t s) {
   if (N <= 0 || nq <= 0 || k <= 0) return hipSuccess;
   if (k > N) return hipErrorInvalidValue;
+  if (N <= kSelMost * kTopThreads) {
+    const auto f = N <= 4 * kTopThreads    ? k_bf_select_wg<4>
+                   : N <= 16 * kTopThreads ? k_bf_select_wg<16>
+                                           : k_bf_select_wg<kSelMost>;
+    hipLaunchKernelGGL(f, dim3(nq), dim3(kTopThreads), 0, s, scores, ld_scores, N, k, out_idx, out_dist);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_bf_state_init, dim3(nblocks((int64_t)nq * 8, 256)), dim3(256), 0, s, state, nq, k);
   hipLaunchKernelGGL(k_bf_fill_i32, dim3(nblocks((int64_t)nq * 256, 256)), dim3(256), 0, s,
                      reinterpret_cast<int32_t*>(hist), (int64_t)nq * 256, 0);

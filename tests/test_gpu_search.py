@@ -356,6 +356,23 @@ def test_prefilter_ranks_or_selects(gpu_ctx, mode, crowd):
     _check(idx, vecs, ids, mode, q, 3, False, "tie at the third place")
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1025, 4096, 4097, 16384, 16385, 32768, 32769])
+def test_selection_sizes_match_oracle(gpu_ctx, n):
+    """The one-launch selection at the edges of its sizes and the general one
+    past them (9 dimensions: never prefiltered), with the k-th place tied and
+    not, k = 1 and k = all included."""
+    rng = np.random.default_rng(n)
+    vecs = rng.standard_normal((n, 9)).astype(np.float32)
+    if n > 8:
+        vecs[n // 2] = vecs[n - 1] = vecs[3]
+    ids = rng.permutation(2 * n)[:n].astype(np.int32)
+    idx = _build(gpu_ctx, ids, vecs, MODES[0])
+    q = np.stack([vecs[min(3, n - 1)], rng.standard_normal(9)]).astype(np.float32)
+    for k in sorted({1, 2, 3, 100, n} if n <= 1025 else {1, 2, 3, 100}):
+        say(f"selection n={n} k={k}")
+        _check(idx, vecs, ids, MODES[0], q, k, False, f"k={k}")
+
+
 @pytest.mark.parametrize("dim,n", [(1, 3), (7, 64), (64, 65), (71, 200), (200, 129)])
 @pytest.mark.parametrize("mode", MODES)
 def test_build_tiles_match_oracle(gpu_ctx, mode, dim, n):
