@@ -410,14 +410,17 @@ struct Lane {
 // A large batch runs as up to kLanes sequence groups on as many streams: the
 // groups' kernels overlap on the GPU (each kernel's ramp-up and tail filled by
 // the other group's work, and at times one group's bandwidth-bound row kernels
-// beside the other's GEMMs), with every sequence's arithmetic unchanged.  A
-// group gets at least kLaneMinTokens tokens.  Two groups measured best at
+// beside the other's GEMMs), with every sequence's arithmetic unchanged
+// (lane_count has the sizes that do).  Two groups measured best at
 // 64 x 512 tokens on MI355X (first: 19.2 ms per batch against 20.1 for one,
 // 19.4 for three; with the fused GEMM + residual post-norm kernels: 16.80
 // against 17.56 for three; four leave two streams on one of the process's
 // four hardware queues and lose to one group).
 constexpr int kLanes = 2;
-constexpr int kLaneMinTokens = 4096;
+constexpr int kLaneTokens = 8192;       // two groups from here on
+constexpr int kLaneTokensEven = 6144;   // and from here when the groups are alike (lane_count)
+constexpr int kLaneTokensShort = 4096;  // and here when no sequence is over kLaneShortLen
+constexpr int kLaneShortLen = 128;
 
 struct sg_model {
   sg_ctx* ctx = nullptr;
@@ -784,6 +787,36 @@ void lane_split(const int32_t* off, int n_seq, int G, int* b) {
   }
 }
 
+// Sequence groups of a batch, and their boundaries b.  ms per forward, one group
+// / two: 6652 tokens in 14 sequences 5.49 / 5.10, 7350 in 16 6.11 / 5.41, 7187
+// in 4 9.00 / 8.24, 6985 in 400 5.11 / 4.65.  Unequal groups lose, in tokens
+// (5630 in 3, 67 % of them in one group: 7.61 / 8.36) or in attention (one of
+// 2048 and 45 of 100: 7.50 / 7.95; exact attention, four of 1000 and 120 of 20, 75 %
+// of it in one group: 20.98 / 22.84), and under about 5500 tokens so does attention, whose items one group alone runs as two workgroups each to
+// fill the GPU (4999 in 11: 4.40 / 4.56, 5391 in 6: 5.52 / 5.96) -- unless the
+// sequences are short and attention is little of the work (4160 in 300:
+// 3.95 / 3.41, 4478 in 50: 3.88 / 3.62; 3232 in 36: 3.06 / 3.09).
+int lane_count(const int32_t* off, int n_seq, int* b) {
+  static_assert(kLanes == 2, "sizes measured for two groups");
+  const int T = off[n_seq];
+  if (n_seq >= 2 && T >= kLaneTokensShort) {
+    lane_split(off, n_seq, 2, b);
+    const int64_t big = std::max(off[b[1]], T - off[b[1]]);
+    int longest = 0;
+    int64_t sq[2] = {0, 0};  // attention work
+    for (int i = 0; i < n_seq; i++) {
+      const int64_t n = off[i + 1] - off[i];
+      longest = std::max(longest, (int)n);
+      sq[i >= b[1]] += n * n;
+    }
+    const int least = longest <= kLaneShortLen ? kLaneTokensShort : kLaneTokensEven;
+    const bool even = 5 * big <= 3 * (int64_t)T && 3 * std::max(sq[0], sq[1]) <= 2 * (sq[0] + sq[1]);
+    if (T >= kLaneTokens || (T >= least && even)) return 2;
+  }
+  lane_split(off, n_seq, 1, b);
+  return 1;
+}
+
 int forward_device_locked(sg_model* m, const int32_t* d_tokens, const int32_t* off, int n_seq, int out_dim,
                           float* d_out, hipStream_t s, int stop = -1, const Trace* tr = nullptr) {
   int len_err_seq = n_seq;
@@ -797,13 +830,12 @@ int forward_device_locked(sg_model* m, const int32_t* d_tokens, const int32_t* o
     SG_TRY(token_error(w0, d_tokens, s));
     return length_error(m, off[len_err_seq + 1] - off[len_err_seq]);
   }
-  const int T = off[n_seq], L = m->cfg.num_layers, GQ = m->cfg.num_heads / m->cfg.num_kv_heads;
+  const int L = m->cfg.num_layers, GQ = m->cfg.num_heads / m->cfg.num_kv_heads;
   // Sequence groups: one for the per-layer and profiled paths (their outputs
   // and timings cover the whole batch in order), else up to kLanes.
   int G = 1;
-  if (stop < 0 && !tr && !m->prof.on) G = std::max(1, std::min(std::min(kLanes, n_seq), T / kLaneMinTokens));
-  int b[kLanes + 1];
-  lane_split(off, n_seq, G, b);
+  int b[kLanes + 1] = {0, n_seq};
+  if (stop < 0 && !tr && !m->prof.on) G = lane_count(off, n_seq, b);
   hipStream_t st[kLanes];
   st[0] = s;
   if (G > 1) {

@@ -341,6 +341,29 @@ def test_sequence_groups_match_one_stream(tiny_gpu):
 
 
 @pytest.mark.parametrize("mode", ["fast", "exact"])
+@pytest.mark.parametrize("lens", [[128] * 32, [128] * 31 + [127], [129] + [127] * 32, [1] * 4096, [512] * 12,
+                                  [512] * 11 + [511], [2048] * 3, [1229] * 4 + [1228],
+                                  [2048] + [60] * 69, [1000] * 6 + [999, 400], [1] * 3000 + [2048, 2048], [2048] * 3 + [2047]])
+def test_sequence_group_sizes_match_one_stream(tiny_gpu, lens, mode):
+    """Batches at the edges of the sizes that run as two sequence groups (4096
+    tokens in short sequences, 6144 otherwise, groups of at most 60 % of the
+    tokens and two thirds of the attention, 8192 whatever the groups): the same bits as on one stream."""
+    from semantica_gpu import _lib
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    toks = np.random.default_rng(len(lens)).integers(0, 4096, size=int(off[-1])).astype(np.int32)
+    say(f"sequence groups: {len(lens)} sequences, {off[-1]} tokens, {mode}")
+    tiny_gpu.set_attention_mode(_lib.SG_ATTN_EXACT if mode == "exact" else _lib.SG_ATTN_FAST)
+    try:
+        y = tiny_gpu.forward_packed(toks, off, 768)
+        tiny_gpu.profile_enable(True)
+        y1 = tiny_gpu.forward_packed(toks, off, 768)
+    finally:
+        tiny_gpu.profile_enable(False)
+        tiny_gpu.set_attention_mode(_lib.SG_ATTN_FAST)
+    assert np.array_equal(y.view(np.uint32), y1.view(np.uint32))
+
+
+@pytest.mark.parametrize("mode", ["fast", "exact"])
 def test_short_sequence_fusions_match_unfused(full_gpu, mode):
     """Short sequences take fused launches.  When every sequence of a batch
     lies inside one 32-row workgroup of the row kernels, the post-norms
