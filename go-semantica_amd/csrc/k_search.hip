@@ -577,7 +577,8 @@ __global__ __launch_bounds__(64) void k_bf_stream(const float* __restrict__ scor
 //   4. k_bf_top: selects the exact top k of those scores.
 // eps bounds |approximate - reference-order| score for every stored vector
 // (bf_prep: fp16 rounding of both operands, the accumulation on either side,
-// against the largest stored norm).  At least k vectors have an exact score of
+// against the largest stored norm; the operands are the reference's: whole
+// groups' codes as they are, the tail's clamped).  At least k vectors have an exact score of
 // T - eps or more, so the k-th best exact score v_k is at least that and every
 // vector that reaches v_k has an approximate score of at least T - 2 eps: it is
 // in a listed block, and the result is the exact top k.  A query for which this
@@ -888,7 +889,10 @@ __global__ __launch_bounds__(kPfThreads<CT>, 2) void k_bf_approx(const T* __rest
 #pragma unroll
               for (int u = 0; u < 8; u++) {
                 float v = u < R ? (float)tp[min(u, R - 1)] : 0.0f;
-                if constexpr (!BfElem<T>::kQuant) v = v * vscale;
+                if constexpr (BfElem<T>::kQuant)
+                  v = fmaxf(v, (float)BfElem<T>::kLo);  // bf_lut's clamp
+                else
+                  v = v * vscale;
                 tl[t][u] = lh == 0 ? (_Float16)v : (_Float16)0.0f;
               }
             }

@@ -388,3 +388,54 @@ def test_build_tiles_match_oracle(gpu_ctx, mode, dim, n):
     raw = search.Serializer().serialize(_build(gpu_ctx, ids, vecs, mode))
     want = o.bf_quantize(o.bf_normalize(vecs), mode)
     assert raw[20 + 4 * n:] == np.ascontiguousarray(want).tobytes()
+
+
+def _image(ids, data, mode):
+    """A serialized index (storage.go:14-92) of rows as given: codes and norms
+    that Build never stores, which a file may hold."""
+    n, dim = data.shape
+    head = struct.pack("<4sHHIB7x", b"BRUT", 1, dim, n, mode)
+    return head + np.ascontiguousarray(ids, np.int32).tobytes() + np.ascontiguousarray(data).tobytes()
+
+
+def _check_image(ctx, data, mode, queries, k, tag):
+    from semantica_gpu import search
+    ids = np.random.default_rng(k).permutation(2 * len(data))[:len(data)].astype(np.int32)
+    idx = search.Serializer().deserialize(ctx, _image(ids, data, mode))
+    try:
+        for normalized in (True, False):
+            gi, gd, gn = idx.search_batch(queries, k, normalized=normalized)
+            for q, x in enumerate(queries):
+                wi, wd = o.bf_search(data, mode, ids, x if normalized else o.bf_normalize(x), k)
+                assert gn[q] == len(wi), (tag, normalized, q)
+                assert np.array_equal(gi[q], wi), (tag, normalized, q)
+                assert np.array_equal(gd[q].view(np.uint32), wd.view(np.uint32)), (tag, normalized, q)
+    finally:
+        idx.close()
+
+
+@pytest.mark.parametrize("mode", MODES[1:])
+@pytest.mark.parametrize("dim,n,k", [(23, 9000, 1), (20, 9800, 3), (23, 13400, 10), (257, 9000, 1), (24, 9000, 1)])
+def test_prefilter_most_negative_codes(gpu_ctx, mode, dim, n, k):
+    """Deserialized indexes with the most negative code, which the tail clamps
+    to -127 / -32767 and the whole groups do not (quant.go:57-77,
+    dot_amd64.s).  k vectors whose tails are all most negative score below one
+    whose clamped tail and first element beat them, but above it by the codes
+    as they are."""
+    rng = np.random.default_rng(dim + k + mode)
+    dt, lo, unit = ((np.int8, -128, 1), (np.int16, -32768, 256))[mode - 1]
+    R = dim % 8
+    data = (rng.integers(-3, 4, (n, dim)) * unit).astype(dt)
+    data[rng.integers(0, n, n // 100), rng.integers(1, dim - R, n // 100)] = lo
+    at = 64 * 8 * (1 + np.arange(k)) + 5  # one per block, the blocks eight apart
+    best = 64 * 8 * (k + 2) + 9
+    data[at, dim - R:] = lo
+    data[at, 0] = -np.arange(k) * unit
+    data[best, dim - R:] = lo + 1
+    data[best, 0] = unit
+    q = (1e-3 * rng.standard_normal((3, dim))).astype(np.float32)
+    q[0, 0] = 0.5
+    q[0, dim - R:] = -1.0
+    q[1, dim - R:] = 1.0
+    say(f"most negative codes mode={MODE_NAMES[mode]} dim={dim} k={k}")
+    _check_image(gpu_ctx, data, mode, q, k, "most negative codes")
