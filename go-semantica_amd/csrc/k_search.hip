@@ -583,8 +583,9 @@ __global__ __launch_bounds__(64) void k_bf_stream(const float* __restrict__ scor
 // vector that reaches v_k has an approximate score of at least T - 2 eps: it is
 // in a listed block, and the result is the exact top k.  A query for which this
 // does not decide -- a tie straddling the k-th place, more than `cap` listed
-// blocks, a query that is zero, tiny, huge or not finite -- is flagged, and the
-// caller runs it through bf_score / bf_select.
+// blocks, a query that is zero, tiny, huge or not finite, scores that could leave
+// float32's normal range (kPfScoreLeast) -- is flagged, and the caller runs it
+// through bf_score / bf_select.
 // 64 queries x 10^6 x 768 int8, top 10, MI355X: 151 us for step 1 (5.1 TB/s, the
 // rate of a large copy) and 76 for the rest, against 2796 for the reference-order
 // scores of every pair and 870 for selecting among them.
@@ -592,6 +593,13 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kPfBlock = sgk::kBfBlock;  // vectors per block: two 32-row MFMA tiles
+// Least and largest product of the query's norm and the largest stored one.  No
+// partial sum of the reference's order exceeds it (Cauchy-Schwarz, and roundings
+// of under 1e-3 in all), so below 1e37 none is infinite.  What eps leaves out is
+// the absolute error of results below float32's normal range, 2^-150 each (2^-126
+// were they flushed to zero): at most 2 dim + 48 of them, 5.6e-35, against a
+// slack in eps of 2.4e-5 times the product, 2.4e-30 from 1e-25 on.
+constexpr float kPfScoreLeast = 1.0e-25f, kPfScoreMost = 1.0e37f;
 // Threads per workgroup: two column tiles' fragments fill much of the LDS (one
 // workgroup per CU); one leaves room for several smaller workgroups, which
 // share a short index out more evenly.
@@ -785,9 +793,11 @@ __global__ __launch_bounds__(kPrepThreads) void k_bf_prep(float* __restrict__ qu
     const float rel = 4.8829e-4f * (exact_v ? 1.0f : 2.0f) + (float)(dim + 32) * 1.2e-7f +
                       (float)(dim / 8 + 24) * 6.0e-8f + 1.0e-6f;
     const float rd = sqrtf((float)dim) * 3.0e-8f;
+    const float unit = (1.0f / sc) * (1.0f / vunit);  // k_bf_approx's units to scores
+    const float most = xn * vnorm_s * unit;  // bounds |score|; 0 or infinite where unit leaves the range
     eps[2 * q] = 1.05f * (rel * xn * vnorm_s + rd * (xn + vnorm_s));
-    eps[2 * q + 1] = (1.0f / sc) * (1.0f / vunit);  // k_bf_approx's units to scores
-    flags[q] = ok ? 0 : 1;
+    eps[2 * q + 1] = unit;
+    flags[q] = ok && most >= kPfScoreLeast && most <= kPfScoreMost ? 0 : 1;
   }
   const int G = dim >> 3, R = dim & 7, ct = q >> 5, c = q & 31;
   const int ks_main = (G + 1) >> 1, ks = ks_main + (R ? 1 : 0);

@@ -439,3 +439,27 @@ def test_prefilter_most_negative_codes(gpu_ctx, mode, dim, n, k):
     q[1, dim - R:] = 1.0
     say(f"most negative codes mode={MODE_NAMES[mode]} dim={dim} k={k}")
     _check_image(gpu_ctx, data, mode, q, k, "most negative codes")
+
+
+@pytest.mark.parametrize("norm,query", [(1e10, 1e30), (1e18, 1e22), (1e7, 2e29), (1e-20, 1e-25), (1e-14, 1e-30),
+                                        (1e-16, 3e-26), (1e-20, 1e-20), (1e-10, 1e-10), (1e8, 1e8)])
+@pytest.mark.parametrize("dim", [16, 257])
+def test_prefilter_scores_outside_float32(gpu_ctx, norm, query, dim):
+    """Deserialized float32 indexes searched as given, where products leave
+    float32's range: scores that differ become +inf, or fall on a few steps
+    of the subnormal grid or on zero, and the reference resolves these ties
+    by stored order.  k strong vectors, weaker ones that tie with them, and
+    the rest negative."""
+    rng = np.random.default_rng(dim)
+    n, k = 14000, 10
+    data = np.zeros((n, dim), np.float32)
+    data[:, 0] = -norm * rng.uniform(0.5, 1.0, n)
+    data[:, dim - 1] = 1e-3 * norm
+    data[64 * (2 * np.arange(100) + 1) + 7, 0] = norm * rng.uniform(0.8, 0.97, 100)  # other blocks than the strong ones
+    data[64 * 4 * (3 + 2 * np.arange(k)) + 11, 0] = norm * rng.uniform(0.98, 1.0, k)
+    q = np.zeros((3, dim), np.float32)
+    q[0, 0] = query
+    q[1, 0] = query * 2.2
+    q[2, dim - 1] = query
+    say(f"score range dim={dim} norm={norm:g} query={query:g}")
+    _check_image(gpu_ctx, data, o.BF_F32, q, k, "score range")
