@@ -600,6 +600,12 @@ constexpr int kPfBlock = sgk::kBfBlock;  // vectors per block: two 32-row MFMA t
 // were they flushed to zero): at most 2 dim + 48 of them, 5.6e-35, against a
 // slack in eps of 2.4e-5 times the product, 2.4e-30 from 1e-25 on.
 constexpr float kPfScoreLeast = 1.0e-25f, kPfScoreMost = 1.0e37f;
+// Least stored norm.  k_bf_vnorm sums float32 squares, whose absolute error is
+// 2^-126 each at most where they underflow: 2.8e-35 over the 2304 dimensions a
+// prefiltered index has, 1.4e-5 of a norm of 1e-15 (its user allows for 1e-2).
+// Below, a vector of many tiny elements can seem shorter than one of few, and the
+// largest norm come out too small.  (Norms past 1.8e19 come out infinite.)
+constexpr float kPfNormLeast = 1.0e-15f;
 // Threads per workgroup: two column tiles' fragments fill much of the LDS (one
 // workgroup per CU); one leaves room for several smaller workgroups, which
 // share a short index out more evenly.
@@ -1524,7 +1530,7 @@ hipError_t approx_t(const void* grp, const void* tail, int N, int dim, float vsc
 bool bf_prefilter_ok(int N, int dim, int k, float vnorm) {
   const int nb = (N + kBfBlock - 1) / kBfBlock;
   return N <= (1 << 30) && dim >= 16 && (size_t)pf_ksteps(dim) * 1024 <= kBfPfLds && nb >= 2 * bf_prefilter_cap(k) &&
-         vnorm >= 1.0e-30f && vnorm <= 1.0e30f;
+         vnorm >= kPfNormLeast && vnorm <= 1.0e30f;
 }
 
 int bf_prefilter_queries(int dim) { return (size_t)pf_ksteps(dim) * 2048 <= kBfPfLds ? 64 : 32; }

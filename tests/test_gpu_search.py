@@ -463,3 +463,22 @@ def test_prefilter_scores_outside_float32(gpu_ctx, norm, query, dim):
     q[2, dim - 1] = query
     say(f"score range dim={dim} norm={norm:g} query={query:g}")
     _check_image(gpu_ctx, data, o.BF_F32, q, k, "score range")
+
+
+def test_prefilter_norms_below_float32_squares(gpu_ctx):
+    """Deserialized float32 vectors whose squares underflow: their norms
+    (3e-22, over 1024 dimensions) are ten times that of the one vector whose
+    single element's square does not.  The best vector rounds down to fp16 in
+    every element, the second best up, by nearly half a unit each."""
+    n, dim, k = 9000, 1024, 1
+    rng = np.random.default_rng(3)
+    data = (2e-25 * rng.standard_normal((n, dim))).astype(np.float32)
+    unit, h, t = 2.0 ** -77, 2.0 ** -11, 2.0 ** -20  # 6.6e-24
+    data[1000] = unit * (1 + h + t)
+    data[5000, :512] = unit * (1 + 3 * h - t)
+    data[5000, 512:] = unit * (1 + h - t)
+    data[7000] = 0.0
+    data[7000, 3] = 4e-23
+    q = np.stack([np.full(dim, 2.0 ** 66), rng.standard_normal(dim)]).astype(np.float32)
+    say("norms below float32 squares")
+    _check_image(gpu_ctx, data, o.BF_F32, q, k, "tiny norms")
