@@ -839,17 +839,17 @@ __global__ __launch_bounds__(kNT, 2) void k_attn_small(
 }
 
 // The fragments of already normed and rotated Q, K and of V in one launch: a
-// workgroup per 32-key tile and operand head (query heads, kv heads of K, of
-// V).  Q and K: a wave per 16-key subtile and half of the dims, lane l fragment
+// workgroup per operand head (query heads, kv heads of K, of V) and 32-key tile,
+// one row of workgroups (the grid's second dimension would end at 65535 heads).  Q and K: a wave per 16-key subtile and half of the dims, lane l fragment
 // lane l, so every store is 1 KB contiguous; pad keys repeat the last one.
 __global__ __launch_bounds__(sgd::kKvThreads) void k_qkv_split(
     const float* __restrict__ q, int ldq, const float* __restrict__ k, const float* __restrict__ v, int ldkv, int H,
     int HKV, const int32_t* __restrict__ seq_off, const int32_t* __restrict__ voff,
-    const sg_item* __restrict__ vtiles, _Float16* __restrict__ qf, _Float16* __restrict__ kf,
+    const sg_item* __restrict__ vtiles, int n_vtiles, _Float16* __restrict__ qf, _Float16* __restrict__ kf,
     _Float16* __restrict__ vf, int n_tiles) {
   __shared__ __attribute__((aligned(16))) float tv[kBK][sgd::kVtRowStride];
-  const sg_item t = vtiles[blockIdx.x];
-  const int y = blockIdx.y;
+  const sg_item t = vtiles[blockIdx.x % n_vtiles];
+  const int y = blockIdx.x / n_vtiles;
   if (y >= H + HKV) {  // workgroup-uniform
     sgd::v_split_tile(t, y - H - HKV, tv, v, ldkv, seq_off, voff, vf, n_tiles);
     return;
@@ -917,9 +917,11 @@ hipError_t qkv_split(const float* q, int ldq, const float* k, const float* v, in
                      const int32_t* seq_off, const int32_t* voff, const sg_item* vtiles, int n_vtiles, _Float16* qf,
                      _Float16* kf, _Float16* vf, int n_tiles, hipStream_t s) {
   if (n_vtiles <= 0) return hipSuccess;
-  if ((ldq & 3) || (ldkv & 3) || H <= 0 || HKV <= 0 || H + 2 * HKV > 65535) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_qkv_split, dim3(n_vtiles, H + 2 * HKV), dim3(sgd::kKvThreads), 0, s, q, ldq, k, v, ldkv, H, HKV,
-                     seq_off, voff, vtiles, qf, kf, vf, n_tiles);
+  if ((ldq & 3) || (ldkv & 3) || H < 0 || HKV <= 0) return hipErrorInvalidValue;
+  const int64_t nwg = (int64_t)n_vtiles * ((int64_t)H + 2 * (int64_t)HKV);
+  if (nwg > INT32_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_qkv_split, dim3((unsigned)nwg), dim3(sgd::kKvThreads), 0, s, q, ldq, k, v, ldkv, H, HKV, seq_off,
+                     voff, vtiles, n_vtiles, qf, kf, vf, n_tiles);
   return hipGetLastError();
 }
 

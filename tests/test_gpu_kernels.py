@@ -591,6 +591,31 @@ def test_attention_exact_bit_exact(gpu_ctx, oracle, lens, heads, nonfinite):
         assert clamped > 0
 
 
+def test_attention_head_counts(gpu_ctx):
+    """No query heads (nothing to write), and more operand heads than a launch
+    has workgroups in a grid's second dimension, each head the same bits as
+    alone in a launch of four."""
+    import torch
+    from semantica_gpu import kernels
+    rng = np.random.default_rng(22)
+    off = np.array([0, 2], np.int32)
+    say("attention without query heads")
+    q, k, v = (dev(rng.standard_normal((2, n)).astype(np.float32)) for n in (4, 256, 256))
+    out = torch.full((2, 256), 7.0, dtype=torch.float32, device="cuda")
+    kernels.attention(gpu_ctx, out, q, k, v, 0, 1, 256, off)
+    assert (host(out) == 7.0).all()
+    say("attention of 22000 heads")
+    H = 22000
+    q, k, v = (dev(rng.standard_normal((2, H * 256)).astype(np.float32)) for _ in range(3))
+    out = torch.empty_like(q)
+    kernels.attention(gpu_ctx, out, q, k, v, H, H, 256, off)
+    for h in (0, 1, 10923, H - 4):
+        one = slice(h * 256, (h + 4) * 256)
+        want = torch.empty((2, 1024), dtype=torch.float32, device="cuda")
+        kernels.attention(gpu_ctx, want, *(t[:, one].contiguous() for t in (q, k, v)), 4, 4, 256, off)
+        assert np.array_equal(host(out[:, one]).view(np.uint32), host(want).view(np.uint32)), h
+
+
 def test_attention_register_scores_match_spilling_launch(gpu_ctx):
     """The same sequences with and without a 600-key companion (which moves the
     launch to the kernel variant that spills scores past 512 keys) give
