@@ -1113,6 +1113,7 @@ constexpr int kRdRows = 6144, kLds8Rows = 12288, kGeluLdsRows = 4096;
 // gemm_q8_res_norm: the fused kernel from kResRows rows (below, gemm_q8 and
 // post_res_norm run as two launches).
 constexpr int kResRows = 8192;
+static_assert(kResRows >= kWaveRows, "row_max_form's launches take the next norm's maxima from post_res_norm");
 // Register-direct launches of at most kPipeTiles workgroups -- fewer than
 // two waves per SIMD, so the other waves cannot fill a wave's MFMA latency --
 // take the MFMA-ahead loop with a 3-stage ring (at M = 32: 4.8 vs 5.4 us for

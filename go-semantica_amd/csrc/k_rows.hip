@@ -362,7 +362,7 @@ __device__ __forceinline__ void store_codes_wave(const f32x4_t (&x)[NV], float i
 
 // ------------------------------------------------------ wave-per-row forms --
 //
-// The row kernels for launches of fewer than kWaveRows rows.  There a kernel's
+// The row kernels for launches of fewer than sgk::kWaveRows rows.  There a kernel's
 // time is the latency of one workgroup, not bandwidth: with 8 lanes per row a
 // lane carries 96 values of a 768-wide row through the elementwise work and
 // each norm makes 24 dependent LDS round trips, and 32 rows share a workgroup
@@ -377,7 +377,6 @@ __device__ __forceinline__ void store_codes_wave(const f32x4_t (&x)[NV], float i
 // and the embedding 17 -> 4 us at 509 rows.  The chains' eightfold VALU and
 // LDS work costs about 1.7 us per 1000 rows of post-norm, so the two forms
 // meet near 8192 rows, where the 8-lane groups fill every CU (256 workgroups).
-constexpr int kWaveRows = 8192;
 constexpr int kWaveWaves = kThreads / SG_WAVE;  // rows per workgroup
 
 // k_embed_norm (h stored, xn not; the row's max|xn| into rmax).

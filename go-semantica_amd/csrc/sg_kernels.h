@@ -74,6 +74,8 @@ hipError_t first_bad_token(const int32_t* tokens, int T, int vocab, int32_t* fir
 // (and the CSR seq_off) takes each sequence's maximum over its rows.  The
 // atomics on amax cost ~13 ns each, one after another (the sequences' maxima
 // share a cache line): with a wave per row they were most of the kernel.
+// The fused GEMM + post-norm writes only amax: it serves none of these launches.
+constexpr int kWaveRows = 8192;  // the form's launches have fewer rows
 bool row_max_form(int T, int d);
 // Embedding gather * sqrt(d) -> h; then RMSNorm(w) -> xn (stored when xn != null) and
 // per-sequence max|xn| -> amax.  A token outside [0, vocab) is read as token 0
