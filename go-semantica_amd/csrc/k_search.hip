@@ -803,7 +803,7 @@ __global__ __launch_bounds__(kPrepThreads) void k_bf_prep(float* __restrict__ qu
     const float most = xn * vnorm_s * unit;  // bounds |score|; 0 or infinite where unit leaves the range
     eps[2 * q] = 1.05f * (rel * xn * vnorm_s + rd * (xn + vnorm_s));
     eps[2 * q + 1] = unit;
-    flags[q] = ok && most >= kPfScoreLeast && most <= kPfScoreMost ? 0 : 1;
+    flags[q] = ok && most >= kPfScoreLeast && most <= kPfScoreMost ? 0 : sgk::kBfUnfit;
   }
   const int G = dim >> 3, R = dim & 7, ct = q >> 5, c = q & 31;
   const int ks_main = (G + 1) >> 1, ks = ks_main + (R ? 1 : 0);
@@ -1061,7 +1061,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restri
   if (threadIdx.x == 0) {
     eps[2 * q] = cut * eps[2 * q + 1];
     count[q] = cnt <= cap ? cnt : 0;
-    if (cnt > cap) flags[q] = 1;
+    if (cnt > cap) flags[q] = sgk::kBfOpen;
   }
 }
 
@@ -1208,7 +1208,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict_
   }
   const int n = count[q] * kPfBlock;
   if (flags[q] || n < k) {
-    if (threadIdx.x == 0) flags[q] = 1;
+    if (threadIdx.x == 0 && flags[q] == 0) flags[q] = sgk::kBfOpen;
     return;
   }
   const float* cs = cand + (int64_t)q * cap * kPfBlock;
@@ -1259,7 +1259,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict_
       }
     }
     __syncthreads();
-    if (threadIdx.x == 0 && tie) flags[q] = 1;
+    if (threadIdx.x == 0 && tie) flags[q] = sgk::kBfOpen;
     return;
   }
   auto key = [=](int i) {
@@ -1270,7 +1270,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict_
   int above, at;
   wg_select<3>(each_key(key, n), k, hist, T, above, at);
   if (above + at != k) {
-    if (threadIdx.x == 0) flags[q] = 1;
+    if (threadIdx.x == 0) flags[q] = sgk::kBfOpen;
     return;
   }
   if (threadIdx.x == 0) cnt = 0;

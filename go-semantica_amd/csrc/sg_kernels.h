@@ -292,6 +292,9 @@ constexpr size_t kBfPfLds = 144 << 10;  // LDS for the queries' fragments
 constexpr int bf_prefilter_cap(int k) { return 4 * k + 64; }  // listed blocks per query
 bool bf_prefilter_ok(int N, int dim, int k, float vnorm);
 int bf_prefilter_queries(int dim);  // queries per call
+// Why a query was not decided: the query itself is not one for the prefilter, or
+// the stored vectors leave it open (too many blocks, a tie at the k-th place).
+constexpr int kBfUnfit = 1, kBfOpen = 2;
 struct sg_bf_work {
   _Float16* qfrag;   // 64 x (dim rounded up to 32) + 1024
   float* eps;        // [nq][2]: the bound (then the score that the k best reach), its unit
@@ -301,7 +304,7 @@ struct sg_bf_work {
   float* cand;       // [nq][cap * kBfBlock]
   int32_t* out_idx;  // [nq][k]
   float* out_dist;   // [nq][k]
-  int32_t* flags;    // [nq]: 1 = not decided, run the query through bf_score / bf_select
+  int32_t* flags;    // [nq]: not 0 = not decided, run the query through bf_score / bf_select
 };
 // queries [nq][dim]: normalized in place when `normalize` (bf_normalize's
 // arithmetic).  out_idx / out_dist as bf_select's, for the unflagged queries.

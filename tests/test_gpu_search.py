@@ -482,3 +482,22 @@ def test_prefilter_norms_below_float32_squares(gpu_ctx):
     q = np.stack([np.full(dim, 2.0 ** 66), rng.standard_normal(dim)]).astype(np.float32)
     say("norms below float32 squares")
     _check_image(gpu_ctx, data, o.BF_F32, q, k, "tiny norms")
+
+
+def test_prefilter_backs_off_from_crowded_collections(gpu_ctx):
+    """Searches of one index in a row, of queries that the prefilter leaves open
+    (near-duplicates) and ones that it decides, alone and in batches of several
+    passes, so that searches with it and without it follow on each other."""
+    rng = np.random.default_rng(17)
+    n, dim, k = 20000, 64, 10
+    base = rng.standard_normal(dim)
+    vecs = rng.standard_normal((n, dim)).astype(np.float32)
+    vecs[:15000] = base + 1e-5 * rng.standard_normal((15000, dim))
+    ids = rng.permutation(n).astype(np.int32)
+    idx = _build(gpu_ctx, ids, vecs, MODES[0])
+    near = (base + 0.05 * rng.standard_normal((70, dim))).astype(np.float32)
+    far = (-base + 0.5 * rng.standard_normal((70, dim))).astype(np.float32)
+    say("back-off: crowded and clear queries in turn")
+    for i, q in enumerate([near[:1], near[1:2], near[2:3], far[:1], far[1:2], near, far, np.zeros((1, dim), np.float32),
+                           near[:5], far[:5], far, np.concatenate([near[:6], far[:2]]), far[2:4]]):
+        _check(idx, vecs, ids, MODES[0], q, k, False, i)
