@@ -365,32 +365,40 @@ def test_sequence_group_sizes_match_one_stream(tiny_gpu, lens, mode):
 
 @pytest.mark.parametrize("mode", ["fast", "exact"])
 def test_short_sequence_fusions_match_unfused(full_gpu, mode):
-    """Short sequences take fused launches.  When every sequence of a batch
-    lies inside one 32-row workgroup of the row kernels, the post-norms
-    quantize the next GEMM operand themselves (k_post_res_norm_q), and when
-    every sequence is one attention work item (at most 32 tokens with 3 query
-    heads) the attention kernel quantizes its own output (fast mode).  A
-    sequence's embedding does not depend on the rest of its batch, so the same
-    sequences embedded in batches that take both fused forms, only the
-    attention one (a sequence crosses a 32-row boundary), or neither (a
-    40-token sequence crosses it and needs two attention items) agree bit for
-    bit, over 24 layers at full size."""
+    """Short sequences take a fused launch: when every sequence of a batch is one
+    attention work item (at most 32 tokens with 3 query heads), the attention
+    kernel of launches of more than 64 items (k_attn_rs) quantizes its own
+    output (fast mode).  Up to 64 items k_attn_small leaves chunk maxima to the
+    quantizer, and beside a 40-token sequence (two items) k_attn_rs leaves the
+    sequences' maxima, its items run in halves below 256.  A sequence's
+    embedding does not depend on the rest of its batch, so the same sequences
+    embedded in all of these agree bit for bit, over 24 layers at full size."""
     from semantica_gpu import _lib
     rng = np.random.default_rng(31)
     x1, x2, x3, x40 = (rng.integers(2, 262144, size=n).astype(np.int32) for n in (32, 7, 19, 40))
-    batches = {
-        "fused (one 32-token sequence)": [x1],
-        "fused (7 + 19 tokens in one row block)": [x2, x3],
-        "fused (four sequences in row blocks)": [x1, x2, x3, x2[:5]],
-        "attention-fused only (7 + 32: a sequence crosses row 32)": [x2, x1, x3],
-        "unfused (a 40-token sequence first)": [x40, x1, x2, x3],
+    lens = [1, 2, 7, 15, 16, 17, 31, 32] + rng.integers(1, 33, 62).tolist()
+    many = [rng.integers(2, 262144, size=n).astype(np.int32) for n in lens]
+    ones = [rng.integers(2, 262144, size=1).astype(np.int32) for _ in range(190)]
+    batches = {  # name: sequences, attention items
+        "small form (one 32-token sequence)": ([x1], 1),
+        "small form (7 + 19 tokens)": ([x2, x3], 2),
+        "small form (four sequences)": ([x1, x2, x3, x2[:5]], 4),
+        "small form (7 + 32: a sequence crosses row 32)": ([x2, x1, x3], 3),
+        "small form (a 40-token sequence first)": ([x40, x1, x2, x3], 5),
+        "small form (half of the short ones)": (many[:35], 35),
+        "small form (the other half)": (many[35:], 35),
+        "fused": (many, 70),
+        "fused, more items than CUs": (many + ones, 260),
+        "unfused, items in halves": (many + [x40], 72),
+        "unfused, whole items": (many + [x40] + ones, 262),
     }
     full_gpu.set_attention_mode(_lib.SG_ATTN_EXACT if mode == "exact" else _lib.SG_ATTN_FAST)
     try:
         got = {}
-        for name, seqs in batches.items():
+        for name, (seqs, items) in batches.items():
             toks = np.concatenate(seqs)
             off = np.concatenate([[0], np.cumsum([len(q) for q in seqs])]).astype(np.int32)
+            assert items == sum(-(-3 * -(-len(q) // 16) // 8) for q in seqs) and len(toks) < 4096  # one group
             say(f"short-sequence fusions ({mode}): {name}")
             y = full_gpu.forward_packed(toks, off, 768)
             for q, e in zip(seqs, y):
