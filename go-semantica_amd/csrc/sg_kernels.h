@@ -291,6 +291,16 @@ constexpr int kBfBlock = 64;            // vectors per block
 constexpr size_t kBfPfLds = 144 << 10;  // LDS for the queries' fragments
 constexpr int bf_prefilter_cap(int k) { return 4 * k + 64; }  // listed blocks per query
 bool bf_prefilter_ok(int N, int dim, int k, float vnorm);
+// A query's listed blocks and candidates grow with k and are one workgroup's
+// work at two of the four steps, so few queries for many vectors are better off
+// with the full path's grid-wide passes.  us a search, full / prefiltered:
+//   10^6 x 768 int8, 1 query    k 500 284 / 243   700 290 / 267   1000 306 / 338
+//   4,000,000 x 64 int8, 1      k 500 213 / 158   1000 237 / 249  4000 440 / 646
+//   300,000 x 256 float32, 1    k 500 153 / 142
+//   4,000,000 x 256 float32, 4  k 1000 1229 / 1074 4000 1942 / 2085
+//   10^6 x 256 float32, 16      k 1000 1290 / 1125; 4,000,000: k 4000 5752 / 4929
+constexpr int kBfMostK = 512;    // k up to here for any number of queries
+constexpr int kBfManyQueries = 16;  // any k from this many on
 int bf_prefilter_queries(int dim);  // queries per call
 // Why a query was not decided: the query itself is not one for the prefilter, or
 // the stored vectors leave it open (too many blocks, a tie at the k-th place).

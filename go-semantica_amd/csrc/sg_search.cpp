@@ -393,7 +393,7 @@ int sg_index_search(sg_index* x, const float* queries, int32_t n_queries, int32_
   }
   SG_HIP(hipSetDevice(sgi::ctx_device(x->ctx)));
   hipStream_t s = sgi::ctx_stream(x->ctx, stream);
-  bool pre = sgk::bf_prefilter_ok(N, dim, k, x->vnorm);
+  bool pre = sgk::bf_prefilter_ok(N, dim, k, x->vnorm) && (k <= sgk::kBfMostK || n_queries >= sgk::kBfManyQueries);
   if (pre && x->pf_wait > 0) {
     x->pf_wait--;
     pre = false;

@@ -501,3 +501,19 @@ def test_prefilter_backs_off_from_crowded_collections(gpu_ctx):
     for i, q in enumerate([near[:1], near[1:2], near[2:3], far[:1], far[1:2], near, far, np.zeros((1, dim), np.float32),
                            near[:5], far[:5], far, np.concatenate([near[:6], far[:2]]), far[2:4]]):
         _check(idx, vecs, ids, MODES[0], q, k, False, i)
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_prefilter_large_k(gpu_ctx, mode):
+    """k at the edge of what few queries are prefiltered for, and past it with
+    few and with many: selections of more candidates than are ranked against
+    each other."""
+    rng = np.random.default_rng(23 + mode)
+    n, dim = 320000, 17
+    vecs = rng.standard_normal((n, dim)).astype(np.float32)
+    ids = rng.permutation(n).astype(np.int32)
+    idx = _build(gpu_ctx, ids, vecs, mode)
+    q = rng.standard_normal((16, dim)).astype(np.float32)
+    for nq, k in ((1, 512), (3, 512), (1, 513), (16, 600)):
+        say(f"large k mode={MODE_NAMES[mode]} q={nq} k={k}")
+        _check(idx, vecs, ids, mode, q[:nq], k, False, (nq, k))
