@@ -84,18 +84,6 @@ int seq_groups(int S, int G) {
   return (chunks + sgk::kAttnChunks - 1) / sgk::kAttnChunks;
 }
 
-// Fills `host` with [row_seq | row_pos | row_key | row_slot | seq_off | voff | items | vtiles |
-// spill_off] and
-// copies it to `dev` on stream s, asynchronously: kernels launched on s after
-// this see the metadata, and the next stage_meta waits for the copy before it
-// rewrites `host`.
-// G: query heads per kv head.
-//
-// Workgroup order.  Workgroup i of a launch runs on XCD i % 8 (the dispatcher
-// deals workgroups round-robin over the eight XCDs, each with its own L2), so
-// sequences are binned to XCDs (largest first, onto the least-loaded bin) and
-// the list interleaves the bins: all workgroups of a sequence then share one
-// L2 copy of its K and V^T.
 // The gate/up GEMM folds every workgroup's max|g| into its sequences' by atomics,
 // 13 ns each, one after another within a cache line: 13 sequences of 5-60 tokens
 // in one line made the launch 17.9 us, a line per sequence 16.3.
@@ -103,7 +91,20 @@ constexpr int kSlot = 32;  // floats
 constexpr int kAttnLptItems = 512;  // two rounds of attention workgroups on 256 CUs
 constexpr int kAttnCus = 256;
 
-int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev, hipStream_t s, Meta& m) {
+// Fills `host` with [row_seq | row_pos | row_key | row_slot | seq_off | voff |
+// items | vtiles | spill_off] and copies it to `dev` on stream s,
+// asynchronously: kernels launched on s after this see the metadata, and the
+// next stage_meta waits for the copy before it rewrites `host`.
+// G: query heads per kv head.  model: for a model's forward; the kernel seam has
+// no use for row_key and row_slot, which take the host 14 us at 32,768 tokens.
+//
+// Workgroup order.  Workgroup i of a launch runs on XCD i % 8 (the dispatcher
+// deals workgroups round-robin over the eight XCDs, each with its own L2), so
+// sequences are binned to XCDs (largest first, onto the least-loaded bin) and
+// the list interleaves the bins: all workgroups of a sequence then share one
+// L2 copy of its K and V^T.
+int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev, hipStream_t s, Meta& m,
+               bool model = false) {
   constexpr int kXcd = 8;
   const int T = off[n_seq];
   int n_items = 0, n_vt = 0;
@@ -115,7 +116,8 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
     n_spill += (int64_t)seq_groups(S, G) * sgk::attention_spill_tiles(S);
   }
   if (n_spill > INT32_MAX) return fail(SG_ERR_INVALID, "batch too large for the attention spill layout");
-  const size_t bytes = sizeof(int32_t) * ((size_t)4 * T + 2 * (n_seq + 1)) +
+  const size_t per_row = model ? 4 : 2;
+  const size_t bytes = sizeof(int32_t) * (per_row * T + 2 * (n_seq + 1)) +
                        sizeof(sg_item) * ((size_t)n_items + n_vt) + sizeof(int32_t) * (size_t)n_seq + 64;
   SG_TRY(host.ensure(bytes));
   SG_TRY(dev.ensure(bytes));
@@ -124,7 +126,7 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
   int32_t* rp = rs + T;
   int32_t* rk = rp + T;
   int32_t* rl = rk + T;
-  int32_t* so = rl + T;
+  int32_t* so = rs + per_row * T;
   int32_t* vo = so + n_seq + 1;
   sg_item* it = reinterpret_cast<sg_item*>(vo + n_seq + 1);
   sg_item* vt = it + n_items;
@@ -138,9 +140,12 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
     for (int r = off[i]; r < off[i + 1]; r++) {
       rs[r] = i;
       rp[r] = r - off[i];
-      rk[r] = vo[i] + r - off[i];
-      rl[r] = i * kSlot;
     }
+    if (model)
+      for (int r = off[i]; r < off[i + 1]; r++) {
+        rk[r] = vo[i] + r - off[i];
+        rl[r] = i * kSlot;
+      }
     for (int k0 = 0; k0 < S; k0 += 32) vt[nv++] = sg_item{i, k0};
     sp[i] = ns;
     ns += seq_groups(S, G) * sgk::attention_spill_tiles(S);
@@ -211,9 +216,9 @@ int stage_meta(const int32_t* off, int n_seq, int G, HostBuf& host, DevBuf& dev,
   m.Tp = vo[n_seq];
   m.row_seq = d;
   m.row_pos = d + T;
-  m.row_key = d + 2 * (size_t)T;
-  m.row_slot = d + 3 * (size_t)T;
-  m.seq_off = d + 4 * (size_t)T;
+  m.row_key = model ? d + 2 * (size_t)T : nullptr;
+  m.row_slot = model ? d + 3 * (size_t)T : nullptr;
+  m.seq_off = d + per_row * T;
   m.voff = m.seq_off + n_seq + 1;
   m.items = reinterpret_cast<sg_item*>(m.voff + n_seq + 1);
   m.vtiles = m.items + n_items;
@@ -857,7 +862,7 @@ int forward_device_locked(sg_model* m, const int32_t* d_tokens, const int32_t* o
     sub.resize(n + 1);
     for (int i = 0; i <= n; i++) sub[i] = off[b[g] + i] - off[b[g]];
     Lane& w = m->lanes[g];
-    SG_TRY(stage_meta(sub.data(), n, GQ, w.meta_h, w.meta_d, st[g], meta[g]));
+    SG_TRY(stage_meta(sub.data(), n, GQ, w.meta_h, w.meta_d, st[g], meta[g], true));
     SG_TRY(ensure_workspace(m, w, meta[g]));
   }
   int rc = SG_OK;
