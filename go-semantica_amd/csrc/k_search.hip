@@ -1004,18 +1004,19 @@ __device__ __forceinline__ void wg_select(F visit, int k, uint32_t* hist, uint32
   at = in_bin;
 }
 
-// visit of n keys key(i), i < n, the loads of kKeyBatch of a thread's keys in
-// flight together (a workgroup alone on its CU waits for each of them otherwise).
+// visit of n keys key(i), i < n, the loads of B of a thread's keys in flight
+// together (a workgroup alone on its CU waits for each of them otherwise; where a
+// thread has few keys, the loads past the last one cost more than that).
 constexpr int kKeyBatch = 8;
-template <typename K>
+template <int B, typename K>
 __device__ __forceinline__ auto each_key(K key, int n) {
   return [=](auto f) {
-    for (int i0 = 0; i0 < n; i0 += kKeyBatch * kTopThreads) {
-      uint32_t u[kKeyBatch];
+    for (int i0 = 0; i0 < n; i0 += B * kTopThreads) {
+      uint32_t u[B];
 #pragma unroll
-      for (int b = 0; b < kKeyBatch; b++) u[b] = key(min(i0 + b * kTopThreads + (int)threadIdx.x, n - 1));
+      for (int b = 0; b < B; b++) u[b] = key(min(i0 + b * kTopThreads + (int)threadIdx.x, n - 1));
 #pragma unroll
-      for (int b = 0; b < kKeyBatch; b++) {
+      for (int b = 0; b < B; b++) {
         if (i0 + b * kTopThreads >= n) break;  // workgroup-uniform
         f(i0 + b * kTopThreads + (int)threadIdx.x < n, u[b]);
       }
@@ -1048,7 +1049,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_blocks(const float* __restri
   // for a quarter of the keys.  Its low bits are zero, and the cut's own
   // rounding is covered by eps' slack.
   wg_select<2>(
-      each_key(
+      each_key<1>(
           [=](int i) {
             float m = bm[4 * i];
 #pragma unroll
@@ -1286,7 +1287,7 @@ __global__ __launch_bounds__(kTopThreads) void k_bf_top(const float* __restrict_
   auto key = [=](float d) { return d >= low ? bf_key(d) : 0u; };
   uint32_t T;
   int above, at;
-  wg_select<3>(each_key([=](int i) { return key(cs[i]); }, n), k, hist, T, above, at);
+  wg_select<3>(each_key<kKeyBatch>([=](int i) { return key(cs[i]); }, n), k, hist, T, above, at);
   if (above + at != k) {
     if (threadIdx.x == 0) flags[q] = sgk::kBfOpen;
     return;
