@@ -620,10 +620,8 @@ __global__ __launch_bounds__(kThreads) void k_gelu_mul(float* __restrict__ g, in
 }
 
 
-// Per-row max|x| folded into the row's sequence maximum (absMaxScalar,
-// quantize.go:80-90, over a whole sequence).
-// The sequences' max|x| into amax (zeroed before), a wave per kMaxRows rows with
-// the loads of 5 x 64 columns' float4s of all its rows in flight.  One atomic
+// The sequences' max|x| (absMaxScalar, quantize.go:80-90, over a whole sequence)
+// into amax (zeroed before), a wave per kMaxRows rows with the loads of 5 x 64 columns' float4s of all its rows in flight.  One atomic
 // per workgroup of one sequence: the sequences' maxima share a cache line and
 // its atomics go one after another, 13 ns each (one per row made 2048 rows of
 // 768 take 26 us, more than the quantization itself).
@@ -852,15 +850,14 @@ hipError_t embed_only(const int32_t* tokens, int T, const int8_t* eq, const floa
 }
 
 hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, const float* amax,
-                    int8_t* q8, int a_rows, int8_t* i8, float* row_scale, hipStream_t s, const float* cmax,
+                    int8_t* q8, int a_rows, float* row_scale, hipStream_t s, const float* cmax,
                     const int32_t* seq_off, int H) {
   if (rows <= 0) return hipSuccess;
-  if (cmax && (!seq_off || H <= 0 || !q8 || rows >= kWaveRows || (reinterpret_cast<uintptr_t>(x) & 15) ||
+  if (cmax && (!seq_off || H <= 0 || rows >= kWaveRows || (reinterpret_cast<uintptr_t>(x) & 15) ||
                (cols != 256 && cols != 512 && cols != 768 && cols != 1024)))
     return hipErrorInvalidValue;  // the wave form's launches
-  if (cols % 4 || ldx % 4 || (!q8 && !i8)) return hipErrorInvalidValue;
-  if (q8 && (cols % 32 || a_rows < rows)) return hipErrorInvalidValue;
-  if (q8 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+  if (ldx % 4 || !q8 || cols % 32 || a_rows < rows) return hipErrorInvalidValue;
+  if ((reinterpret_cast<uintptr_t>(x) & 15) == 0) {
     // Fewer rows than kWaveRows: latency-bound, a wave per row.
     const bool small = rows < kWaveRows;
     switch (cols) {  // the widths the forward quantizes: attention output, hidden, FFN
@@ -880,7 +877,7 @@ hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* 
     }
   }
   hipLaunchKernelGGL(k_quantize, dim3(blocks_for(rows, kThreads / SG_WAVE)), dim3(kThreads), 0, s, x, ldx, rows, cols,
-                     row_seq, amax, q8, a_rows, q8 ? nullptr : i8, row_scale, 0, nullptr);
+                     row_seq, amax, q8, a_rows, nullptr, row_scale, 0, nullptr);
   return hipGetLastError();
 }
 

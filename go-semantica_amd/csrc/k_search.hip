@@ -933,10 +933,10 @@ __global__ __launch_bounds__(kPfThreads<CT>, 2) void k_bf_approx(const T* __rest
 }
 
 // The value T of a workgroup's radix select over the keys that visit(f) hands to
-// f(valid, key), a whole wave at a time: the keys'
-// top bits (kSelBits0 + kSelBits1 [+ kSelBits2]) of the k-th largest key with
-// the rest zero; above = keys above T's bin, at = keys in it.  hist: 2048 + 64
-// words of LDS.  Every thread of the workgroup calls this.
+// f(valid, key), a whole wave at a time: the k-th largest key's top 11 bits a
+// pass (10 in the third) with the rest zero; above = keys above T's bin, at =
+// keys in it.  hist: 2048 + 64 words of LDS.  Every thread of the workgroup calls
+// this.
 constexpr int kTopThreads = 1024;
 template <int PASSES, typename F>
 __device__ __forceinline__ void wg_select(F visit, int k, uint32_t* hist, uint32_t& T, int& above, int& at) {

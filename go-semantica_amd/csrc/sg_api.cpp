@@ -579,7 +579,7 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
     return sgk::norm_quantize(h, w, eps, T, d, meta.row_seq, am, a8, ar, sx, s, rmax, meta.seq_off);
   };
   auto quant = [&](const float* x, int cols, float* am, const float* cmax = nullptr) {
-    return sgk::quantize(x, cols, T, cols, meta.row_seq, am, a8, ar, nullptr, sx, s, cmax, meta.seq_off, c.num_heads);
+    return sgk::quantize(x, cols, T, cols, meta.row_seq, am, a8, ar, sx, s, cmax, meta.seq_off, c.num_heads);
   };
   auto tap = [&](float* dst, const float* src, int l, int cols) {
     return hipMemcpyAsync(dst + (size_t)l * T * cols, src, sizeof(float) * (size_t)T * cols, hipMemcpyDeviceToDevice,
@@ -677,7 +677,7 @@ int run_forward(sg_model* m, Lane& w, const int32_t* d_tokens, const Meta& meta,
     SG_LAUNCH(SG_K_GEMM, gemm_ops(2 * ff, d),
               sgk::gemm_q8_gelu(a8, ar, ly.wgu, ly.sgu, sx, g, T, ff, d, meta.row_slot, gsite(l), s, true));
     SG_LAUNCH(SG_K_QUANTIZE, quant_bytes(ff),
-              sgk::quantize(g, ff, T, ff, meta.row_slot, gsite(l), a8, ar, nullptr, sx, s));
+              sgk::quantize(g, ff, T, ff, meta.row_slot, gsite(l), a8, ar, sx, s));
     const bool last = l + 1 == L;
     const float* w_next = last ? m->out_norm : m->layers[l + 1].attn_norm;
     if (sgk::gemm_res_norm_fused(T, d, ly.post_ffw, w_next)) {

@@ -392,8 +392,6 @@ __device__ __forceinline__ void sg_wave_tile_put(const f32x4_t (&x)[NV], float* 
 }
 
 // 1 / rms of the row in `tile` (written by this wave; the LDS operations of a
-// wave complete in issue order), as sg_rmsnorm8 forms it.
-// 1 / rms of the row in `tile` (written by this wave; the LDS operations of a
 // wave complete in issue order), as sg_rmsnorm8 forms it, in every lane.
 template <int NV>
 __device__ __forceinline__ float sg_wave_inv_rms(const float* tile, int lane, float eps) {

@@ -84,13 +84,13 @@ hipError_t embed_norm(const int32_t* tokens, int T, const int8_t* eq, const floa
                       float sqrt_d, const float* w, float eps, const int32_t* row_seq, float* h, float* xn,
                       float* amax, int32_t* err, hipStream_t s, float* rmax = nullptr);
 // Per-sequence symmetric quantization of x[rows][cols] (stride ldx) using amax[row_seq[r]].
-// Writes the int8 codes block-major q8[cols/32][a_rows][32] (q8 != null, the GEMM
-// operand) or row-major i8[rows][cols] (q8 == null), and row_scale[rows].
-// cmax (with the CSR seq_off, H heads; q8 and rows < the row_max_form limit):
+// Writes the int8 codes block-major q8[cols/32][a_rows][32] (the GEMM operand)
+// and row_scale[rows].
+// cmax (with the CSR seq_off, H heads; rows < kWaveRows):
 // the sequence's maximum is taken over attention_small's chunk maxima instead
 // of amax.
 hipError_t quantize(const float* x, int ldx, int rows, int cols, const int32_t* row_seq, const float* amax,
-                    int8_t* q8, int a_rows, int8_t* i8, float* row_scale, hipStream_t s, const float* cmax = nullptr,
+                    int8_t* q8, int a_rows, float* row_scale, hipStream_t s, const float* cmax = nullptr,
                     const int32_t* seq_off = nullptr, int H = 0);
 // xn = RMSNorm(h; w) recomputed row by row exactly as post_res_norm / embed_norm
 // formed it, quantized with amax[row_seq[r]] into the block-major int8 GEMM
