@@ -269,20 +269,15 @@ __device__ __forceinline__ void attn_rs_item(
   const int qr = r0 + min(qrow, S - 1);
 
   // ---- copies ----
-  // Wave w's kCopies copies of an item: pieces kCopies * w .. of the tile.  For keys
-  // past the sequence's end a lane copies the last one's fragment, which its
-  // neighbours read as well (their scores are masked below; V's pad keys are
-  // zeros): reading the pad keys' own, whatever the buffer holds, made a forward of
-  // 4000 one-token sequences 8.75 ms, 8.45 now.
+  // Wave w's kCopies copies of an item: pieces kCopies * w .. of the tile.  Keys past
+  // the sequence's end hold whatever the buffer held; their scores are masked
+  // below (V's pad keys are zeros).
   const int64_t tile0 = (int64_t)kvh * n_tiles + (vo >> 5);
   const i32x4_t rk = sg_raw_rsrc(kf + tile0 * sgd::kFragTile);
   const i32x4_t rv = sg_raw_rsrc(vf + tile0 * sgd::kFragTile);
   constexpr int kCopies = 32 / W;
-  const int key_last = max(S - 1 - (nt - 1) * kBK - kQW * (w / (W / 2)), 0);  // in the wave's subtile of the last tile
-  const uint32_t vlast = 16u * (lane - ln + min(ln, key_last));
-  auto copy_tile = [&](uint32_t dst, bool isk, int tile) {
+  auto copy_tile = [&](uint32_t dst, bool isk, int tile, uint32_t voff) {
     const uint32_t soff = (uint32_t)tile * kTileBytes + (uint32_t)w * (kCopies * 1024u);
-    const uint32_t voff = isk && tile == nt - 1 ? vlast : 16u * lane;
 #pragma unroll
     for (int i = 0; i < kCopies; i++) sg_lds_copy16(dst + 1024u * i, voff, isk ? rk : rv, soff + 1024u * i);
   };
@@ -299,10 +294,10 @@ __device__ __forceinline__ void attn_rs_item(
   const i32x4_t rsp = sg_raw_rsrc(wspill);
   const int last = 2 * nt - 1;
   auto carries = [&](int src) { return SPILL && src >= nt + kRegTiles - 1 && src < last; };
-  auto issue = [&](int item) {
+  auto issue_at = [&](int item, uint32_t voff) {
     const int src = item < last ? item : last;
     const uint32_t dst = (uint32_t)(uintptr_t)(lds_ptr)(lds + ((unsigned)item % kRing) * kTileBytes + w * (kCopies * 1024));
-    copy_tile(dst, src < nt, src < nt ? src : src - nt);
+    copy_tile(dst, src < nt, src < nt ? src : src - nt, voff);
     if (carries(src)) {
       const uint32_t sd = (uint32_t)(uintptr_t)(lds_ptr)(slds + ((unsigned)item % kRing) * (W * 2048) + w * 2048);
       const uint32_t so = (uint32_t)((src - nt + 1 - kRegTiles) * kScoreBytes + wi * 2048);
@@ -310,6 +305,7 @@ __device__ __forceinline__ void attn_rs_item(
       sg_lds_copy16(sd + 1024u, 16u * lane + 1024u, rsp, so);
     }
   };
+  auto issue = [&](int item) { issue_at(item, 16u * lane); };
   // Wait until item i has landed, item i + 1 (kCopies copies per wave, or two more
   // when it carries scores) may still be in flight.
   auto wait_item = [&](int i) {
@@ -318,7 +314,11 @@ __device__ __forceinline__ void attn_rs_item(
     else
       sg_wait_vmcnt<kCopies>();
   };
-  issue(0);
+  // A sequence of one tile (item 0 is all its K): for its pad keys a lane copies the
+  // last key's fragment, which its neighbours read as well.  Reading the pad keys'
+  // own made a forward of 4000 one-token sequences 8.75 ms, 8.45 now.
+  const int key_last = nt == 1 ? max(S - 1 - kQW * (w / (W / 2)), 0) : kQW;  // in the wave's 16-key subtile
+  issue_at(0, 16u * (lane - ln + min(ln, key_last)));
   issue(1);
   half8_t bqh[kHD / 32], bql[kHD / 32];
   // The Q prologue's LDS tiles sit in stage 2, which no copy touches before
