@@ -1416,6 +1416,44 @@ int sg_qknorm_rope(sg_ctx* ctx, float* q, int32_t ldq, float* k, int32_t ldk, co
   return SG_OK;
 }
 
+}  // extern "C"
+
+namespace {
+constexpr size_t kSeamSplitBytes = size_t(4) << 30;  // split operands of one piece of an sg_attention call
+
+// sg_attention of some sequences, all of whose operands are split at once.
+int attention_piece(sg_ctx* ctx, float* out, const float* q, int ldq, const float* k, const float* v, int ldkv, int H,
+                    int HKV, const int32_t* off, int n_seq, hipStream_t s) {
+  constexpr int kHd = 256;
+  Meta meta;
+  SG_TRY(stage_meta(off, n_seq, H / HKV, ctx->meta_h, ctx->meta_d, s, meta));
+  const float scale = 1.0f / (float)std::sqrt((double)kHd);
+  const size_t qd = (size_t)H * kHd, kvd = (size_t)HKV * kHd, Tp = (size_t)meta.Tp;
+  const size_t split_bytes = (2 * sizeof(_Float16) * (qd + 2 * kvd) * Tp + 255) & ~(size_t)255;
+  const bool small = sgk::attn_small_form(meta.n_items, HKV, meta.max_len);
+  SG_TRY(ctx->split.ensure(split_bytes + (small ? 0 : (size_t)HKV * meta.spill_total * sgk::kAttnSpillTileBytes)));
+  SG_TRY(gemm_scratch_begin(ctx, s));  // after the asynchronous GEMM calls of this context
+  _Float16* qf = ctx->split.as<_Float16>();
+  _Float16* kf = qf + 2 * qd * Tp;
+  _Float16* vf = kf + 2 * kvd * Tp;
+  const int n_tiles = meta.Tp / 32;
+  SG_HIP(sgk::qkv_split(q, ldq, k, v, ldkv, H, HKV, meta.seq_off, meta.voff, meta.vtiles, meta.n_vtiles, qf, kf, vf,
+                        n_tiles, s));
+  if (small) {
+    SG_HIP(sgk::attention_small(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items, meta.n_items, H,
+                                HKV, kHd, scale, nullptr, meta.max_len, s));
+    return SG_OK;
+  }
+  const sg_attn_spill spill{reinterpret_cast<float*>(ctx->split.as<unsigned char>() + split_bytes), meta.spill_off,
+                            meta.spill_total};
+  SG_HIP(sgk::attention(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items, meta.n_items, H, HKV, kHd,
+                        scale, nullptr, meta.max_len, s, nullptr, nullptr, &spill, HKV == 1 ? meta.n_split : 0));
+  return SG_OK;
+}
+}  // namespace
+
+extern "C" {
+
 int sg_attention(sg_ctx* ctx, float* out, const float* q, int32_t ldq, const float* k, const float* v, int32_t ldkv,
                  int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, const int32_t* off, int32_t n_seq,
                  void* stream) {
@@ -1426,33 +1464,30 @@ int sg_attention(sg_ctx* ctx, float* out, const float* q, int32_t ldq, const flo
   std::lock_guard<std::mutex> lk(ctx->mu);
   SG_TRY(set_device(ctx));
   hipStream_t s = pick(ctx, stream);
-  Meta meta;
-  SG_TRY(stage_meta(off, n_seq, n_heads / n_kv_heads, ctx->meta_h, ctx->meta_d, s, meta));
-  const float scale = 1.0f / (float)std::sqrt((double)head_dim);
-  // Split operands as the forward's producers write them.
-  const size_t qd = (size_t)n_heads * head_dim, kvd = (size_t)n_kv_heads * head_dim, Tp = (size_t)meta.Tp;
-  const size_t split_bytes = (2 * sizeof(_Float16) * (qd + 2 * kvd) * Tp + 255) & ~(size_t)255;
-  const bool small = sgk::attn_small_form(meta.n_items, n_kv_heads, meta.max_len);
-  SG_TRY(ctx->split.ensure(split_bytes + (small ? 0 : (size_t)n_kv_heads * meta.spill_total * sgk::kAttnSpillTileBytes)));
-  SG_TRY(gemm_scratch_begin(ctx, s));  // after the asynchronous GEMM calls of this context
-  _Float16* qf = ctx->split.as<_Float16>();
-  _Float16* kf = qf + 2 * qd * Tp;
-  _Float16* vf = kf + 2 * kvd * Tp;
-  const int n_tiles = meta.Tp / 32;
-  SG_HIP(sgk::qkv_split(q, ldq, k, v, ldkv, n_heads, n_kv_heads, meta.seq_off, meta.voff, meta.vtiles, meta.n_vtiles,
-                        qf, kf, vf, n_tiles, s));
-  if (small) {
-    SG_HIP(sgk::attention_small(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items,
-                                meta.n_items, n_heads, n_kv_heads, head_dim, scale, nullptr,
-                                meta.max_len, s));
-    SG_HIP(hipStreamSynchronize(s));
-    return SG_OK;
+  // Split operands as the forward's producers write them: every sequence padded to
+  // whole tiles, 32 times the data for a sequence of one token.  So a call whose
+  // operands would pass kSeamSplitBytes runs as pieces of whole sequences (which
+  // do not depend on each other).
+  const size_t qd = (size_t)n_heads * head_dim, kvd = (size_t)n_kv_heads * head_dim;
+  const size_t key_bytes = 2 * sizeof(_Float16) * (qd + 2 * kvd);
+  std::vector<int32_t> sub;
+  for (int s0 = 0, s1; s0 < n_seq; s0 = s1) {
+    size_t bytes = 0;
+    for (s1 = s0; s1 < n_seq; s1++) {
+      const size_t more = key_bytes * sgk::attn_key_pad(off[s1 + 1] - off[s1]);
+      if (s1 > s0 && bytes + more > kSeamSplitBytes) break;
+      bytes += more;
+    }
+    const int32_t* po = off;
+    if (s1 - s0 < n_seq) {
+      sub.assign(off + s0, off + s1 + 1);
+      for (int32_t& o : sub) o -= off[s0];
+      po = sub.data();
+    }
+    const size_t r0 = (size_t)off[s0];
+    SG_TRY(attention_piece(ctx, out + r0 * qd, q + r0 * ldq, ldq, k + r0 * ldkv, v + r0 * ldkv, ldkv, n_heads, n_kv_heads,
+                           po, s1 - s0, s));
   }
-  const sg_attn_spill spill{reinterpret_cast<float*>(ctx->split.as<unsigned char>() + split_bytes), meta.spill_off,
-                            meta.spill_total};
-  SG_HIP(sgk::attention(qf, kf, vf, n_tiles, out, (int)qd, meta.seq_off, meta.voff, meta.items,
-                        meta.n_items, n_heads, n_kv_heads, head_dim, scale, nullptr,
-                        meta.max_len, s, nullptr, nullptr, &spill, n_kv_heads == 1 ? meta.n_split : 0));
   SG_HIP(hipStreamSynchronize(s));
   return SG_OK;
 }

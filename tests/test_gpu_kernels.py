@@ -655,6 +655,33 @@ def test_attention_head_counts(gpu_ctx):
         assert np.array_equal(host(out[:, one]).view(np.uint32), host(want).view(np.uint32)), h
 
 
+def test_attention_pieces_match(gpu_ctx):
+    """A call whose padded operands pass 4 GB runs as pieces of whole sequences:
+    the same bits as the calls on its parts, across a piece's boundary too."""
+    import torch
+    from semantica_gpu import kernels
+    lens = np.ones(29000, np.int64)  # 5 KB per padded token: a piece ends near sequence 26,000
+    lens[::500] = 40
+    lens[25900:26100:20] = 33
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(off[-1])
+    assert 5120 * int(((lens + 31) // 32 * 32).sum()) > 1.05 * 2 ** 32
+    say(f"attention pieces {len(lens)} sequences, {T} tokens")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn((T, n), generator=g, device="cuda") for n in (768, 256, 256))
+    out = torch.empty_like(q)
+    kernels.attention(gpu_ctx, out, q, k, v, 3, 1, 256, off)
+    for a, b in ((0, 400), (25700, 26300), (28600, 29000)):
+        r = slice(int(off[a]), int(off[b]))
+        part = torch.empty((r.stop - r.start, 768), device="cuda")
+        kernels.attention(gpu_ctx, part, q[r].contiguous(), k[r].contiguous(), v[r].contiguous(), 3, 1, 256,
+                          off[a:b + 1] - off[a])
+        assert torch.equal(out[r].view(torch.int32), part.view(torch.int32)), (a, b)
+    # one token attends to itself alone: its value row, in split fp16
+    one = torch.from_numpy(off[:-1][lens == 1].astype(np.int64)).cuda()
+    assert float((out[one] - v[one].repeat(1, 3)).abs().max()) < 1e-5
+
+
 @pytest.mark.parametrize("more,least,most", [(0, 1, 64), (4, 65, 128), (20, 256, 10**6)])
 def test_attention_register_scores_match_spilling_launch(gpu_ctx, more, least, most):
     """The same sequences with and without a 600-key companion (which moves a
